@@ -27,6 +27,7 @@ typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef _Float16 v4h __attribute__((ext_vector_type(4)));
 typedef __fp16 v4fp16 __attribute__((__vector_size__(8)));  // the transposing LDS read's type
 typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float v4f __attribute__((ext_vector_type(4)));
 
 constexpr int FA_BQ = 32;   // query positions per workgroup
 constexpr int FA_BK = 64;   // keys per tile
@@ -827,98 +828,305 @@ ghip_fa_merge(const float *__restrict__ part, const float *__restrict__ sinks, f
 // the keys of one (query, head) row in order and keeps the unnormalized V
 // accumulator in f16, rounding after every rescale and every multiply-add.
 // That rounding is part of the reference's result (it moves outputs by up to
-// a few 1e-3 at S ~ 1000), so this route reproduces the walk: one wavefront
-// per row, lane j scores key k0 + j of each 64-key tile (q rounded to f16,
-// fp32 dot), then the wavefront steps through the tile's keys in order, each
-// lane updating its D/64 accumulator elements with the reference's
-// operations -- skip masked (-inf) keys, new max => rescale by exp(Mold - M)
-// and round, then acc = f16(fma(v, vs, acc)), S = fma(S, ms, vs).
-template <int D>
-__device__ __forceinline__ void fa_rowseq_impl(const FaParams &p) {
-    constexpr int PL = D / 64;  // accumulator elements per lane
-    __shared__ float qs[4][D];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int row = blockIdx.x * 4 + w;  // row = t * H + h
-    const bool valid = row < p.T * p.H;
-    const int t = valid ? row / p.H : 0, h = valid ? row % p.H : 0;
-    const int hk = h / (p.H / p.H_kv);
-    const float slope = head_slope(p, h);
-    const float *qr = p.q + (int64_t)h * p.q_nb2 + (int64_t)t * p.q_nb1;
-    for (int d = lane; d < D; d += 64) qs[w][d] = h2f(f2h_rn(qr[d]));
-    __syncthreads();
-    if (!valid) return;
-    const uint16_t *kbase = p.k + (int64_t)hk * p.k_nb2;
-    const uint16_t *vbase = p.v + (int64_t)hk * p.v_nb2;
-    float acc[PL];
+// a few 1e-3 at S ~ 1000), so the accumulator takes the reference's steps in
+// the reference's order -- skip masked (-inf) keys, new max => rescale by
+// exp(Mold - M) and round, then acc = f16(fma(v, vs, acc)) -- while all that
+// does not depend on it is done for many keys at once.
+//
+// A workgroup owns NC of the G * T rows that read one KV head: NC wavefronts
+// walk a row each, four more prepare their tiles of 64 keys, in three steps
+// that run side by side on three successive tiles (one barrier per tile):
+//  * scores of tile i + 2: preparing wavefront w multiplies keys 16w .. 16w+15
+//    with all the rows on v_mfma_f32_16x16x32_f16 (K fragments straight from
+//    memory, one tile ahead) and leaves scaled, masked scores in LDS (masked
+//    keys as FR_DEAD);
+//  * softmax of tile i + 1, a row at a time: lane j holds key j's score.
+//    Without a new max among them one exp per lane gives the keys' vs; with
+//    one, a prefix max over the lanes gives the running max before and after
+//    every key, and with it the key's vs and, where the max moves, its ms.
+//    V of the tile goes through registers into LDS;
+//  * the walk over tile i: lane l owns dims PL*l .., per key one readlane and
+//    PL fused multiply-adds with f16 rounding (v_fma_mix).  Sixteen keys
+//    with a new max among them rescale at every key (by 1 where the max
+//    stays); a tile with masked keys tests every key.
+//
+// Bound by the walk, a serial chain of 4 + 8 PL clocks per key (v_fma_mix
+// issues in 8) on one wavefront per row, and by the preparation's share of the
+// same SIMDs.  Measured: 37 rows of 64 / 8 heads, D = 64, 1061 keys, sinks:
+// 188 us with one wavefront per row that scored a key per lane and took one
+// exp per key, 66 us with matrix-core scores and an exp per lane in the
+// walking wavefront itself, 59 us with wavefronts of their own for that,
+// 42 us with a tile's loads issued before its arithmetic, no branches for the
+// tiles whose max moves and the walk at a raised priority.
+constexpr uint32_t FR_DEAD = 0xFFFFFFFFu;  // no score has this NaN's payload
+
+// running max over the lanes up to and including each lane
+DEV float wave_cummax(float v) {
+    const int ninf = __float_as_int(-__builtin_inff());
+#define FR_STEP(ctrl, rmask) \
+    v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(ninf, __float_as_int(v), (ctrl), (rmask), 0xF, false)));
+    FR_STEP(0x111, 0xF)  // row_shr:1, 2, 4, 8: within each 16-lane row
+    FR_STEP(0x112, 0xF)
+    FR_STEP(0x114, 0xF)
+    FR_STEP(0x118, 0xF)
+    FR_STEP(0x142, 0xA)  // row_bcast:15 into rows 1 and 3
+    FR_STEP(0x143, 0xC)  // row_bcast:31 into rows 2 and 3
+#undef FR_STEP
+    return v;
+}
+DEV float readlane_f(float v, int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); }
+
+template <int D, int NC>
+__device__ __forceinline__ void fa_rows_impl(const FaParams &p) {
+    constexpr int PL = D / 64, KS = D / 32, RP = NC / 4;  // rows per preparing wavefront
+    constexpr int VP = FA_BK * D * 2 / 16 / 256;           // 16-byte V pieces per preparing thread and tile
+    __shared__ __attribute__((aligned(16))) uint32_t sc[2][NC][FA_BK + 4];
+    __shared__ __attribute__((aligned(16))) uint16_t vt[2][FA_BK][D];
+    __shared__ float vsb[2][NC][FA_BK], msb[2][NC][FA_BK];
+    __shared__ uint64_t liveb[2][NC], evb[2][NC];
+    __shared__ float Mb[NC], Sb[NC];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int G = p.H / p.H_kv, nrow = G * p.T;
+    const int hk = (int)blockIdx.x % p.H_kv, r0 = (int)blockIdx.x / p.H_kv * NC;
+    const int ntile = (p.S + FA_BK - 1) / FA_BK;
+
+    if (w >= NC) {  // prepare
+        const int pw = w - NC, tid = threadIdx.x - 64 * NC;
+        const int c = lane & 15, g4 = lane >> 4;
+        // this lane's score column: row r0 + c (rows past the end repeat the last)
+        const int ci = min(r0 + c, nrow - 1), ct = ci / G, ch = hk * G + (ci - ct * G);
+        const float slope = head_slope(p, ch);
+        const uint16_t *mrow = p.mask ? p.mask + (int64_t)(ch % p.mask_ne2) * p.mask_nb2 + (int64_t)ct * p.mask_nb1 : nullptr;
+        const int mk = 16 * pw + 4 * g4;  // the lane's four keys of a tile
+        const uint8_t *kb = (const uint8_t *)(p.k + (int64_t)hk * p.k_nb2) + 16 * g4;
+        const uint8_t *vb = (const uint8_t *)(p.v + (int64_t)hk * p.v_nb2) + 16 * (tid % (D / 8));
+        const int vkey = tid / (D / 8), kkey = 16 * pw + c;
+        constexpr int VKS = 256 / (D / 8);  // keys between a thread's V pieces
+        v8h qf[KS];
+        {
+            const float *qr = p.q + (int64_t)ch * p.q_nb2 + (int64_t)ct * p.q_nb1 + 8 * g4;
 #pragma unroll
-    for (int i = 0; i < PL; i++) acc[i] = 0.0f;
-    float M = -__builtin_inff(), S = 0.0f;
-    for (int k0 = 0; k0 < p.S; k0 += 64) {
-        const int key = k0 + lane;
-        float s = -__builtin_inff();
-        bool live = false;
-        if (key < p.S) {
-            const float mv = p.mask ? slope * h2f(p.mask[(int64_t)(h % p.mask_ne2) * p.mask_nb2 + (int64_t)t * p.mask_nb1 + key]) : 0.0f;
-            if (mv != -__builtin_inff()) {
-                live = true;
-                const uint8_t *kr = (const uint8_t *)(kbase + (int64_t)key * p.k_nb1);
-                float dot = 0.0f;
-#pragma unroll 4
-                for (int d8 = 0; d8 < D; d8 += 8) {
-                    const uint4 kv = ld16(kr + 2 * d8);
-                    const uint32_t kw[4] = {kv.x, kv.y, kv.z, kv.w};
+            for (int ks = 0; ks < KS; ks++)
 #pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        dot = fmaf(h2f(kw[e] & 0xffff), qs[w][d8 + 2 * e], dot);
-                        dot = fmaf(h2f(kw[e] >> 16), qs[w][d8 + 2 * e + 1], dot);
+                for (int e = 0; e < 8; e++) qf[ks][e] = (_Float16)qr[32 * ks + e];
+        }
+        uint4 kr[KS], vr[VP];
+        uint32_t mr[2] = {0, 0};  // the four mask values, as loaded
+        const uint8_t *kp = kb + (int64_t)kkey * p.k_nb1 * 2, *vp = vb + (int64_t)vkey * p.v_nb1 * 2;
+        auto load_k = [&](int tile) {  // K and mask; keys past the end repeat the last
+            const int k0 = tile * FA_BK;
+            const bool full = k0 + FA_BK <= p.S;
+            const uint8_t *r = full ? kp + (int64_t)k0 * p.k_nb1 * 2 : kb + (int64_t)min(k0 + kkey, p.S - 1) * p.k_nb1 * 2;
+#pragma unroll
+            for (int ks = 0; ks < KS; ks++) kr[ks] = ld16(r + 64 * ks);
+            if (mrow && full) __builtin_memcpy(mr, mrow + k0 + mk, 8);
+            if (mrow && !full) {
+#pragma unroll
+                for (int i = 0; i < 2; i++)
+                    mr[i] = mrow[min(k0 + mk + 2 * i, p.S - 1)] | ((uint32_t)mrow[min(k0 + mk + 2 * i + 1, p.S - 1)] << 16);
+            }
+        };
+        auto load_v = [&](int tile) {
+            const int k0 = tile * FA_BK;
+            const uint8_t *r[VP];
+            if (k0 + FA_BK <= p.S) {
+#pragma unroll
+                for (int i = 0; i < VP; i++) r[i] = vp + (int64_t)(k0 + i * VKS) * p.v_nb1 * 2;
+            } else {
+#pragma unroll
+                for (int i = 0; i < VP; i++) r[i] = vb + (int64_t)min(k0 + vkey + i * VKS, p.S - 1) * p.v_nb1 * 2;
+            }
+#pragma unroll
+            for (int i = 0; i < VP; i++) vr[i] = ld16(r[i]);
+        };
+        float M[RP], S[RP];  // S: this lane's keys' share
+#pragma unroll
+        for (int r = 0; r < RP; r++) {
+            M[r] = -__builtin_inff();
+            S[r] = 0.0f;
+        }
+        if (ntile > 0) {
+            load_k(0);
+            load_v(0);
+        }
+        for (int it = -2; it < ntile; it++) {
+            const int ta = it + 2, tb = it + 1;
+            // what the last step loaded is used up and the next loads issued
+            // before the rest, so that they have a whole step to arrive
+            v4f d = {0.0f, 0.0f, 0.0f, 0.0f};
+            const uint32_t mc[2] = {mr[0], mr[1]};
+            if (ta < ntile) {
+#pragma unroll
+                for (int ks = 0; ks < KS; ks++)
+                    d = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, kr[ks]), qf[ks], d, 0, 0, 0);
+            }
+            if (tb >= 0 && tb < ntile) {
+#pragma unroll
+                for (int i = 0; i < VP; i++) reinterpret_cast<uint4 *>(&vt[tb & 1][0][0])[i * 256 + tid] = vr[i];
+            }
+            if (ta + 1 < ntile) load_k(ta + 1);
+            if (tb >= 0 && tb + 1 < ntile) load_v(tb + 1);
+            if (ta < ntile) {
+                uint32_t sb[4];
+                d *= p.scale;
+                if (p.softcap != 0.0f) {
+#pragma unroll
+                    for (int i = 0; i < 4; i++) d[i] = p.softcap * tanhf(d[i]);
+                }
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const float mv = mrow ? slope * h2f(mc[i >> 1] >> (16 * (i & 1))) : 0.0f;
+                    const float s = d[i] + mv;
+                    const bool live = ta * FA_BK + mk + i < p.S && mv != -__builtin_inff();
+                    sb[i] = live ? __float_as_uint(s) : FR_DEAD;
+                }
+                if (c < NC) *reinterpret_cast<uint4 *>(&sc[ta & 1][c][mk]) = make_uint4(sb[0], sb[1], sb[2], sb[3]);
+            }
+            if (tb >= 0 && tb < ntile) {
+                const int q = tb & 1;
+#pragma unroll
+                for (int r = 0; r < RP; r++) {
+                    const int row = pw * RP + r;
+                    const uint32_t b = sc[q][row][lane];
+                    const bool lv = b != FR_DEAD;
+                    const float s = lv ? __uint_as_float(b) : -__builtin_inff();
+                    uint64_t ev = 0;
+                    float vs, ms = 1.0f;
+                    if (__ballot(s > M[r]) == 0) {
+                        vs = expf(s - M[r]);
+                        S[r] += lv ? vs : 0.0f;
+                    } else {
+                        const float cum = wave_cummax(s);
+                        const float run = fmaxf(M[r], cum);  // the max after key `lane`
+                        const float prev = fmaxf(M[r], __int_as_float(__builtin_amdgcn_update_dpp(
+                                                           __float_as_int(-__builtin_inff()), __float_as_int(cum), 0x138, 0xF, 0xF, false)));
+                        const bool up = lv && s > prev;
+                        const float e = expf(up ? prev - s : s - prev);
+                        vs = up ? 1.0f : e;
+                        ms = up ? e : 1.0f;
+                        ev = __ballot(up);
+                        // S after the tile, scaled to its last max
+                        const float Mn = readlane_f(run, 63);
+                        const float wt = !lv ? 0.0f : run == Mn ? vs : vs * expf(run - Mn);
+                        S[r] = (M[r] == Mn ? S[r] : S[r] * expf(M[r] - Mn)) + wt;
+                        M[r] = Mn;
+                        msb[q][row][lane] = ms;
+                    }
+                    vsb[q][row][lane] = vs;
+                    const uint64_t live = __ballot(lv);
+                    if (lane == 0) {
+                        liveb[q][row] = live;
+                        evb[q][row] = ev;
                     }
                 }
-                s = dot * p.scale;
-                if (p.softcap != 0.0f) s = p.softcap * tanhf(s);
-                s += mv;
             }
-        }
-        const uint64_t livemask = __ballot(live);
-        const int nk = min(64, p.S - k0);
-        for (int j = 0; j < nk; j++) {
-            if (!((livemask >> j) & 1)) continue;
-            const float sj = __shfl(s, j, 64);
-            const uint16_t *vr = vbase + (int64_t)(k0 + j) * p.v_nb1 + PL * lane;
-            float vv[PL];
+            if (it == ntile - 1) {
 #pragma unroll
-            for (int i = 0; i < PL; i++) vv[i] = h2f(vr[i]);
-            float ms = 1.0f, vs = 1.0f;
-            if (sj > M) {
-                const float Mold = M;
-                M = sj;
-                ms = expf(Mold - M);
-#pragma unroll
-                for (int i = 0; i < PL; i++) acc[i] = h2f(f2h_rn(acc[i] * ms));
-            } else {
-                vs = expf(sj - M);
+                for (int r = 0; r < RP; r++) {
+                    const float st = wave_sum_dpp(S[r]);
+                    if (lane == 0) {
+                        Mb[pw * RP + r] = M[r];
+                        Sb[pw * RP + r] = st;
+                    }
+                }
             }
-#pragma unroll
-            for (int i = 0; i < PL; i++) acc[i] = h2f(f2h_rn(fmaf(vv[i], vs, acc[i])));
-            S = fmaf(S, ms, vs);
+            __syncthreads();
         }
+        return;
     }
+
+    // walk (ahead of the preparing wavefronts of the same SIMD: the step waits for it)
+    __builtin_amdgcn_s_setprio(2);
+    _Float16 acc[PL];
+#pragma unroll
+    for (int i = 0; i < PL; i++) acc[i] = (_Float16)0.0f;
+    auto add = [&](const _Float16 (&v)[PL], float vj) {
+#pragma unroll
+        for (int i = 0; i < PL; i++) acc[i] = (_Float16)fmaf((float)v[i], vj, (float)acc[i]);
+    };
+    auto rescale = [&](float mj) {
+#pragma unroll
+        for (int i = 0; i < PL; i++) acc[i] = (_Float16)((float)acc[i] * mj);
+    };
+    for (int it = -2; it < ntile; it++) {
+        if (it >= 0) {
+            const int q = it & 1;
+            const uint16_t *vl = &vt[q][0][PL * lane];
+            const float vs = vsb[q][w][lane];
+            auto uni = [](uint64_t x) {  // the same in every lane
+                return (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)x) |
+                       ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(x >> 32)) << 32);
+            };
+            const uint64_t live = uni(liveb[q][w]), ev = uni(evb[q][w]);
+            const float ms = ev ? msb[q][w][lane] : 1.0f;
+            if (live == ~0ull) {
+                _Float16 vv[2][16][PL];
+#pragma unroll
+                for (int j = 0; j < 16; j++) __builtin_memcpy(vv[0][j], vl + j * D, 2 * PL);
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    if (u < 3) {
+#pragma unroll
+                        for (int j = 0; j < 16; j++) __builtin_memcpy(vv[(u + 1) & 1][j], vl + (16 * u + 16 + j) * D, 2 * PL);
+                    }
+                    float vj[16];
+#pragma unroll
+                    for (int j = 0; j < 16; j++) vj[j] = readlane_f(vs, 16 * u + j);
+                    if (((uint32_t)(ev >> (16 * u)) & 0xFFFFu) == 0) {
+#pragma unroll
+                        for (int j = 0; j < 16; j++) add(vv[u & 1][j], vj[j]);
+                    } else {
+#pragma unroll
+                        for (int j = 0; j < 16; j++) {
+                            rescale(readlane_f(ms, 16 * u + j));
+                            add(vv[u & 1][j], vj[j]);
+                        }
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            } else {
+#pragma unroll 1
+                for (int c8 = 0; c8 < 64; c8 += 8) {
+                    const uint32_t lb = (uint32_t)(live >> c8) & 0xFFu;
+                    if (lb == 0) continue;
+                    _Float16 vv[8][PL];
+#pragma unroll
+                    for (int j = 0; j < 8; j++) __builtin_memcpy(vv[j], vl + (c8 + j) * D, 2 * PL);
+#pragma unroll
+                    for (int j = 0; j < 8; j++)
+                        if ((lb >> j) & 1) {
+                            rescale(readlane_f(ms, c8 + j));
+                            add(vv[j], readlane_f(vs, c8 + j));
+                        }
+                }
+            }
+        }
+        __syncthreads();
+    }
+    const int idx = r0 + w;
+    if (idx >= nrow) return;
+    const int t = idx / G, h = hk * G + (idx - t * G);
+    const float M = ntile > 0 ? Mb[w] : -__builtin_inff();
+    float S = ntile > 0 ? Sb[w] : 0.0f;
+    float a[PL];
+#pragma unroll
+    for (int i = 0; i < PL; i++) a[i] = (float)acc[i];
     if (p.sinks) {
         const float sh = p.sinks[h];
         float ms = 1.0f, vs = 1.0f;
         if (sh > M) {
             ms = expf(M - sh);
-            M = sh;
 #pragma unroll
-            for (int i = 0; i < PL; i++) acc[i] *= ms;
+            for (int i = 0; i < PL; i++) a[i] *= ms;
         } else {
             vs = expf(sh - M);
         }
         S = opaque(S * ms) + vs;  // unfused, as the reference
     }
     const float sinv = S == 0.0f ? 0.0f : 1.0f / S;
-    float *o = p.dst + (int64_t)row * D + PL * lane;
+    float *o = p.dst + ((int64_t)t * p.H + h) * D + PL * lane;
 #pragma unroll
-    for (int i = 0; i < PL; i++) o[i] = acc[i] * sinv;
+    for (int i = 0; i < PL; i++) o[i] = a[i] * sinv;
 }
 
 // General shapes (any DK, DV <= 256, F32 or F16 K and V, any H / H_kv): one
@@ -1027,7 +1235,9 @@ extern "C" __global__ void __launch_bounds__(512) ghip_fa_fwd_d128(FaParams p) {
 extern "C" __global__ void __launch_bounds__(512) ghip_fa_fwd_d64(FaParams p) { fa_fwd_impl<64, false>(p); }
 extern "C" __global__ void __launch_bounds__(512) ghip_fa_fwd_sc_d128(FaParams p) { fa_fwd_impl<128, true>(p); }
 extern "C" __global__ void __launch_bounds__(512) ghip_fa_fwd_sc_d64(FaParams p) { fa_fwd_impl<64, true>(p); }
-extern "C" __global__ void __launch_bounds__(256) ghip_fa_rowseq_d128(FaParams p) { fa_rowseq_impl<128>(p); }
-extern "C" __global__ void __launch_bounds__(256) ghip_fa_rowseq_d64(FaParams p) { fa_rowseq_impl<64>(p); }
+extern "C" __global__ void __launch_bounds__(512) ghip_fa_rows4_d128(FaParams p) { fa_rows_impl<128, 4>(p); }
+extern "C" __global__ void __launch_bounds__(768) ghip_fa_rows8_d128(FaParams p) { fa_rows_impl<128, 8>(p); }
+extern "C" __global__ void __launch_bounds__(512) ghip_fa_rows4_d64(FaParams p) { fa_rows_impl<64, 4>(p); }
+extern "C" __global__ void __launch_bounds__(768) ghip_fa_rows8_d64(FaParams p) { fa_rows_impl<64, 8>(p); }
 extern "C" __global__ void __launch_bounds__(256) ghip_fa_decode_d128(FaParams p) { fa_decode_impl<128>(p); }
 extern "C" __global__ void __launch_bounds__(256) ghip_fa_decode_d64(FaParams p) { fa_decode_impl<64>(p); }

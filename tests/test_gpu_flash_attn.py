@@ -280,3 +280,36 @@ def test_single_slice_direct(be, monkeypatch, T, S, D, masked, sinks):
                                    n_chunks=8)
         err = float(np.max(np.abs(outs[1][:, h:h + 1] - want)))
         assert err <= TOL, f"head {h}: max-abs {err:.3e}"
+
+
+@pytest.mark.parametrize("H,Hkv,D,T,S,holes,sinks,softcap", [
+    (8, 2, 128, 1, 1, False, True, 0.0),       # one key
+    (8, 2, 64, 2, 63, True, False, 0.0),       # below one 64-key tile
+    (6, 2, 128, 3, 64, False, True, 0.0),      # one whole tile; rows past the end of a workgroup
+    (4, 4, 64, 7, 129, True, True, 0.0),       # one key in the last tile, one head per KV head
+    (8, 1, 128, 5, 320, True, False, 20.0),    # softcap
+    (64, 8, 64, 56, 200, True, True, 0.0),     # 448 workgroups: 8 rows each
+    (64, 8, 128, 63, 70, False, False, 0.0),
+])
+def test_few_rows(be, H, Hkv, D, T, S, holes, sinks, softcap):
+    """The few-row walk at its tile and row-group edges: masked keys scattered
+    over the tiles (whole tiles among them) with infinities in their V rows,
+    K and V with keys outside heads (strided rows), against the oracle."""
+    rng = np.random.default_rng(H + T + S)
+    q = rng.standard_normal((H, T, D)).astype(np.float32)
+    k, v = (rng.standard_normal((S, Hkv, D)).astype(np.float16) for _ in range(2))
+    m = causal_mask(T, S)
+    if holes:
+        m[:, rng.random(S) < 0.3] = -np.inf
+        m[:, :S // 3] = -np.inf
+        m[:, S - T:] = causal_mask(T, T)
+        m += (rng.integers(-2, 3, (T, S)) * 0.5).astype(np.float16)
+        dead = np.isinf(m).all(axis=0)
+        v[dead] = np.inf
+    sk = rng.standard_normal(H).astype(np.float32) if sinks else None
+    kt, vt = (np.ascontiguousarray(a.transpose(1, 0, 2)) for a in (k, v))
+    want, _ = O.flash_attn_ext(q, kt, vt, m, sk, 1.0 / np.sqrt(D), 0.0, softcap)
+    t = lambda a: torch.from_numpy(a).cuda() if a is not None else None
+    got = be.flash_attn_ext(t(q), t(k).permute(1, 0, 2), t(v).permute(1, 0, 2), t(m), t(sk), 1.0 / np.sqrt(D), 0.0,
+                            softcap).cpu().numpy()
+    assert np.max(np.abs(got - want)) <= TOL
