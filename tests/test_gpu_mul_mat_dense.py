@@ -89,3 +89,35 @@ def test_dense_batched_planes(be):
     for p in range(4):
         want = O.mul_mat_dense(O.F16, wb[p // 2], k, rows, x[p].numpy(), m)
         assert rel_err(got[p], want) <= TOL
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (9, 33, 8),           # one step's first piece; 32 x 32 tiles, ragged rows
+    (32, 32, 64),         # one whole step, one whole tile
+    (33, 65, 72),         # a step of one piece
+    (65, 127, 584),       # past the first eight steps
+    (40, 70, 77),         # K not a multiple of 8: rows that end inside a piece
+    (9, 16, 3),
+    (200, 3841, 256),     # 64 x 64 tiles
+    (520, 6017, 136),     # 128 x 128 tiles
+])
+@pytest.mark.parametrize("ty", ["f16", "bf16"])
+def test_prefill_gemm(be, ty, M, N, K):
+    """F16 / BF16 weights from 9 rows (the matrix cores) at the edges of tiles,
+    steps and pieces, with strided rows, against 64-bit sums of the exact
+    products.  Bound: every partial sum is rounded at most 64 times inside a
+    step, 8 times over the steps of a group, K / 512 + 1 times over the groups
+    and 3 times over wavefronts, each by 2^-24 of the terms' magnitude."""
+    import ghip
+    td = torch.float16 if ty == "f16" else torch.bfloat16
+    g = torch.Generator().manual_seed(M + N + K)
+    w = (torch.randn((N, K + 5), generator=g) * 0.02).to(td)
+    w[0, : min(3, K)] = 1e-6  # f16 subnormals
+    x = torch.randn((M, K + 3), generator=g)
+    xr, wr = x[:, :K].to(td).double(), w[:, :K].double()
+    want, mag = xr @ wr.t(), xr.abs() @ wr.abs().t()
+    out = torch.full((M + 1, N + 2), 7.0, device="cuda")
+    got = be.mul_mat(w.cuda()[:, :K], ghip.F16 if ty == "f16" else ghip.BF16, K, x.cuda()[:, :K], out=out[:M, :N])
+    err = (got.cpu().double() - want).abs()
+    assert bool((err <= (64 + 8 + K // 512 + 1 + 3) * 2.0 ** -24 * mag).all()), float((err / mag.clamp_min(1e-30)).max())
+    assert bool((out[M] == 7.0).all()) and bool((out[:, N:] == 7.0).all())
