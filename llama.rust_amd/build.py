@@ -17,7 +17,7 @@ CSRC = os.path.join(HERE, "csrc")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 HIPCC = os.path.join(ROCM, "bin", "hipcc")
 
-KERNELS = ["ghip_quant", "ghip_gemv", "ghip_wquant", "ghip_gemm", "ghip_fa", "ghip_moe", "ghip_skinny", "ghip_iq", "ghip_dense"]
+KERNELS = ["ghip_quant", "ghip_kq", "ghip_gemv", "ghip_wquant", "ghip_gemm", "ghip_fa", "ghip_moe", "ghip_skinny", "ghip_iq", "ghip_dense"]
 DEVICE_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17",
     # exact fp32 semantics: products and sums round on their own, fused
@@ -40,6 +40,7 @@ EXTRA_FLAGS = {
     "ghip_moe": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "ghip_fa": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "ghip_gemm": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+    "ghip_kq": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "ghip_dense": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "ghip_skinny": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
 }

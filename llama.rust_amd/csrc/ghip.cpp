@@ -20,7 +20,7 @@
 
 namespace {
 
-const char *const kModules[] = {"ghip_quant.hsaco", "ghip_gemv.hsaco", "ghip_wquant.hsaco", "ghip_gemm.hsaco", "ghip_fa.hsaco", "ghip_moe.hsaco", "ghip_skinny.hsaco", "ghip_iq.hsaco", "ghip_dense.hsaco"};
+const char *const kModules[] = {"ghip_quant.hsaco", "ghip_kq.hsaco", "ghip_gemv.hsaco", "ghip_wquant.hsaco", "ghip_gemm.hsaco", "ghip_fa.hsaco", "ghip_moe.hsaco", "ghip_skinny.hsaco", "ghip_iq.hsaco", "ghip_dense.hsaco"};
 
 struct TypeInfo {
     int blck;
@@ -224,6 +224,13 @@ struct ghip_context {
         if (st == GHIP_STATUS_SUCCESS) *out = (uint8_t *)*out + hold;
         return st;
     }
+    // would workspace(bytes) succeed (short of a failing hipMalloc)?
+    bool workspace_fits(size_t bytes, hipStream_t s) const {
+        bytes += hold;
+        if (call_ws) return bytes <= call_ws_size;
+        if (user_ws) return bytes <= user_ws_size;
+        return dry_run || bytes <= ws_size || !capturing(s);
+    }
     ghip_status workspace_base(size_t bytes, hipStream_t s, void **out) {
         if (dry_run && !call_ws && !user_ws) {
             // an address range no allocation uses: the launches are checked, never run
@@ -308,7 +315,28 @@ struct MulMatPlan {
     int64_t n_mat;    // leading activation rows quantized with quantize_mat_q8_K_4x8 values
     int64_t nb;       // blocks per weight row
     bool act_pre;     // src1 already holds the vec_dot_type blocks
+    int kq_ns = 0;        // K slices of the Q2_K / Q3_K / Q6_K prefill GEMM (ghip_kq.hip); 0: not on it
+    bool kq_reg = false;  // ... over a registered weight's records
 };
+
+// Q2_K / Q3_K / Q6_K prefill: the int8 GEMM of ghip_kq.hip
+bool kq_type(int t) { return t == GHIP_TYPE_Q2_K || t == GHIP_TYPE_Q3_K || t == GHIP_TYPE_Q6_K; }
+// Activation rows from which it beats the decode kernels (groups of 4 or 8
+// rows) with the records rebuilt by the call: 17 x 4096 -> 14336 Q3_K 44 us
+// against 66, Q2_K 46 against 56; at 16 rows they tie.
+int kq_min_rows(int t) { return t == GHIP_TYPE_Q6_K ? env_int("GHIP_GEMM_Q6K_MIN_ROWS", 64) : 17; }
+// K slices that give about 512 workgroups of 64 x 128 outputs (two per CU), at
+// least four super-blocks each (one workgroup per CU leaves a SIMD's one
+// wavefront waiting: 512 x 14336 -> 4096 Q3_K 91 us without the split, 71 with); the slices' partial sums are added in order by
+// ghip_gemm_splitk_reduce (four outputs a thread)
+int kq_nsplit(int64_t M, int64_t N, int64_t nb) {
+    const int64_t tiles = ((M + 63) / 64) * ((N + 127) / 128);
+    if (N % 4 || tiles >= 384 || nb < 8) return 1;
+    const int64_t want = (512 + tiles - 1) / tiles, nbs = std::max<int64_t>(4, (nb + want - 1) / want);
+    return (int)((nb + nbs - 1) / nbs);
+}
+
+int kq_plan_ns(MulMatPlan p);
 
 // IQ1 / IQ2 / IQ3 codebook weights (ghip_iq.hip gemv_grid_impl), Q8_K activations
 bool grid_type(int t) {
@@ -397,6 +425,8 @@ bool plan_mul_mat(ghip_context *ctx, const ghip_tensor *a, const ghip_tensor *b,
     if (p.act_pre) p.act_row_bytes = (int64_t)b->nb[1];
     if (p.N > INT32_MAX || p.nb > INT32_MAX) { st = ctx->fail(st, "mul_mat: dimension too large"); return false; }
     if (p.M < 0 || p.N < 0) { st = ctx->fail(st, "mul_mat: negative dimension"); return false; }
+    // (mul_mat_plane takes it back where its workspace is not to be had)
+    p.kq_ns = kq_type(p.wtype) && p.M >= kq_min_rows(p.wtype) && p.M <= INT32_MAX ? kq_plan_ns(p) : 0;
     st = GHIP_STATUS_SUCCESS;
     return true;
 }
@@ -842,7 +872,6 @@ ghip_status run_gemv(ghip_context *ctx, const MulMatPlan &p, const void *w, cons
 // out for the GEMM (codes | bsum16 | d, tokens padded to 128), then the int8
 // MFMA GEMM runs on 128 x 128 tiles.
 constexpr size_t kGemmSmem128 = 116224, kGemmSmem64 = 76544;  // sizeof(g3::Smem<BM>) in ghip_gemm.hip
-constexpr size_t kGemmSmemQ6 = 152320;
 constexpr size_t kGemmSmemQ8 = 22528;                          // sizeof(g8::Smem) in ghip_gemm.hip                         // sizeof(g6::Smem) in ghip_gemm.hip
 constexpr size_t kGemmSmemW8 = 148480;  // 2 * sizeof(g4::Stage<256>) in ghip_gemm.hip
 // GHIP_GEMM_BM=128 selects the 128 x 128 tiles of gemm_q4K_impl
@@ -884,18 +913,38 @@ int gemm_nsplit(const MulMatPlan &p) {
     const int64_t nbs = (p.nb + want - 1) / want;  // super-blocks per slice
     return (int)((p.nb + nbs - 1) / nbs);
 }
-// Q6_K prefill workspace: f16 codes [Mpad][K] | dT [nb][Mpad] | repacked weights [N][nb][336]
-constexpr size_t kQ6R = 336;
+// Q2_K / Q3_K / Q6_K prefill workspace: int8 codes [Mpad][K] | bsT [nb][Mpad][16]
+// f16 | dT [nb][Mpad] | weight records (not for a registered weight) | split-K
+// partials [ns][M][N].  Record bytes per (32-row tile, super-block): kq_rec in ghip_kq.hip.
+size_t kq_weight_bytes(int wtype, int64_t N, int64_t nb) {
+    const size_t rec = wtype == GHIP_TYPE_Q6_K ? 8832 : wtype == GHIP_TYPE_Q3_K ? 8320 : 9472;
+    return (size_t)((N + 31) / 32) * (size_t)nb * rec;
+}
+// a registered weight's copy (Q6_K: 336 bytes per row and super-block at
+// least, the size its budget has always counted)
+size_t kq_copy_bytes(int wtype, int64_t N, int64_t nb) {
+    const size_t n = kq_weight_bytes(wtype, N, nb);
+    return wtype == GHIP_TYPE_Q6_K ? std::max(n, (size_t)N * (size_t)nb * 336) : n;
+}
+struct KqLayout {
+    int64_t Mpad;
+    size_t bs_off, dt_off, w_off, part_off, total;
+};
+KqLayout kq_layout(const MulMatPlan &p) {
+    KqLayout L;
+    auto up = [](size_t x) { return (x + 255) & ~(size_t)255; };
+    L.Mpad = (p.M + 127) / 128 * 128;
+    L.bs_off = (size_t)L.Mpad * (size_t)p.K;
+    L.dt_off = L.bs_off + (size_t)(p.nb * L.Mpad) * 32;
+    L.w_off = up(L.dt_off + (size_t)(p.nb * L.Mpad) * 4);
+    L.part_off = L.w_off + (p.kq_reg ? 0 : up(kq_weight_bytes(p.wtype, p.N, p.nb)));
+    L.total = L.part_off + (p.kq_ns > 1 ? (size_t)p.kq_ns * (size_t)p.M * (size_t)p.N * 4 : 0);
+    return L;
+}
 // registered MXFP4 experts (ghip_mxfp4_repack): 128-row blocks, groups of 4
 // 17-byte blocks, 80-byte windows -> one 10240-byte run per (expert, row block, group)
 constexpr int64_t kMoeRows = 128, kMoeGroup = 4;
 constexpr size_t kMoeWindowRun = 128 * 80;
-size_t gemm_q6k_bytes(const MulMatPlan &p, size_t *codes_b, size_t *dt_b) {
-    const size_t Mpad = (size_t)(p.M + 127) / 128 * 128, nbk = (size_t)p.K / 256;
-    *codes_b = (Mpad * (size_t)p.K * 2 + 255) & ~(size_t)255;
-    *dt_b = (nbk * Mpad * 4 + 255) & ~(size_t)255;
-    return *codes_b + *dt_b + (size_t)p.N * nbk * kQ6R;
-}
 // Q4_0 / Q5_0 / Q8_0 prefill workspace: act codes [Mpad][Kpad] | da [nbp][Mpad] |
 // weight codes [Npad][Kpad] | dw [nbp][Npad] (K padded to 128, rows to 128)
 struct Q8Layout {
@@ -924,61 +973,87 @@ size_t gemm_layout_bytes(const MulMatPlan &p) {
         const Q8Layout L = q8_layout(p.M, p.N, p.K);
         return L.act_b + L.da_b + L.w_b + L.dw_b + q8_extra_b(p.wtype, L);
     }
-    if (p.wtype == GHIP_TYPE_Q6_K) {
-        size_t a, b;
-        return gemm_q6k_bytes(p, &a, &b);
-    }
+    if (p.kq_ns) return kq_layout(p).total;
     const size_t Mpad = (size_t)(p.M + 127) / 128 * 128, nbk = (size_t)p.K / 256;
     const int ns = gemm_nsplit(p);
     const size_t part = ns > 1 ? (size_t)ns * (size_t)p.M * (size_t)p.N * 4 : 0;
     return ((Mpad * (size_t)p.K + nbk * Mpad * 32 + nbk * Mpad * 4 + 255) & ~(size_t)255) + part;
 }
-// Q6_K: repack the weights into aligned records, lay the codes out as f16, then
-// the f16-MFMA GEMM on 64 x 128 tiles (one workgroup per CU, 137 KB of LDS)
-// The Q6_K weights as the GEMM's 336-byte records: rebuilt into the
-// workspace by every call, unless ghip_weight_register keeps a copy.
-ghip_status q6k_repack(ghip_context *ctx, const void *w, int64_t row_bytes, int64_t N, int64_t nbk, uint8_t *rep,
-                       hipStream_t s) {
-    const int64_t nblk = N * nbk;  // four blocks per workgroup
-    ctx->expect(rep, (size_t)nblk * kQ6R, "Q6_K repack");
-    return ctx->launch("ghip_q6K_repack", dim3((unsigned)((nblk + 3) / 4)), dim3(256), 0, s, (const uint8_t *)w,
-                       row_bytes, (int)N, (int)nbk, rep);
+// Q8_K activations in the GEMMs' layout, from Q8_K rows (bf == nullptr) or
+// quantized straight from f32 rows: codes [Mpad][K] | bsT [nb][Mpad][16] f16 | dT [nb][Mpad]
+ghip_status gemm_act(ghip_context *ctx, const MulMatPlan &p, const uint8_t *act, const ghip_tensor *bf, int64_t Mpad,
+                     int8_t *codes, uint16_t *bsT, float *dT, hipStream_t s) {
+    const int64_t nbk = p.K / 256;
+    const unsigned lgrid = (unsigned)((p.M * nbk + 3) / 4);
+    ctx->expect(codes, (size_t)(Mpad * p.K), "activation codes");
+    ctx->expect(bsT, (size_t)(nbk * Mpad * 32), "activation bsum16");
+    ctx->expect(dT, (size_t)(nbk * Mpad * 4), "activation scales");
+    return bf ? ctx->launch("ghip_gemm_act_q8K", dim3(lgrid), dim3(256), 0, s, (const float *)bf->data,
+                            (int64_t)bf->nb[1] / 4, (int)p.M, (int)Mpad, (int)nbk, (int)p.n_mat, codes, bsT, dT)
+              : ctx->launch("ghip_gemm_act_layout", dim3(lgrid), dim3(256), 0, s, act, (int64_t)p.act_row_bytes,
+                            (int)p.M, (int)Mpad, (int)nbk, codes, bsT, dT);
 }
-const uint8_t *registered_q6k(ghip_context *ctx, const MulMatPlan &p, const void *w) {
-    auto it = ctx->wcache.find({w, GHIP_TYPE_Q6_K, p.K, p.N, 1, (uint64_t)p.w_row_bytes, 0});
+// Q6_K from 64 rows has always needed its GEMM's workspace and is refused
+// without it; the others were served by the decode kernels' small one
+bool kq_required(const MulMatPlan &p) { return p.wtype == GHIP_TYPE_Q6_K && p.M >= 64 && p.K >= 512; }
+// the K split, for those calls within the bytes they have always asked for
+// (f16 codes, scales, 336 bytes per row and super-block)
+int kq_plan_ns(MulMatPlan p) {
+    p.kq_ns = kq_nsplit(p.M, p.N, p.nb);
+    if (!kq_required(p)) return p.kq_ns;
+    auto up = [](size_t x) { return (x + 255) & ~(size_t)255; };
+    const size_t Mpad = (size_t)(p.M + 127) / 128 * 128, nb = (size_t)p.nb;
+    const size_t was = up(Mpad * (size_t)p.K * 2) + up(nb * Mpad * 4) + (size_t)p.N * nb * 336;
+    while (p.kq_ns > 1 && kq_layout(p).total > was) p.kq_ns--;
+    const int64_t nbs = (p.nb + p.kq_ns - 1) / p.kq_ns;
+    return p.kq_ns = (int)((p.nb + nbs - 1) / nbs);  // no empty slice
+}
+const char *kq_name(int wtype) {
+    return wtype == GHIP_TYPE_Q6_K ? "q6_K" : wtype == GHIP_TYPE_Q3_K ? "q3_K" : "q2_K";
+}
+// the weight's records, per call or kept by ghip_weight_register
+ghip_status kq_repack(ghip_context *ctx, int wtype, const void *w, int64_t row_bytes, int64_t N, int64_t nb,
+                      uint8_t *rec, hipStream_t s) {
+    ctx->expect(rec, kq_weight_bytes(wtype, N, nb), "weight records");
+    return ctx->launch(std::string("ghip_kq_repack_") + kq_name(wtype), dim3((unsigned)(((N + 31) / 32 * nb + 3) / 4)),
+                       dim3(256), 0, s, (const uint8_t *)w, row_bytes, (int)N, (int)nb, (int64_t)((N + 31) / 32 * nb), rec);
+}
+const uint8_t *kq_registered(ghip_context *ctx, const MulMatPlan &p, const void *w) {
+    auto it = ctx->wcache.find({w, p.wtype, p.K, p.N, 1, (uint64_t)p.w_row_bytes, 0});
     return it == ctx->wcache.end() ? nullptr : (const uint8_t *)it->second.p;
 }
-ghip_status run_gemm_q6k(ghip_context *ctx, const MulMatPlan &p, const void *w, const uint8_t *act,
-                         const ghip_tensor *bf, float *dst, int64_t ldd, int32_t *sub, void *layout_ws, hipStream_t s) {
-    size_t codes_b, dt_b;
-    gemm_q6k_bytes(p, &codes_b, &dt_b);
-    const int64_t Mpad = (p.M + 127) / 128 * 128, nbk = p.K / 256;
-    uint16_t *codes = (uint16_t *)layout_ws;
-    float *dT = (float *)((uint8_t *)layout_ws + codes_b);
-    const uint8_t *rep = registered_q6k(ctx, p, w);
-    ghip_status st = GHIP_STATUS_SUCCESS;
-    if (!rep) {
-        uint8_t *r = (uint8_t *)layout_ws + codes_b + dt_b;
-        st = q6k_repack(ctx, w, p.w_row_bytes, p.N, nbk, r, s);
+// Q2_K / Q3_K / Q6_K from Q8_K rows (bf == nullptr) or f32 rows: the codes into
+// the layout, the weight records if none are kept, then the int8 GEMM
+ghip_status run_gemm_kq(ghip_context *ctx, const MulMatPlan &p, const void *w, const uint8_t *act,
+                        const ghip_tensor *bf, float *dst, int64_t ldd, int32_t *sub, void *layout_ws, hipStream_t s) {
+    const KqLayout L = kq_layout(p);
+    uint8_t *base = (uint8_t *)layout_ws;
+    int8_t *codes = (int8_t *)base;
+    uint16_t *bsT = (uint16_t *)(base + L.bs_off);
+    float *dT = (float *)(base + L.dt_off);
+    ghip_status st;
+    const uint8_t *rec = kq_registered(ctx, p, w);
+    if (!rec) {
+        rec = base + L.w_off;
+        st = kq_repack(ctx, p.wtype, w, p.w_row_bytes, p.N, p.nb, base + L.w_off, s);
         if (st != GHIP_STATUS_SUCCESS) return st;
-        rep = r;
     }
-    ctx->expect(codes, (size_t)(Mpad * p.K * 2), "activation codes");
-    ctx->expect(dT, (size_t)(nbk * Mpad * 4), "activation scales");
-    if (bf)  // f32 activations: quantized straight into the layout
-        st = ctx->launch("ghip_gemm_act_q8K_f16", dim3((unsigned)((p.M * nbk + 3) / 4)), dim3(256), 0, s,
-                         (const float *)bf->data, (int64_t)bf->nb[1] / 4, (int)p.M, (int)Mpad, (int)nbk, (int)p.n_mat,
-                         codes, dT);
-    else
-        st = ctx->launch("ghip_gemm_act_layout_f16", dim3((unsigned)((p.M * nbk + 3) / 4)), dim3(256), 0, s, act,
-                         (int64_t)p.act_row_bytes, (int)p.M, (int)Mpad, (int)nbk, codes, dT);
+    st = gemm_act(ctx, p, act, bf, L.Mpad, codes, bsT, dT, s);
     if (st != GHIP_STATUS_SUCCESS) return st;
-    const unsigned grid = (unsigned)(((p.M + 63) / 64) * ((p.N + 127) / 128));
-    ctx->expect(dst, win2d(p.M, ldd, p.N), "dst");
+    const int ns = p.kq_ns;
+    const int64_t nbs = (p.nb + ns - 1) / ns;
+    float *out = ns > 1 ? (float *)(base + L.part_off) : dst;
+    if (ns > 1) ctx->expect(out, (size_t)ns * (size_t)(p.M * p.N) * 4, "split-K partials");
+    else ctx->expect(dst, win2d(p.M, ldd, p.N), "dst");
     if (sub) ctx->expect(sub, sub_bytes(p, p.M), "sub-sums");
-    return ctx->launch(sub ? "ghip_gemm_q6_K_sub" : "ghip_gemm_q6_K", dim3(grid), dim3(256), kGemmSmemQ6, s,
-                       (const uint8_t *)rep, (int)p.N, (int)nbk, (const uint16_t *)codes, (const float *)dT, (int)p.M,
-                       (int)Mpad, dst, ldd, sub);
+    const unsigned grid = (unsigned)(((p.M + 63) / 64) * ((p.N + 127) / 128));
+    st = ctx->launch(std::string("ghip_gemm_kq_") + kq_name(p.wtype) + (sub ? "_sub" : ""), dim3(grid, ns), dim3(256), 0,
+                     s, rec, (int)p.N, (int)p.nb, (const int8_t *)codes, (const uint16_t *)bsT, (const float *)dT,
+                     (int)p.M, (int)L.Mpad, out, ns > 1 ? (int64_t)p.N : ldd, sub, (int)nbs, ns > 1 ? p.M * p.N : (int64_t)0);
+    if (st != GHIP_STATUS_SUCCESS || ns == 1) return st;
+    ctx->expect(dst, win2d(p.M, ldd, p.N), "dst");
+    return ctx->launch("ghip_gemm_splitk_reduce", dim3((unsigned)((p.M * p.N / 4 + 255) / 256)), dim3(256), 0, s,
+                       (const float *)out, ns, (int)p.M, (int)p.N, dst, ldd);
 }
 
 const char *q8w_repack_name(int wtype) {
@@ -1057,21 +1132,13 @@ ghip_status run_gemm_q8(ghip_context *ctx, const MulMatPlan &p, const void *w, c
 // straight into the GEMM layout
 ghip_status run_gemm(ghip_context *ctx, const MulMatPlan &p, const void *w, const uint8_t *act, const ghip_tensor *bf,
                      float *dst, int64_t ldd, int32_t *sub, void *layout_ws, hipStream_t s) {
-    if (p.wtype == GHIP_TYPE_Q6_K) return run_gemm_q6k(ctx, p, w, act, bf, dst, ldd, sub, layout_ws, s);
+    if (p.kq_ns) return run_gemm_kq(ctx, p, w, act, bf, dst, ldd, sub, layout_ws, s);
     if (gemm_q8_family(p.wtype)) return run_gemm_q8(ctx, p, w, bf, dst, ldd, sub, layout_ws, s);
     const int64_t Mpad = (p.M + 127) / 128 * 128, K = p.K, nbk = p.K / 256;
     int8_t *codes = (int8_t *)layout_ws;
     uint16_t *bsT = (uint16_t *)(codes + Mpad * K);
     float *dT = (float *)(bsT + nbk * Mpad * 16);
-    const unsigned lgrid = (unsigned)((p.M * nbk + 3) / 4);
-    ctx->expect(codes, (size_t)(Mpad * K), "activation codes");
-    ctx->expect(bsT, (size_t)(nbk * Mpad * 32), "activation bsum16");
-    ctx->expect(dT, (size_t)(nbk * Mpad * 4), "activation scales");
-    ghip_status st =
-        bf ? ctx->launch("ghip_gemm_act_q8K", dim3(lgrid), dim3(256), 0, s, (const float *)bf->data,
-                         (int64_t)bf->nb[1] / 4, (int)p.M, (int)Mpad, (int)nbk, (int)p.n_mat, codes, bsT, dT)
-           : ctx->launch("ghip_gemm_act_layout", dim3(lgrid), dim3(256), 0, s, act, (int64_t)p.act_row_bytes,
-                         (int)p.M, (int)Mpad, (int)nbk, codes, bsT, dT);
+    ghip_status st = gemm_act(ctx, p, act, bf, Mpad, codes, bsT, dT, s);
     if (st != GHIP_STATUS_SUCCESS) return st;
     const GemmKernel &gk = gemm_kernel_for(p);
     const unsigned grid = (unsigned)gemm_tiles(gk, p.M, p.N);
@@ -1100,8 +1167,7 @@ bool use_gemm(const MulMatPlan &p) {
     if (p.wtype == GHIP_TYPE_Q4_K) return p.M >= env_int("GHIP_GEMM_MIN_ROWS", 16);
     // Q5_K: the wide Q4_K tiles with a fifth-bit plane, from 16 rows
     if (p.wtype == GHIP_TYPE_Q5_K) return p.M >= env_int("GHIP_GEMM_Q5K_MIN_ROWS", 16);
-    // Q6_K: the f16-MFMA GEMM from 64 activation rows (below, the 8-column decode kernels)
-    if (p.wtype == GHIP_TYPE_Q6_K) return p.M >= env_int("GHIP_GEMM_Q6K_MIN_ROWS", 64) && p.K >= 512;
+    if (kq_type(p.wtype)) return p.kq_ns > 0;
     // Q4_0 / Q5_0 / Q8_0 from f32 activations: the int8-MFMA GEMM from 32 rows
     if (gemm_q8_family(p.wtype)) return !p.act_pre && p.M >= env_int("GHIP_GEMM_Q8_MIN_ROWS", 32);
     return false;
@@ -1197,6 +1263,20 @@ ghip_status mul_mat_plane(ghip_context *ctx, const ghip_tensor *a, const ghip_te
     if (d) ctx->allow(d->data, win2d(p.M, (int64_t)d->nb[1], (int64_t)d->ne[0] * 4, 1), "dst");
     ctx->allow(sub, sub_bytes(p, p.M), "sub-sums");
     ctx->allow(act_out, (size_t)(p.M * p.act_row_bytes), "activation output");
+    if (kq_type(p.wtype) && !act_out) {
+        // a kept copy of the records also pays at fewer rows (Q6_K keeps one
+        // rule: registered and not give the same bits).  Where the workspace
+        // cannot hold the layout (a caller's or a fixed one, or growth under
+        // capture), first without the K split, else the decode kernels.
+        p.kq_reg = kq_registered(ctx, p, a->data) != nullptr;
+        if (!p.kq_ns && p.kq_reg && p.wtype != GHIP_TYPE_Q6_K && p.M >= 9 && p.M <= INT32_MAX)
+            p.kq_ns = kq_nsplit(p.M, p.N, p.nb);
+        auto fits = [&] { return ctx->workspace_fits(mul_mat_ws_bytes(p, d != nullptr, false, nullptr, nullptr), s); };
+        if (!kq_required(p)) {
+            if (p.kq_ns > 1 && !fits()) p.kq_ns = 1;
+            if (p.kq_ns == 1 && !fits()) p.kq_ns = 0;
+        }
+    }
     size_t act_bytes, lay_bytes;
     const size_t need = mul_mat_ws_bytes(p, d != nullptr, act_out != nullptr, &act_bytes, &lay_bytes, sub != nullptr);
     void *ws = nullptr;
@@ -2267,11 +2347,18 @@ ghip_status ghip_weight_register(ghip_context *ctx, const ghip_tensor *w, void *
     if (w->ne[0] <= 0 || w->ne[1] <= 0 || w->ne[2] <= 0 || w->ne[3] != 1)
         return ctx->fail(GHIP_STATUS_BACKEND_ERROR, "weight_register: empty or 4-D weight");
     const bool q6k = w->type == GHIP_TYPE_Q6_K, mx = w->type == GHIP_TYPE_MXFP4, q8 = gemm_q8_family(w->type);
+    // Q2_K / Q3_K: records of the prefill GEMM for 2-D weights where they can be
+    // built now; otherwise the weight is read in its GGUF layout, like the
+    // types without a copy
+    const bool k23 = k23_type(w->type) && w->ne[2] == 1 && w->ne[0] % 256 == 0 && w->ne[1] <= INT32_MAX &&
+                     w->nb[0] == (uint64_t)type_info(w->type).bytes &&
+                     w->nb[1] >= (uint64_t)(w->ne[0] / 256 * type_info(w->type).bytes) && !ctx->dry_run &&
+                     !ghip_context::capturing((hipStream_t)stream);
     if ((q6k || q8) && w->ne[2] != 1)
         return ctx->fail(GHIP_STATUS_BACKEND_ERROR,
                          "weight_register: Q6_K / Q4_0 / Q5_0 / Q8_0 / IQ4_NL / IQ4_XS / Q1_0 / Q2_0 weights are 2-D");
     // every other type is read in its GGUF layout: nothing to build
-    if (!(q6k || mx || q8) || !repack_enabled()) return GHIP_STATUS_SUCCESS;
+    if (!(q6k || mx || q8 || k23) || !repack_enabled()) return GHIP_STATUS_SUCCESS;
     size_t bytes;
     int64_t nbk = 0, nrb = 0, ngp = 0;
     Q8Layout QL{};
@@ -2282,13 +2369,16 @@ ghip_status ghip_weight_register(ghip_context *ctx, const ghip_tensor *w, void *
         if (w->ne[1] > INT32_MAX) return ctx->fail(GHIP_STATUS_BACKEND_ERROR, "weight_register: dimension too large");
         QL = q8_layout(1, w->ne[1], w->ne[0]);
         bytes = QL.w_b + QL.dw_b + q8_extra_b(w->type, QL);
+    } else if (k23) {
+        nbk = w->ne[0] / 256;
+        bytes = kq_copy_bytes(w->type, w->ne[1], nbk);
     } else if (q6k) {
         if (w->ne[0] % 256 || w->nb[0] != 210 || w->nb[1] < (uint64_t)(w->ne[0] / 256 * 210))
             return ctx->fail(GHIP_STATUS_BACKEND_ERROR, "weight_register: bad Q6_K geometry");
         if (w->ne[1] > INT32_MAX || w->ne[0] / 256 > INT32_MAX)
             return ctx->fail(GHIP_STATUS_BACKEND_ERROR, "weight_register: dimension too large");
         nbk = w->ne[0] / 256;
-        bytes = (size_t)w->ne[1] * (size_t)nbk * kQ6R;
+        bytes = kq_copy_bytes(w->type, w->ne[1], nbk);
     } else {
         if (w->ne[0] % 32 || w->nb[0] != 17 || w->nb[1] < (uint64_t)(w->ne[0] / 32 * 17) ||
             (w->ne[2] > 1 && w->nb[2] < w->nb[1] * (uint64_t)w->ne[1]))
@@ -2311,13 +2401,15 @@ ghip_status ghip_weight_register(ghip_context *ctx, const ghip_tensor *w, void *
     void *rep = nullptr;
     if (hipMalloc(&rep, bytes) != hipSuccess) {
         (void)hipGetLastError();
+        if (k23) return GHIP_STATUS_SUCCESS;  // not kept
         return ctx->fail(GHIP_STATUS_OUT_OF_MEMORY, "weight_register: hipMalloc(%zu) failed", bytes);
     }
     if (q8) {
         st = q8w_repack(ctx, w->type, w->data, (int64_t)w->nb[1], w->ne[1], w->ne[0] / type_info(w->type).blck, QL, (int8_t *)rep,
                         (float *)((uint8_t *)rep + QL.w_b), s);
-    } else if (q6k) {
-        st = q6k_repack(ctx, w->data, (int64_t)w->nb[1], w->ne[1], nbk, (uint8_t *)rep, s);
+    } else if (q6k || k23) {
+        ctx->allow(rep, bytes, "weight records");
+        st = kq_repack(ctx, w->type, w->data, (int64_t)w->nb[1], w->ne[1], nbk, (uint8_t *)rep, s);
     } else {
         const int64_t chunks = (int64_t)(bytes / 16);
         st = ctx->launch("ghip_mxfp4_repack", dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, s,

@@ -585,252 +585,6 @@ extern "C" __global__ void __launch_bounds__(512, 1)
 }
 
 
-
-
-// ---------------------------------------------------------------- Q6_K prefill
-// Many activation rows with Q6_K weights (vec_dot_q6_K_q8_K, vec_dot.rs:982-1040,
-// per super-block  is = sum_s sc_s * sum_16 (q6 - 32) * q8,  out += (d * is) * d8).
-//
-// On the f16 matrix cores with exact operands:
-//  * activations: the Q8_K codes as f16 (exact), written by ghip_gemm_act_layout_f16;
-//  * weights: (q - 32) * sc with the signed scale split sc = 16*sh + sl
-//    (sl = sc & 15, sh = sc >> 4), two f16 planes per K-step:
-//      (q - 32) * sl        |.| <= 480,  an integer, exact in f16;
-//      (q - 32) * 16 * sh   a multiple of 16 with |.| <= 4096, exact in f16.
-//    Every product with a code (|q8| <= 128) is exact in fp32; each plane has
-//    its own fp32 accumulator per super-block, whose sums stay exact integers
-//    (below 2^24, or multiples of 16 below 2^28), and is = lo + hi in int32.
-// The 210-byte blocks start at odd 2-byte offsets; ghip_q6K_repack rewrites
-// them (per call, or once for a registered weight) into aligned 336-byte
-// records:  q[256] (6-bit values 0..63 in element order) | 16 x (f16 sl,
-// f16 16*sh) | d f32 | pad.
-constexpr int Q6R_BYTES = 336;
-
-// one 64-lane group per block: the block's bytes arrive with coalesced dword
-// loads from its 4-byte-aligned base into LDS, then lane u writes elements
-// 4u .. 4u+3 (and lanes 0..19 the scale pairs, d and padding)
-extern "C" __global__ void __launch_bounds__(256)
-ghip_q6K_repack(const uint8_t *__restrict__ W, int64_t w_row_bytes, int N, int nb, uint8_t *__restrict__ out) {
-    __shared__ uint32_t stage[4][56];  // 224 bytes per group
-    const int grp = threadIdx.x >> 6, u = threadIdx.x & 63;
-    const int64_t blk = (int64_t)blockIdx.x * 4 + grp;  // row * nb + block
-    const bool live = blk < (int64_t)N * nb;
-    const int64_t row = live ? blk / nb : 0;
-    const int b = live ? (int)(blk - row * nb) : 0;
-    const uint8_t *src = W + row * w_row_bytes + (int64_t)b * Q6K_BYTES;
-    const uintptr_t base4 = (uintptr_t)src & ~(uintptr_t)3;
-    const int sh = (int)((uintptr_t)src - base4);  // 0 or 2
-    const uintptr_t end = (uintptr_t)(W + (int64_t)(N - 1) * w_row_bytes + (int64_t)nb * Q6K_BYTES);
-    // dwords 0..53 cover the block's 210 bytes plus the shift; none past the matrix
-    if (live && u < 54 && base4 + 4 * u + 4 <= end)
-        stage[grp][u] = *reinterpret_cast<const uint32_t *>(base4 + 4 * u);
-    __syncthreads();
-    if (!live) return;
-    const uint8_t *blkb = reinterpret_cast<const uint8_t *>(stage[grp]) + sh;
-    uint8_t *dst = out + blk * Q6R_BYTES;
-    // element i of half j = i / 128, l = i % 128: ql[64j + l % 64] nibble l / 64,
-    // qh[32j + l % 32] bits 2 * (l / 32) (dequantize_row_q6_K)
-    const int e4 = 4 * u, j = e4 >> 7, l = e4 & 127;
-    const uint8_t *ql = blkb + 64 * j + (l & 63);
-    const uint8_t *qh = blkb + 128 + 32 * j + (l & 31);
-    const int nsh = 4 * (l >> 6), hsh = 2 * (l >> 5);
-    uint32_t v = 0;
-#pragma unroll
-    for (int k = 0; k < 4; k++) v |= (uint32_t)(((ql[k] >> nsh) & 15) | (((qh[k] >> hsh) & 3) << 4)) << (8 * k);
-    *reinterpret_cast<uint32_t *>(dst + e4) = v;
-    if (u < 16) {
-        // sub-block u's signed scale split 16 * sh + sl, as the f16 pair
-        // (sl, 16 * sh) the GEMM multiplies the weight planes by
-        const int sc = (int)(int8_t)blkb[192 + u];
-        const int sl = sc & 15;
-        const _Float16 fl = (_Float16)(float)sl, fh = (_Float16)(float)(sc - sl);
-        *reinterpret_cast<uint32_t *>(dst + 256 + 4 * u) =
-            (uint32_t)__builtin_bit_cast(uint16_t, fl) | ((uint32_t)__builtin_bit_cast(uint16_t, fh) << 16);
-    } else if (u == 16) {
-        *reinterpret_cast<float *>(dst + 320) = h2f((uint32_t)blkb[208] | ((uint32_t)blkb[209] << 8));
-    } else if (u < 20) {
-        *reinterpret_cast<uint32_t *>(dst + 324 + 4 * (u - 17)) = 0u;
-    }
-}
-
-// Q8_K rows -> f16 codes [Mpad][K] and block scales dT [nb][Mpad] (tokens padded
-// to a multiple of 128); one wavefront per (token, super-block)
-extern "C" __global__ void __launch_bounds__(256)
-ghip_gemm_act_layout_f16(const uint8_t *__restrict__ q8k, int64_t row_bytes, int M, int Mpad, int nb,
-                         _Float16 *__restrict__ codes, float *__restrict__ dT) {
-    const int64_t task = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
-    if (task >= (int64_t)M * nb) return;
-    const int m = (int)(task / nb), b = (int)(task % nb);
-    const uint8_t *blk = q8k + (int64_t)m * row_bytes + (int64_t)b * Q8K_BYTES;
-    const uint32_t c4 = ld4(blk + 4 + 4 * lane);
-    _Float16 *o = codes + (int64_t)m * nb * QK_K + b * QK_K + 4 * lane;
-#pragma unroll
-    for (int k = 0; k < 4; k++) o[k] = (_Float16)(float)(int8_t)(c4 >> (8 * k));
-    if (lane == 0) dT[(int64_t)b * Mpad + m] = __uint_as_float(ld4(blk));
-}
-
-namespace g6 {
-constexpr int BM = 64, BN = 128;
-struct Smem {
-    _Float16 act[2][BM * QK_K];     // [stage][token][256], 16-byte slots swizzled by token % 32
-    uint8_t w[2][BN * Q6R_BYTES];   // [stage][row][336]
-    float da[3][BM];                // block scales of the tokens, a 3-slot ring
-};
-}  // namespace g6
-typedef _Float16 v2h __attribute__((ext_vector_type(2)));
-
-// 64 tokens x 128 rows per 256-thread workgroup; wavefront w owns rows
-// 32w .. 32w+31 and both 32-token tiles.  K-step ks (16 elements of
-// sub-block ks): lane l takes elements 16ks + 8(l/32) .. +7 of row l % 32 (B)
-// and of token l % 32 of each tile (A).
-template <bool SUBSUMS>
-__device__ __forceinline__ void gemm_q6K_impl(const uint8_t *__restrict__ R, int N, int nb,
-                                              const _Float16 *__restrict__ codes, const float *__restrict__ dT,
-                                              int M, int Mpad, float *__restrict__ dst, int64_t ldd,
-                                              int32_t *__restrict__ sub) {
-    constexpr int BM = g6::BM, BN = g6::BN;
-    extern __shared__ __attribute__((aligned(16))) uint8_t smem_raw[];
-    g6::Smem &SM = *reinterpret_cast<g6::Smem *>(smem_raw);
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int li = lane & 31, h = lane >> 5;
-    const int64_t K = (int64_t)nb * QK_K;
-    const int n_tiles_m = (M + BM - 1) / BM, n_tiles_n = (N + BN - 1) / BN;
-    const int total = n_tiles_m * n_tiles_n;
-    int id = blockIdx.x;
-    if (total % 8 == 0) id = (blockIdx.x & 7) * (total >> 3) + (blockIdx.x >> 3);
-    const int m0 = (id % n_tiles_m) * BM;
-    const int n0 = (id / n_tiles_m) * BN;
-
-    // buffer descriptors over this tile's activations, weight records and
-    // block scales; the per-lane offsets are fixed, super-block b adds a
-    // scalar offset.  Weight rows past N read as zeros (range-checked).
-    const brsrc ra = make_rsrc(codes + (int64_t)m0 * K, (uint32_t)((int64_t)BM * K * 2));
-    const brsrc rw = make_rsrc(R + (int64_t)n0 * nb * Q6R_BYTES, (uint32_t)((int64_t)min(BN, N - n0) * nb * Q6R_BYTES));
-    const brsrc rd = make_rsrc(dT + m0, (uint32_t)(((int64_t)nb * Mpad - m0) * 4));
-    uint32_t va[8], vw[11];
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-        const int tok = 2 * (8 * wave + i) + (lane >> 5);
-        const int slot = (lane & 31) ^ (tok & 31);
-        va[i] = (uint32_t)tok * (uint32_t)K * 2u + 16u * (uint32_t)slot;
-    }
-#pragma unroll
-    for (int i = 0; i < 11; i++) {
-        const int c = 64 * (4 * i + wave) + lane;
-        const int row = c / 21, k16 = c - 21 * row;
-        vw[i] = (uint32_t)row * (uint32_t)nb * Q6R_BYTES + 16u * (uint32_t)k16;
-    }
-
-    // ---- direct loads of super-block b: wavefront w moves act pieces
-    // 8w .. 8w+7 (2 tokens each), weight pieces w, w+4, .. (64 16-byte
-    // chunks each, 21 per row) and (w = 0) the block scales
-    auto issue = [&](int b, int p) {
-#pragma unroll
-        for (int i = 0; i < 8; i++)
-            b2lds(ra, reinterpret_cast<uint8_t *>(SM.act[p]) + 1024 * (8 * wave + i), va[i], (uint32_t)b * 512u);
-#pragma unroll
-        for (int i = 0; i < 11; i++) {
-            const int g = 4 * i + wave;  // 42 groups of 64 chunks
-            if (g < BN * (Q6R_BYTES / 16) / 64) b2lds(rw, SM.w[p] + 1024 * g, vw[i], (uint32_t)b * Q6R_BYTES);
-        }
-        if (wave == 0 && lane < BM / 4) b2lds(rd, SM.da[b % 3], 16u * lane, (uint32_t)b * (uint32_t)Mpad * 4u);
-    };
-
-    v16f out[2];
-#pragma unroll
-    for (int tm = 0; tm < 2; tm++)
-#pragma unroll
-        for (int v = 0; v < 16; v++) out[tm][v] = 0.0f;
-    const int wr = 32 * wave + li;  // this lane's weight row (B operand column)
-    const uint32_t aoff[2] = {(uint32_t)li * QK_K, (uint32_t)(32 + li) * QK_K};  // halfs
-    const uint32_t asw = (uint32_t)(li & 31);
-    const v2h bias = {(_Float16)-1056.0f, (_Float16)-1056.0f};  // 1024 + 32
-
-    issue(0, 0);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    for (int b = 0; b < nb; b++) {
-        const int p = b & 1;
-        if (b + 1 < nb) issue(b + 1, p ^ 1);
-        const uint8_t *wrow = SM.w[p] + wr * Q6R_BYTES;
-        const float dw = *reinterpret_cast<const float *>(wrow + 320);
-        // One accumulator per scale plane: the low plane's sums stay below
-        // 256 * 480 * 127 < 2^24 and the high plane's are multiples of 16
-        // below 256 * 4096 * 127 < 2^28, so both are exact integers in fp32
-        // for any valid block, and so is is = lo + hi added as int32.
-        v16f accl[2], acch[2];
-        const v16f zf = {};
-#pragma unroll
-        for (int tm = 0; tm < 2; tm++) {
-            accl[tm] = zf;
-            acch[tm] = zf;
-        }
-#pragma unroll 16
-        for (int ks = 0; ks < 16; ks++) {
-            const uint2 qv = *reinterpret_cast<const uint2 *>(wrow + 16 * ks + 8 * h);
-            // the sub-block's signed scale split 16 * sh + sl, as f16 pairs
-            const uint32_t sp = *reinterpret_cast<const uint32_t *>(wrow + 256 + 4 * ks);
-            const v2h pl = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(sp, sp, 0x01000100u));
-            const v2h ph = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(sp, sp, 0x03020302u));
-            v8h blo, bhi;
-            const uint32_t qw[2] = {qv.x, qv.y};
-#pragma unroll
-            for (int d = 0; d < 2; d++) {
-                // bytes q -> f16 (1024 + q) by placing 0x64 above each byte, then - 1056
-                const v2h e0 = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(0x64646464u, qw[d], 0x04010400u)) + bias;
-                const v2h e1 = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(0x64646464u, qw[d], 0x04030402u)) + bias;
-                const v2h l0 = e0 * pl, l1 = e1 * pl, h0 = e0 * ph, h1 = e1 * ph;
-                blo[4 * d] = l0[0]; blo[4 * d + 1] = l0[1]; blo[4 * d + 2] = l1[0]; blo[4 * d + 3] = l1[1];
-                bhi[4 * d] = h0[0]; bhi[4 * d + 1] = h0[1]; bhi[4 * d + 2] = h1[0]; bhi[4 * d + 3] = h1[1];
-            }
-#pragma unroll
-            for (int tm = 0; tm < 2; tm++) {
-                const v8h a = *reinterpret_cast<const v8h *>(SM.act[p] + aoff[tm] + 8 * ((uint32_t)(2 * ks + h) ^ asw));
-                accl[tm] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, blo, accl[tm], 0, 0, 0);
-                acch[tm] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, bhi, acch[tm], 0, 0, 0);
-            }
-        }
-        // ---- out += (d * is) * d8 (vec_dot_q6_K_q8_K's per-block order)
-        const float *dab = SM.da[b % 3];
-#pragma unroll
-        for (int tm = 0; tm < 2; tm++) {
-#pragma unroll
-            for (int v = 0; v < 16; v++) {
-                const int tl = 32 * tm + crow(v, lane);
-                const int isi = (int)accl[tm][v] + (int)acch[tm][v];
-                if constexpr (SUBSUMS)
-                    if (m0 + tl < M && n0 + wr < N) sub[((int64_t)(m0 + tl) * N + (n0 + wr)) * nb + b] = isi;
-                out[tm][v] = fmaf(dw * (float)isi, dab[tl], out[tm][v]);
-            }
-        }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // super-block b+1 is in LDS
-        __syncthreads();
-    }
-    const int n = n0 + wr;
-#pragma unroll
-    for (int tm = 0; tm < 2; tm++)
-#pragma unroll
-        for (int v = 0; v < 16; v++) {
-            const int m = m0 + 32 * tm + crow(v, lane);
-            if (m < M && n < N) dst[(int64_t)m * ldd + n] = out[tm][v];
-        }
-}
-extern "C" __global__ void __launch_bounds__(256, 1)
-    ghip_gemm_q6_K(const uint8_t *__restrict__ R, int N, int nb, const _Float16 *__restrict__ codes,
-                   const float *__restrict__ dT, int M, int Mpad, float *__restrict__ dst, int64_t ldd,
-                   int32_t *__restrict__ sub) {
-    gemm_q6K_impl<false>(R, N, nb, codes, dT, M, Mpad, dst, ldd, sub);
-}
-extern "C" __global__ void __launch_bounds__(256, 1)
-    ghip_gemm_q6_K_sub(const uint8_t *__restrict__ R, int N, int nb, const _Float16 *__restrict__ codes,
-                       const float *__restrict__ dT, int M, int Mpad, float *__restrict__ dst, int64_t ldd,
-                       int32_t *__restrict__ sub) {
-    gemm_q6K_impl<true>(R, N, nb, codes, dT, M, Mpad, dst, ldd, sub);
-}
-static_assert(sizeof(g6::Smem) == 152320, "host code launches with this LDS size");
-
 // split-K partial sums [nsplit][M][N] -> dst, slices added in order; four
 // consecutive outputs per thread (N % 4 == 0)
 extern "C" __global__ void __launch_bounds__(256)
@@ -839,19 +593,21 @@ ghip_gemm_splitk_reduce(const float *__restrict__ part, int nsplit, int M, int N
     const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
     if (i >= (int64_t)M * N) return;
     const int m = (int)(i / N), n = (int)(i % N);
-    float4 acc = *reinterpret_cast<const float4 *>(part + i);
+    float acc[4], lost[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // lost: what the sum's roundings dropped, carried along
+    __builtin_memcpy(acc, part + i, 16);
     for (int z = 1; z < nsplit; z++) {
-        const float4 v = *reinterpret_cast<const float4 *>(part + (int64_t)z * M * N + i);
-        acc.x += v.x;
-        acc.y += v.y;
-        acc.z += v.z;
-        acc.w += v.w;
+        float v[4];
+        __builtin_memcpy(v, part + (int64_t)z * M * N + i, 16);
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const float y = v[k] + lost[k], t = acc[k] + y;
+            lost[k] = y - (t - acc[k]);
+            acc[k] = t;
+        }
     }
     float *d = dst + (int64_t)m * ldd + n;
-    d[0] = acc.x;
-    d[1] = acc.y;
-    d[2] = acc.z;
-    d[3] = acc.w;
+#pragma unroll
+    for (int k = 0; k < 4; k++) d[k] = acc[k];
 }
 static_assert(sizeof(g3::Smem<128>) == 116224 && sizeof(g3::Smem<64>) == 76544, "host code launches with these LDS sizes");
 static_assert(2 * sizeof(g4::Stage<256>) == 148480, "host code launches with this LDS size");
@@ -873,12 +629,10 @@ extern "C" __global__ void __launch_bounds__(512, 1)
 // ghip_quantize_q8_K (same arithmetic, ghip_q8k.h) written directly in the
 // GEMM layouts, so the Q8_K rows never go through HBM.  One wavefront per
 // (token, super-block); rows m < n_mat take the quantize_mat_q8_K_4x8 values.
-//   F16 = false (Q4_K GEMM): codes [Mpad][K] int8 | bsT [nb][Mpad][16] f16 | dT [nb][Mpad]
-//   F16 = true  (Q6_K GEMM): codes [Mpad][K] f16  | dT [nb][Mpad]
-template <bool F16>
-__device__ __forceinline__ void act_q8K_layout(const float *__restrict__ x, int64_t x_stride, int M, int Mpad, int nb,
-                                               int n_mat, void *__restrict__ codes, _Float16 *__restrict__ bsT,
-                                               float *__restrict__ dT) {
+//   codes [Mpad][K] int8 | bsT [nb][Mpad][16] f16 | dT [nb][Mpad]
+extern "C" __global__ void __launch_bounds__(256)
+ghip_gemm_act_q8K(const float *__restrict__ x, int64_t x_stride, int M, int Mpad, int nb, int n_mat,
+                  int8_t *__restrict__ codes, _Float16 *__restrict__ bsT, float *__restrict__ dT) {
     const int64_t task = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     if (task >= (int64_t)M * nb) return;
@@ -888,29 +642,12 @@ __device__ __forceinline__ void act_q8K_layout(const float *__restrict__ x, int6
     int q[4];
     float d;
     q8K_block(xs, lane, m < n_mat, q, d);
-    const int64_t e = (int64_t)m * nb * QK_K + (int64_t)b * QK_K + 4 * lane;
-    if constexpr (F16) {
-        typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-        const h4 v = {(_Float16)(float)q[0], (_Float16)(float)q[1], (_Float16)(float)q[2], (_Float16)(float)q[3]};
-        *reinterpret_cast<h4 *>(reinterpret_cast<_Float16 *>(codes) + e) = v;
-    } else {
-        const uint32_t packed = (uint32_t)(q[0] & 0xff) | ((uint32_t)(q[1] & 0xff) << 8) |
-                                ((uint32_t)(q[2] & 0xff) << 16) | ((uint32_t)(q[3] & 0xff) << 24);
-        *reinterpret_cast<uint32_t *>(reinterpret_cast<int8_t *>(codes) + e) = packed;
-        const int s = q8K_bsum16(q, lane);
-        if ((lane & 3) == 0) bsT[((int64_t)b * Mpad + m) * 16 + (lane >> 2)] = (_Float16)(float)s;
-    }
+    const uint32_t packed = (uint32_t)(q[0] & 0xff) | ((uint32_t)(q[1] & 0xff) << 8) |
+                            ((uint32_t)(q[2] & 0xff) << 16) | ((uint32_t)(q[3] & 0xff) << 24);
+    *reinterpret_cast<uint32_t *>(codes + (int64_t)m * nb * QK_K + (int64_t)b * QK_K + 4 * lane) = packed;
+    const int s = q8K_bsum16(q, lane);
+    if ((lane & 3) == 0) bsT[((int64_t)b * Mpad + m) * 16 + (lane >> 2)] = (_Float16)(float)s;
     if (lane == 0) dT[(int64_t)b * Mpad + m] = d;
-}
-extern "C" __global__ void __launch_bounds__(256)
-ghip_gemm_act_q8K(const float *__restrict__ x, int64_t x_stride, int M, int Mpad, int nb, int n_mat,
-                  int8_t *__restrict__ codes, _Float16 *__restrict__ bsT, float *__restrict__ dT) {
-    act_q8K_layout<false>(x, x_stride, M, Mpad, nb, n_mat, codes, bsT, dT);
-}
-extern "C" __global__ void __launch_bounds__(256)
-ghip_gemm_act_q8K_f16(const float *__restrict__ x, int64_t x_stride, int M, int Mpad, int nb, int n_mat,
-                      _Float16 *__restrict__ codes, float *__restrict__ dT) {
-    act_q8K_layout<true>(x, x_stride, M, Mpad, nb, n_mat, codes, nullptr, dT);
 }
 
 // ------------------------------------------------- Q4_0 / Q5_0 / Q8_0 prefill

@@ -1,0 +1,115 @@
+"""The Q2_K / Q3_K / Q6_K prefill GEMM (ghip_kq.hip): integer super-block sums
+equal to the oracle's, f32 results against 64-bit sums of the same terms."""
+import numpy as np
+import pytest
+
+import oracle_lib as O
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+# bytes of a block, offsets of d and dmin
+BLOCK = {O.Q2_K: (84, 80, 82), O.Q3_K: (110, 108, None), O.Q6_K: (210, 208, None)}
+
+
+@pytest.fixture(scope="module")
+def be():
+    import ghip
+    b = ghip.Backend(0)
+    yield b
+    b.close()
+
+
+def weights(ty, rows, k, seed):
+    """random bytes (every scale and code, the extremes among them) with small
+    finite d / dmin"""
+    rng = np.random.default_rng(seed)
+    size, *at = BLOCK[ty]
+    w = rng.integers(0, 256, (rows, k // 256, size), dtype=np.uint8)
+    for o in at:
+        if o is not None:
+            w[:, :, o:o + 2] = (rng.random((rows, k // 256)) * 0.01).astype(np.float16).view(np.uint8).reshape(rows, -1, 2)
+    return w.reshape(rows, -1)
+
+
+def exact(ty, w, k, sub, act):
+    """float64 results and the summed magnitudes of their terms"""
+    size, at_d, at_m = BLOCK[ty]
+    blk = w.reshape(w.shape[0], k // 256, size)
+    f16 = lambda o: blk[:, :, o:o + 2].copy().view(np.float16)[..., 0].astype(np.float64)
+    d8 = act.reshape(act.shape[0], k // 256, 292)[:, :, :4].copy().view(np.float32)[..., 0].astype(np.float64)
+    if at_m is not None:
+        a, b = f16(at_d) * sub[..., 0], f16(at_m) * sub[..., 1]
+    else:
+        a, b = f16(at_d) * sub, 0.0
+    return ((a - b) * d8[:, None, :]).sum(-1), ((np.abs(a) + np.abs(b)) * np.abs(d8)[:, None, :]).sum(-1)
+
+
+@pytest.mark.parametrize("ty", [O.Q2_K, O.Q3_K, O.Q6_K])
+@pytest.mark.parametrize("M,N,K", [
+    (17, 24, 256),     # fewer rows than one 32-row tile, one super-block
+    (64, 128, 512),    # one whole workgroup
+    (65, 129, 1280),   # one row and one token past it; N % 4: no K split
+    (33, 200, 2304),   # K split with a short last slice
+    (130, 160, 4096),
+])
+def test_gemm(be, ty, M, N, K):
+    if ty == O.Q6_K:
+        M += 64  # its GEMM's range
+    w = weights(ty, N, K, M + N)
+    x = np.random.default_rng(K).standard_normal((M, K + 4)).astype(np.float32)
+    wd, xd = torch.from_numpy(w).cuda(), torch.from_numpy(x).cuda()[:, :K]
+    print(f"kq gemm type={ty} M={M} N={N} K={K}", flush=True)
+    act = be.mul_mat_act(wd, ty, K, xd).cpu().numpy()
+    want_sub = np.asarray(O.mul_mat(ty, w, K, N, np.ascontiguousarray(x[:, :K]), M, want_subsums=True)[2])
+    out = torch.full((M + 1, N + 4), 7.0, device="cuda")
+    got = be.mul_mat(wd, ty, K, xd, out=out[:M, :N]).cpu().numpy()
+    sub = be.mul_mat_subsums(wd, ty, K, xd).cpu().numpy()
+    assert np.array_equal(sub, want_sub.reshape(sub.shape))
+    want, mag = exact(ty, w, K, sub.astype(np.float64), act)
+    # three roundings a term, then at most 4 + nb / 4 + 2 additions (K slices included)
+    assert np.all(np.abs(got - want) <= (4 + 4 + K // 1024 + 2) * 2.0 ** -23 * mag)
+    assert bool((out[M] == 7.0).all()) and bool((out[:, N:] == 7.0).all())
+    # the kept records, and Q8_K rows in src1, give the same bits
+    be.register_weight(wd, ty, K)
+    again = be.mul_mat(wd, ty, K, xd).cpu().numpy()
+    pre = be.mul_mat(wd, ty, K, torch.from_numpy(act).cuda()).cpu().numpy()
+    be.unregister_weight(wd, ty, K)
+    assert np.array_equal(again, got) and np.array_equal(pre, got)
+
+
+@pytest.mark.parametrize("ty", [O.Q2_K, O.Q3_K])
+def test_small_workspace(be, ty):
+    """A caller's workspace too small for the GEMM's layout still serves the
+    call: without the K split, then on the decode kernels."""
+    import ghip
+    M, N, K = 20, 128, 4096
+    w = weights(ty, N, K, 5)
+    x = np.random.default_rng(6).standard_normal((M, K)).astype(np.float32)
+    wd, xd = torch.from_numpy(w).cuda(), torch.from_numpy(x).cuda()
+    out = torch.empty((M, N), device="cuda")
+    full = be.workspace_size(ghip.mul_mat_node(wd, ty, K, xd, out))
+    ref = be.mul_mat(wd, ty, K, xd).cpu().numpy()
+    sub = be.mul_mat_subsums(wd, ty, K, xd).cpu().numpy().astype(np.float64)
+    want, mag = exact(ty, w, K, sub, be.mul_mat_act(wd, ty, K, xd).cpu().numpy())
+    for n in (full, full - 1, M * K // 256 * 292):
+        be.set_workspace(torch.empty(n, dtype=torch.uint8, device="cuda"))
+        got = be.mul_mat(wd, ty, K, xd).cpu().numpy()
+        be.set_workspace(None)
+        assert n != full or np.array_equal(got, ref)
+        # (the decode kernels: three roundings a term, 8 additions)
+        assert np.all(np.abs(got - want) <= 16 * 2.0 ** -23 * mag)
+    # capture may not grow the workspace: a fresh context's small one serves
+    be2 = ghip.Backend(0)
+    be2.mul_mat(wd, ty, K, xd[:8], out=out[:8])
+    g = torch.cuda.CUDAGraph()
+    be2.mul_mat_act(wd, ty, K, xd)
+    with torch.cuda.graph(g):
+        be2.mul_mat(wd, ty, K, xd[:17], out=out[:17])
+    for _ in range(3):
+        out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert np.all(np.abs(out[:17].cpu().numpy() - want[:17]) <= 16 * 2.0 ** -23 * mag[:17])
+    del g
+    be2.close()
