@@ -312,8 +312,8 @@ ghip_status ghip_workspace_size(int op, const ghip_tensor *dst, const ghip_tenso
  * and keep device-side copies of it in the layouts the kernels read, built
  * once on `stream` now instead of on every call -- the reference's repack
  * cache (repack_*_cached, crates/ggml/src/repack.rs:4250-4480, and the
- * CPU_REPACK buffer it stands for).  Today those are the Q6_K prefill
- * GEMM's aligned 336-byte records, the Q4_0 / Q5_0 / Q8_0 prefill GEMM's
+ * CPU_REPACK buffer it stands for).  Today those are the Q2_K / Q3_K / Q6_K
+ * prefill GEMM's records (about 1.1 bytes a weight), the Q4_0 / Q5_0 / Q8_0 prefill GEMM's
  * int8 code plane with its f32 block scales, and (3-D MXFP4 expert weights)
  * the MUL_MAT_ID kernel's 80-byte windows; other types are read in their
  * GGUF layout and register as a no-op.  Later MUL_MAT calls whose src0 has the same data

@@ -75,6 +75,11 @@ DEV float h2f(uint32_t bits16) {
     return __half2float(__ushort_as_half((unsigned short)(bits16 & 0xffffu)));
 }
 
+// What the rounding of a sum dropped, carried along to the next term: x, but some
+// finite number where the sum is infinite and x no longer is one (inf - inf), so
+// that the sum stays infinite (of a finite sum |x| < 2^104).
+DEV float sum_lost(float x) { return __builtin_amdgcn_fmed3f(x, -0x1p104f, 0x1p104f); }
+
 // 16 bytes per lane from global memory straight into LDS at lds + 16 * lane
 // (global_load_lds_dwordx4; lds is wave-uniform). The data is in LDS once the
 // issuing wavefront's vmcnt reaches zero.

@@ -601,7 +601,7 @@ ghip_gemm_splitk_reduce(const float *__restrict__ part, int nsplit, int M, int N
 #pragma unroll
         for (int k = 0; k < 4; k++) {
             const float y = v[k] + lost[k], t = acc[k] + y;
-            lost[k] = y - (t - acc[k]);
+            lost[k] = sum_lost(y - (t - acc[k]));
             acc[k] = t;
         }
     }

@@ -203,6 +203,8 @@ __device__ __forceinline__ void gemm_kq_impl(const uint8_t *__restrict__ R, int 
         for (int t = 0; t < 2; t++) {
             const v16f y = part[t] + comp[t], s2 = sum[t] + y;
             comp[t] = y - (s2 - sum[t]);
+#pragma unroll
+            for (int v = 0; v < 16; v++) comp[t][v] = sum_lost(comp[t][v]);
             sum[t] = s2;
             part[t] = v16f{};
         }

@@ -9,7 +9,7 @@ torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
 
 # bytes of a block, offsets of d and dmin
-BLOCK = {O.Q2_K: (84, 80, 82), O.Q3_K: (110, 108, None), O.Q6_K: (210, 208, None)}
+BLOCK = {O.Q2_K: (84, 80, 82), O.Q3_K: (110, 108, None), O.Q6_K: (210, 208, None), O.Q4_K: (144, 0, 2)}
 
 
 @pytest.fixture(scope="module")
@@ -76,6 +76,29 @@ def test_gemm(be, ty, M, N, K):
     pre = be.mul_mat(wd, ty, K, torch.from_numpy(act).cuda()).cpu().numpy()
     be.unregister_weight(wd, ty, K)
     assert np.array_equal(again, got) and np.array_equal(pre, got)
+
+
+@pytest.mark.parametrize("ty,M", [(O.Q2_K, 20), (O.Q3_K, 20), (O.Q6_K, 70), (O.Q4_K, 150)])
+def test_infinite_scale(be, ty, M):
+    """A block scale of infinity gives infinities (NaN where its sum is 0 or two
+    of them cancel), K split and not, and leaves the other rows alone."""
+    K, N = 4096, 136
+    w = weights(ty, N, K, 9)
+    size, at_d, _ = BLOCK[ty]
+    blk = w.reshape(N, K // 256, size)
+    for row, bs in ((3, (0,)), (40, (5,)), (100, (15,)), (135, (2, 9))):
+        for b in bs:
+            blk[row, b, at_d:at_d + 2] = np.array([np.inf], np.float16).view(np.uint8)
+    x = np.random.default_rng(8).standard_normal((M, K)).astype(np.float32)
+    wd, xd = torch.from_numpy(w).cuda(), torch.from_numpy(x).cuda()
+    got = be.mul_mat(wd, ty, K, xd).cpu().numpy()
+    sub = be.mul_mat_subsums(wd, ty, K, xd).cpu().numpy().astype(np.float64)
+    with np.errstate(invalid="ignore"):
+        want, _ = exact(ty, w, K, sub, be.mul_mat_act(wd, ty, K, xd).cpu().numpy())
+    assert np.isinf(want).any() and np.isfinite(want).any()
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(np.where(np.isinf(want), got, 0), np.where(np.isinf(want), want, 0))
+    assert np.isfinite(got[np.isfinite(want)]).all()
 
 
 @pytest.mark.parametrize("ty", [O.Q2_K, O.Q3_K])
