@@ -1162,6 +1162,10 @@ ghip_status run_gemm(ghip_context *ctx, const MulMatPlan &p, const void *w, cons
                        (int)p.N, dst, (int64_t)ldd);
 }
 
+// wavefronts that share K in a 32 x 32 tile of the K-quant experts: 8 where the
+// tiles are few (1536 x 2048 Q4_K, 8 pairs: less to wait for per tile)
+int kq32_waves(int64_t tiles, int64_t nb) { return tiles <= 256 && nb >= 8 ? 8 : 4; }
+
 bool use_gemm(const MulMatPlan &p) {
     if (p.M > INT32_MAX) return false;
     if (p.wtype == GHIP_TYPE_Q4_K) return p.M >= env_int("GHIP_GEMM_MIN_ROWS", 16);
@@ -1715,9 +1719,12 @@ ghip_status mul_mat_id_impl(ghip_context *ctx, const ghip_tensor *as, const ghip
     if (st != GHIP_STATUS_SUCCESS) return st;
     if (kq) {
         const char *tn = p.wtype == GHIP_TYPE_Q4_K ? "q4_K" : p.wtype == GHIP_TYPE_Q5_K ? "q5_K" : "q6_K";
-        const std::string name = std::string("ghip_mmid_") + tn + (sub ? "_sub" : "");
-        const dim3 grid((unsigned)max_tiles, (unsigned)((p.rows + 15) / 16));
-        return ctx->launch(name, grid, dim3(256), 0, s, (const uint8_t *)as->data, (int64_t)as->nb[1],
+        // (about as many tiles as the experts that can be met)
+        const int64_t blocks = (p.rows + 31) / 32, tiles = std::min(p.n_as, n_pairs) + n_pairs / 32;
+        const int kw = sub ? 4 : kq32_waves(tiles * blocks, p.nb);
+        const std::string name = std::string("ghip_mmid_") + tn + (sub ? "_sub" : kw == 8 ? "_k8" : "_k4");
+        const dim3 grid((unsigned)max_tiles, (unsigned)blocks);
+        return ctx->launch(name, grid, dim3(64 * kw), 0, s, (const uint8_t *)as->data, (int64_t)as->nb[1],
                            (int64_t)as->nb[2], (const uint8_t *)act, p.act_row_bytes, (int)p.ne11,
                            (const int32_t *)route, (int)n_pairs, (int)p.n_ids, dst, dst_nb1, dst_nb2, (int)p.rows,
                            (int)p.nb, sub);

@@ -16,6 +16,7 @@
 // is bit-identical to the reference's repack route.
 #include <type_traits>
 #include "ghip_common.h"
+#include "ghip_kplanes.h"
 
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef float v16f __attribute__((ext_vector_type(16)));
@@ -853,103 +854,185 @@ ghip_mxfp4_repack(const uint8_t *__restrict__ W, int64_t nb1, int64_t nb2, int r
 // MUL_MAT_ID with Q4_K, Q5_K or Q6_K experts (forward_mul_mat_id,
 // compute.rs:1917-2202): the activation rows quantized once to Q8_K
 // (quantize_row_q8_K, the reference's wdata pass), the pairs routed by
-// ghip_moe_route, then per (tile, 16 expert rows) one workgroup of four
-// wavefronts, 4 rows each held in registers, walking the tile's pairs.  Per
-// (pair, row) the value is the decode GEMV's: the integer sums of
-// vec_dot_q4_K_q8_K / vec_dot_q5_K_q8_K / vec_dot_q6_K_q8_K per super-block
-// (vec_dot.rs:928-1040) and the same fp32 scaling, summed over the
-// wavefront.  A wavefront covers 16 super-blocks per pass (4 lanes each);
-// wider rows take several passes, their partials added in the lanes first.
-constexpr int MMID_RB = 4;  // rows per wavefront
+// ghip_moe_route, then one workgroup per (tile of at most 32 pairs of an
+// expert, 32 expert rows): C[pair][row] on v_mfma_i32_32x32x32_i8, the expert's
+// rows read once per tile, straight from the GGUF blocks into registers (lane
+// 32h + r: row r, elements 16h .. 16h+15 of every 32).  The KW wavefronts take
+// every KW-th super-block, the next one's loads in flight, and add up in LDS.
+//  * Q4_K / Q5_K: an MFMA gives a 32-element sub-block's exact dots, folded
+//    into the super-block's integer sum by its scale (a lane holds one row, so
+//    one scale, a 24-bit multiply-add); the mins times bsum16 are one f16 MFMA
+//    (exact in f32: m <= 63, |bsum16| <= 2048).
+//  * Q6_K: a lane's 16 elements are one scale group, so the scale goes into the
+//    codes (kq_planes) and the MFMAs sum the whole super-block.
+// Then one f32 scaling per super-block, as vec_dot_q4_K_q8_K and its kin
+// (vec_dot.rs:928-1040).
+//
+// Bound by the expert weights' way from memory; Q4_K, 64 experts of 2048 ->
+// 1536 rows, 64 tokens, top-8 (113 MB): 59 us (1.9 TB/s), 324 with a 64-lane dot per pair and
+// row, which read the expert's rows once per 8 pairs.
+typedef int v16i __attribute__((ext_vector_type(16)));
+constexpr int MMID_BR = 32;  // rows per workgroup
 
-// Lane i's quarter of super-block b: its integer sums (the caller adds the
-// four quarters exactly before any rounding) and the block's scales.
-template <int TYPE>  // 12 Q4_K, 13 Q5_K, 14 Q6_K
-DEV void kq_lane_dot(const uint8_t *__restrict__ wrow, const uint8_t *__restrict__ arow, int b, int i, bool valid,
-                     int32_t *sub_ia, int32_t *sub_im, float *d8o, float *dwo, float *dmo) {
-    if (!valid) return;
-    const uint8_t *ab = arow + (int64_t)b * Q8K_BYTES;
-    const float d8 = __uint_as_float(ld4(ab));
-    *d8o = d8;
-    if constexpr (TYPE == 14) {
-        // lane i: half j = i / 2, 16-element column hh = i % 2 of each quarter q
-        const int j = i >> 1, hh = i & 1;
-        const uint8_t *blk = wrow + (int64_t)b * Q6K_BYTES;
-        const uint4 l0 = ld16(blk + 64 * j + 16 * hh), l1 = ld16(blk + 64 * j + 16 * hh + 32);
-        const uint4 qh = ld16(blk + 128 + 32 * j + 16 * hh);
-        const uint2 scv = ld8(blk + 192 + 8 * j);
-        const float dw = h2f(ld2(blk + 208));
-        const uint32_t la[4] = {l0.x, l0.y, l0.z, l0.w}, lb[4] = {l1.x, l1.y, l1.z, l1.w};
-        const uint32_t hv[4] = {qh.x, qh.y, qh.z, qh.w};
-        int is = 0;
+// One workgroup: C[token][row] of at most 32 tokens (count, a lane's own
+// activation row arow: token li's) and the 32 rows from row - li on (a lane's
+// own row, its weights wrow).  out(i, row) is token i's output for that row,
+// part_of(i) the sub-sums of (token i, row), nb super-blocks.
+template <int TYPE, int KW, bool SUBSUMS, class Out, class Sub>  // 12 Q4_K, 13 Q5_K, 14 Q6_K; KW wavefronts
+__device__ __forceinline__ void kq32_tile(const uint8_t *__restrict__ wrow, int row, int rows,
+                                          const uint8_t *__restrict__ arow, int count, int nb, Out out, Sub part_of) {
+    constexpr bool Q5 = TYPE == 13, Q6 = TYPE == 14;
+    constexpr int NW = Q6 ? 6 : Q5 ? 5 : 4;  // 16-byte pieces of codes per lane and super-block
+    __shared__ __attribute__((aligned(16))) float d8s[KW][32];
+    __shared__ float red[KW][16][64];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int li = lane & 31, h = lane >> 5;
+    struct Ops {  // one super-block
+        uint4 a[8], bs, hd, w[NW];
+        float d8, dw;
+    };
+    auto load = [&](int b, Ops &o) {
+        const uint8_t *ab = arow + (int64_t)b * Q8K_BYTES;
+        const uint8_t *blk = wrow + (int64_t)b * (Q6 ? Q6K_BYTES : Q5 ? 176 : Q4K_BYTES);
+        if constexpr (Q6) {
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const uint4 y = ld16(ab + 4 + 128 * j + 16 * hh + 32 * q);
-            const uint32_t yv[4] = {y.x, y.y, y.z, y.w};
-            int dq = 0;
+            for (int k = 0; k < 4; k++) o.w[k] = ld16(blk + 32 * k + 16 * h);
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                const uint32_t src = (q & 1) ? lb[k] : la[k];
-                const uint32_t nib = (q & 2) ? ((src >> 4) & 0x0f0f0f0f) : (src & 0x0f0f0f0f);
-                dq = dot4(nib | (((hv[k] >> (2 * q)) & 0x03030303) << 4), yv[k], dq);
+            for (int n = 0; n < 2; n++) o.w[4 + n] = ld16(blk + 128 + 32 * n + 16 * h);
+            o.hd = ld16(blk + 192);
+            o.dw = h2f(ld2(blk + 208));
+        } else {
+            o.hd = ld16(blk);
+            if constexpr (Q5) o.w[4] = ld16(blk + 16 + 16 * h);
+#pragma unroll
+            for (int k = 0; k < 4; k++) o.w[k] = ld16(blk + (Q5 ? 48 : 16) + 32 * k + 16 * h);
+            o.bs = ld16(ab + 260 + 16 * h);
+        }
+        o.d8 = __uint_as_float(ld4(ab));
+#pragma unroll
+        for (int c = 0; c < 8; c++) o.a[c] = ld16(ab + 4 + 32 * c + 16 * h);
+    };
+    auto dwords = [](uint4 v, uint32_t (&x)[4]) { x[0] = v.x; x[1] = v.y; x[2] = v.z; x[3] = v.w; };
+    // Q4_K / Q5_K: the sum's and the min product's roundings are carried along
+    // (without, 1.03e-7 from the 64-bit value at K = 14336 where the prefill
+    // GEMM's chain is 0.85e-7)
+    float part[16], lost[16];
+#pragma unroll
+    for (int v = 0; v < 16; v++) part[v] = lost[v] = 0.0f;
+    auto block = [&](int b, const Ops &o) {
+        v16i is;
+        v16f im = {};
+        float dw, dm = 0.0f;
+        if constexpr (Q6) {
+            dw = o.dw;
+            uint32_t sc[4];
+            dwords(o.hd, sc);
+            v16i lo, hi;
+#pragma unroll
+            for (int c = 0; c < 8; c++) {
+                const int n = c >> 2, j = c & 3;  // elements 128n + 32j ..
+                uint32_t l[4], q[4];
+                dwords(o.w[2 * n + (j & 1)], l);
+                dwords(o.w[4 + n], q);
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+                    q[k] = ((l[k] >> (4 * (j >> 1))) & 0x0f0f0f0fu) | (((q[k] >> (2 * j)) & 0x03030303u) << 4);
+                const int s = (int)(int8_t)(sc[c >> 1] >> (16 * (c & 1) + 8 * h));  // group 2c + h
+                v4i pl, ph;
+                kq_planes(make_uint4(q[0], q[1], q[2], q[3]), s, pl, ph);
+                const v4i a = __builtin_bit_cast(v4i, o.a[c]);
+                lo = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, pl, c == 0 ? v16i{} : lo, 0, 0, 0);
+                hi = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, ph, c == 0 ? v16i{} : hi, 0, 0, 0);
             }
-            const int bs32 = 32 * (int)(int16_t)ld2(ab + 260 + 2 * (8 * j + hh + 2 * q));
-            const uint32_t sw = q < 2 ? scv.x : scv.y;
-            const int sc = (int)(int8_t)(sw >> (8 * hh + 16 * (q & 1)));
-            is += sc * (dq - bs32);
-        }
-        *sub_ia = is;
-        *dwo = dw;
-    } else {
-        constexpr bool Q5 = TYPE == 13;
-        constexpr int BB = Q5 ? 176 : Q4K_BYTES;
-        const uint8_t *blk = wrow + (int64_t)b * BB;
-        const uint4 hd = ld16(blk);
-        const uint4 x0 = ld16(blk + (Q5 ? 48 : 16) + 32 * i), x1 = ld16(blk + (Q5 ? 64 : 32) + 32 * i);
-        const float dw = h2f(hd.x), dmin = h2f(hd.x >> 16);
-        int sc0, sc1, m0, m1;
-        k4_scales(hd.y, hd.z, hd.w, scale_sel(i), sc0, sc1, m0, m1);
-        const uint32_t qv[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-        uint32_t lo[8], hi[8];
-#pragma unroll
-        for (int k = 0; k < 8; k++) {
-            lo[k] = qv[k] & 0x0f0f0f0f;
-            hi[k] = (qv[k] >> 4) & 0x0f0f0f0f;
-        }
-        if constexpr (Q5) {
-            const uint4 g0 = ld16(blk + 16), g1 = ld16(blk + 32);
-            const uint32_t hv[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
+            is = hi * 128 + lo;
+        } else {
+            dw = h2f(o.hd.x);
+            dm = h2f(o.hd.x >> 16);
+            // scales and mins of the eight sub-blocks as bytes (get_scale_min_k4)
+            const uint32_t s[2] = {o.hd.y & 0x3f3f3f3fu, (o.hd.w & 0x0f0f0f0fu) | ((o.hd.y >> 2) & 0x30303030u)};
+            const uint32_t m[2] = {o.hd.z & 0x3f3f3f3fu, ((o.hd.w >> 4) & 0x0f0f0f0fu) | ((o.hd.z >> 2) & 0x30303030u)};
+            const uint32_t mh = h ? m[1] : m[0];  // of groups 8h .. 8h+7
+            uint32_t bsw[4];
+            dwords(o.bs, bsw);
+            v8h ba, bm;
 #pragma unroll
             for (int k = 0; k < 8; k++) {
-                const uint32_t q2 = hv[k] >> (2 * i);
-                lo[k] |= (q2 & 0x01010101u) << 4;
-                hi[k] |= (q2 << 3) & 0x10101010u;
+                ba[k] = (_Float16)(short)(bsw[k >> 1] >> (16 * (k & 1)));
+                bm[k] = (_Float16)(unsigned short)((mh >> (8 * (k >> 1))) & 0xffu);
+            }
+            im = __builtin_amdgcn_mfma_f32_32x32x16_f16(ba, bm, im, 0, 0, 0);
+            is = v16i{};
+#pragma unroll
+            for (int c = 0; c < 8; c++) {
+                uint32_t x[4];
+                dwords(o.w[c >> 1], x);
+                v4i q;
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    x[k] = (x[k] >> (4 * (c & 1))) & 0x0f0f0f0fu;
+                    if constexpr (Q5) {
+                        uint32_t hb[4];
+                        dwords(o.w[4], hb);
+                        x[k] |= ((hb[k] >> c) & 0x01010101u) << 4;
+                    }
+                    q[k] = (int)x[k];
+                }
+                const v16i d = __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(v4i, o.a[c]), q, v16i{}, 0, 0, 0);
+                const int sc = (int)((s[c >> 2] >> (8 * (c & 3))) & 0xffu);
+#pragma unroll
+                for (int v = 0; v < 16; v++) is[v] += __mul24(sc, d[v]);
             }
         }
-        const uint4 a0 = ld16(ab + 4 + 64 * i), a1 = ld16(ab + 20 + 64 * i);
-        const uint4 a2 = ld16(ab + 36 + 64 * i), a3 = ld16(ab + 52 + 64 * i);
-        const uint32_t al[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
-        const uint32_t ah[8] = {a2.x, a2.y, a2.z, a2.w, a3.x, a3.y, a3.z, a3.w};
-        int dl = 0, dh = 0;
+        d8s[w][li] = o.d8;  // (this wavefront's own row: no barrier)
 #pragma unroll
-        for (int k = 0; k < 8; k++) {
-            dl = dot4(lo[k], al[k], dl);
-            dh = dot4(hi[k], ah[k], dh);
+        for (int q = 0; q < 4; q++) {
+            const float4 d4 = *reinterpret_cast<const float4 *>(&d8s[w][8 * q + 4 * h]);
+            const float dd[4] = {d4.x, d4.y, d4.z, d4.w};
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const int v = 4 * q + k;
+                if constexpr (Q6) {
+                    part[v] = fmaf(dw * (float)is[v], dd[k], part[v]);
+                } else {
+                    const float t = dm * im[v], e = sum_lost(fmaf(dm, im[v], -t));
+                    const float y = fmaf(fmaf(dw, (float)is[v], -t) - e, dd[k], lost[v]), z = part[v] + y;
+                    lost[v] = sum_lost(y - (z - part[v]));
+                    part[v] = z;
+                }
+                if constexpr (SUBSUMS) {
+                    const int pi = crowm(v, lane);
+                    if (pi < count && row < rows) {
+                        int32_t *sp = part_of(pi) + b * (Q6 ? 1 : 2);
+                        sp[0] = is[v];
+                        if constexpr (!Q6) sp[1] = (int)im[v];
+                    }
+                }
+            }
         }
-        const uint2 bsv = ld8(ab + 260 + 8 * i);  // bsum16 of 16-groups 4i .. 4i+3
-        const int bs0 = (int)(int16_t)(bsv.x & 0xffff) + (int)(int16_t)(bsv.x >> 16);
-        const int bs1 = (int)(int16_t)(bsv.y & 0xffff) + (int)(int16_t)(bsv.y >> 16);
-        const int ia = __mul24(sc0, dl) + __mul24(sc1, dh);
-        const int im = __mul24(m0, bs0) + __mul24(m1, bs1);
-        *sub_ia = ia;
-        *sub_im = im;
-        *dwo = dw;
-        *dmo = dmin;
+    };
+    if (w < nb) {
+        Ops cur, nxt;
+        load(w, cur);
+        for (int b = w; b < nb; b += KW) {
+            load(b + KW < nb ? b + KW : b, nxt);  // (the last again, unused)
+            block(b, cur);
+            cur = nxt;
+        }
+    }
+#pragma unroll
+    for (int v = 0; v < 16; v++) red[w][v][lane] = part[v];
+    __syncthreads();
+    if (row >= rows) return;
+#pragma unroll
+    for (int u = 0; u < 16 / KW; u++) {
+        const int v = 16 / KW * w + u, pi = crowm(v, lane);
+        float y = (red[0][v][lane] + red[1][v][lane]) + (red[2][v][lane] + red[3][v][lane]);
+        if constexpr (KW == 8) y += (red[4][v][lane] + red[5][v][lane]) + (red[6][v][lane] + red[7][v][lane]);
+        if (pi < count) *out(pi) = y;
     }
 }
 
-// grid: (tiles, ceil(rows / 16)); route as written by ghip_moe_route
-template <int TYPE, bool SUBSUMS>
+template <int TYPE, int KW, bool SUBSUMS>
 __device__ __forceinline__ void mmid_kq_impl(const uint8_t *__restrict__ as, int64_t as_nb1, int64_t as_nb2,
                                              const uint8_t *__restrict__ act, int64_t act_rb, int ne11,
                                              const int32_t *__restrict__ route, int n_pairs, int n_ids,
@@ -959,70 +1042,42 @@ __device__ __forceinline__ void mmid_kq_impl(const uint8_t *__restrict__ as, int
     if (tile >= route[0]) return;
     const int32_t *tl = route + 2 + n_pairs + 3 * tile;
     const int e = tl[0], first = tl[1], count = tl[2];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int r0 = (int)blockIdx.y * 16 + wave * MMID_RB;
-    const int i = lane & 3;
-    const uint8_t *ebase = as + (int64_t)e * as_nb2;
-    for (int pi = 0; pi < count; pi++) {
-        const int p = route[2 + first + pi];
-        const int t = p / n_ids, s = p - t * n_ids;
-        const uint8_t *arow = act + ((int64_t)t * ne11 + s % ne11) * act_rb;
-        float part[MMID_RB];
-#pragma unroll
-        for (int rr = 0; rr < MMID_RB; rr++) part[rr] = 0.0f;
-        for (int c = 0; c < nb; c += 16) {
-            const int b = c + (lane >> 2);
-            const bool valid = b < nb;
-#pragma unroll
-            for (int rr = 0; rr < MMID_RB; rr++) {
-                const int r = min(r0 + rr, rows - 1);
-                int32_t ia = 0, im = 0;
-                float d8 = 0.0f, dw = 0.0f, dm = 0.0f;
-                kq_lane_dot<TYPE>(ebase + (int64_t)r * as_nb1, arow, b, i, valid, &ia, &im, &d8, &dw, &dm);
-                // whole super-block sums (exact), then the block scale
-                // d = d8 * dw applied once per super-block (vec_dot.rs:881-909,
-                // vec_dot.rs:998-1028)
-                const int iab = quad_sum_dpp(ia), imb = TYPE == 14 ? 0 : quad_sum_dpp(im);
-                if (i == 0)
-                    part[rr] += TYPE == 14 ? (d8 * dw) * (float)iab
-                                           : fmaf(d8 * dw, (float)iab, (-d8 * dm) * (float)imb);
-                if (SUBSUMS) {
-                    if (i == 0 && valid && r0 + rr < rows) {
-                        int32_t *sp = sub + ((int64_t)p * rows + r0 + rr) * nb * (TYPE == 14 ? 1 : 2);
-                        if (TYPE == 14) sp[b] = iab;
-                        else {
-                            sp[2 * b] = iab;
-                            sp[2 * b + 1] = imb;
-                        }
-                    }
-                }
-            }
-        }
-        float *o = dst + (int64_t)t * dst_nb2 + (int64_t)s * dst_nb1;
-#pragma unroll
-        for (int rr = 0; rr < MMID_RB; rr++) {
-            const float tot = wave_sum_dpp(part[rr]);
-            if (lane == 0 && r0 + rr < rows) o[r0 + rr] = tot;
-        }
-    }
+    const int li = threadIdx.x & 31, row = (int)blockIdx.y * MMID_BR + li;
+    auto pair = [&](int i, int &t, int &s) {
+        const int p = route[2 + first + i];
+        t = p / n_ids;
+        s = p - t * n_ids;
+        return p;
+    };
+    int t, s;
+    pair(min(li, count - 1), t, s);  // past the tile: its last
+    kq32_tile<TYPE, KW, SUBSUMS>(
+        as + (int64_t)e * as_nb2 + (int64_t)min(row, rows - 1) * as_nb1, row, rows,
+        act + ((int64_t)t * ne11 + s % ne11) * act_rb, count, nb,
+        [&](int i) {
+            int ti, si;
+            pair(i, ti, si);
+            return dst + (int64_t)ti * dst_nb2 + (int64_t)si * dst_nb1 + row;
+        },
+        [&](int i) {
+            int ti, si;
+            return sub + ((int64_t)pair(i, ti, si) * rows + row) * nb * (TYPE == 14 ? 1 : 2);
+        });
 }
-#define MMID_KQ(TN, TYPE)                                                                                           \
-    extern "C" __global__ void __launch_bounds__(256)                                                               \
-        ghip_mmid_##TN(const uint8_t *__restrict__ as, int64_t as_nb1, int64_t as_nb2,                             \
-                       const uint8_t *__restrict__ act, int64_t act_rb, int ne11, const int32_t *__restrict__ route, \
-                       int n_pairs, int n_ids, float *__restrict__ dst, int64_t dst_nb1, int64_t dst_nb2, int rows,  \
-                       int nb, int32_t *__restrict__ sub) {                                                          \
-        mmid_kq_impl<TYPE, false>(as, as_nb1, as_nb2, act, act_rb, ne11, route, n_pairs, n_ids, dst, dst_nb1,      \
-                                  dst_nb2, rows, nb, sub);                                                          \
-    }                                                                                                               \
-    extern "C" __global__ void __launch_bounds__(256)                                                               \
-        ghip_mmid_##TN##_sub(const uint8_t *__restrict__ as, int64_t as_nb1, int64_t as_nb2,                        \
-                             const uint8_t *__restrict__ act, int64_t act_rb, int ne11,                             \
-                             const int32_t *__restrict__ route, int n_pairs, int n_ids, float *__restrict__ dst,    \
-                             int64_t dst_nb1, int64_t dst_nb2, int rows, int nb, int32_t *__restrict__ sub) {       \
-        mmid_kq_impl<TYPE, true>(as, as_nb1, as_nb2, act, act_rb, ne11, route, n_pairs, n_ids, dst, dst_nb1,       \
-                                 dst_nb2, rows, nb, sub);                                                           \
+
+#define MMID_KQ_ONE(NAME, TYPE, KW, SUB, WAVES)                                                                     \
+    extern "C" __global__ void __launch_bounds__(64 * KW, WAVES)                                                    \
+        NAME(const uint8_t *__restrict__ as, int64_t as_nb1, int64_t as_nb2, const uint8_t *__restrict__ act,        \
+             int64_t act_rb, int ne11, const int32_t *__restrict__ route, int n_pairs, int n_ids,                   \
+             float *__restrict__ dst, int64_t dst_nb1, int64_t dst_nb2, int rows, int nb,                           \
+             int32_t *__restrict__ sub) {                                                                           \
+        mmid_kq_impl<TYPE, KW, SUB>(as, as_nb1, as_nb2, act, act_rb, ne11, route, n_pairs, n_ids, dst, dst_nb1,     \
+                                    dst_nb2, rows, nb, sub);                                                        \
     }
+#define MMID_KQ(TN, TYPE)                                                                                           \
+    MMID_KQ_ONE(ghip_mmid_##TN##_k4, TYPE, 4, false, 2)                                                             \
+    MMID_KQ_ONE(ghip_mmid_##TN##_k8, TYPE, 8, false, 2)                                                             \
+    MMID_KQ_ONE(ghip_mmid_##TN##_sub, TYPE, 4, true, 1)
 MMID_KQ(q4_K, 12)
 MMID_KQ(q5_K, 13)
 MMID_KQ(q6_K, 14)

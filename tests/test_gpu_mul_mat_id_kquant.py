@@ -148,3 +148,14 @@ def test_invalid_id_gives_nan(be):
     got = be.mul_mat_id(torch.from_numpy(w).cuda(), n, torch.from_numpy(y).cuda(), torch.from_numpy(ids).cuda(),
                         ty=O.Q4_K).cpu().numpy()
     assert np.isnan(got[1]).all() and np.isfinite(got[0]).all() and np.isfinite(got[2]).all()
+
+
+@pytest.mark.parametrize("tid,n,rows,n_as,n_tokens,n_ids", [
+    (O.Q4_K, 256, 33, 2, 40, 2),    # 40 pairs an expert: two tiles; one row past a 32-row block
+    (O.Q5_K, 1024, 64, 1, 33, 1),   # one pair in the second tile; one super-block per wavefront
+    (O.Q6_K, 1280, 31, 3, 50, 2),   # a wavefront with two super-blocks; rows short of a block
+    (O.Q4_K, 1536, 100, 5, 1, 3),   # one token
+])
+def test_expert_tiles(be, tid, n, rows, n_as, n_tokens, n_ids):
+    """The 32-pair x 32-row tiles at their edges, sub-sums bit-exact."""
+    test_random_experts(be, tid, n, rows, n_as, n_tokens, 1, n_ids)
