@@ -1162,12 +1162,68 @@ ghip_status run_gemm(ghip_context *ctx, const MulMatPlan &p, const void *w, cons
                        (int)p.N, dst, (int64_t)ldd);
 }
 
-// wavefronts that share K in a 32 x 32 tile of the K-quant experts: 8 where the
-// tiles are few (1536 x 2048 Q4_K, 8 pairs: less to wait for per tile)
+// Q4_K / Q5_K / Q6_K with a short batch: the 32 x 32 tiles of ghip_moe.hip
+// (ghip_gemm_kq32_*) on Q8_K rows.  Measured against what served the rows
+// before, us, 4096 -> 14336 / 4096 -> 4096 / 14336 -> 4096:
+//  * Q5_K (to 15 rows the 8-column decode kernels, then the prefill GEMM): 9 rows
+//    21 / 13 / 27 against 48 / 25 / 84, 37 rows 37 / 16 / 32 against 39 / 25 / 44;
+//  * Q6_K (8-column decode kernels to 63 rows; a registered weight's records
+//    serve it better from 17 rows, see mul_mat_plane): 24 rows 28 / 18 / 42
+//    against 83 / 42 / 88;
+//  * Q4_K at 9-15 rows where the LDS image of the matrix-core decode kernel does
+//    not fit: - / - / 23 against 74-123 (with it, 17-20 / 13-15 / - against
+//    21 / 14 / -, and siblings in one launch 2 % slower: it stays);
+//  * Q4_K at 16-64 rows, against the prefill GEMM, 24 rows 21 / 14 / 26 and 22 / 17 /
+//    24, 37 rows 31 / 14 / 28 and 23 / 17 / 25: one token tile or few weight rows
+//    (n: of the launch, all grouped matrices), short K.
+bool use_kq32(const MulMatPlan &p, int64_t n = 0) {
+    if (!n) n = p.N;
+    if (p.M < 9 || p.M > 64 || p.kq_ns) return false;
+    if (p.wtype == GHIP_TYPE_Q6_K) return p.M < 64;
+    if (p.wtype == GHIP_TYPE_Q5_K) return true;
+    if (p.wtype != GHIP_TYPE_Q4_K) return false;
+    return p.M < 16 ? !use_skinny(p) : p.nb <= 32 && (p.M <= 32 || n <= 8192);
+}
+// wavefronts that share K in a 32 x 32 tile: 8 where the tiles are few (4096 ->
+// 4096, 24 rows, Q5_K, 128 tiles: 16.1 us with 4, 14.4 with 8; 4096 -> 14336, 448
+// tiles: 22.6 and 25.6)
 int kq32_waves(int64_t tiles, int64_t nb) { return tiles <= 256 && nb >= 8 ? 8 : 4; }
+// Host mirror of Kq32Multi in ghip_moe.hip (kernel argument by value).
+struct Kq32Multi {
+    const uint8_t *W[4];
+    float *dst[4];
+    int64_t ldd[4];
+    int rows[4];
+    int blk0[5];
+};
+// the first n members' W, dst, ldd and rows are set
+ghip_status launch_kq32(ghip_context *ctx, const MulMatPlan &p, Kq32Multi &g, int n, const uint8_t *act, int64_t act_rb,
+                        int32_t *sub, hipStream_t s) {
+    int64_t blk = 0;
+    for (int i = 0; i < 5; i++) {
+        if (i < 4 && i >= n) {
+            g.W[i] = g.W[0];
+            g.dst[i] = g.dst[0];
+            g.ldd[i] = g.ldd[0];
+            g.rows[i] = g.rows[0];
+        }
+        g.blk0[i] = (int)blk;
+        if (i < n) {
+            blk += (g.rows[i] + 31) / 32;
+            ctx->expect(g.dst[i], win2d(p.M, g.ldd[i], g.rows[i]), "dst");
+        }
+    }
+    if (sub) ctx->expect(sub, sub_bytes(p, p.M), "sub-sums");
+    const char *tn = p.wtype == GHIP_TYPE_Q4_K ? "q4_K" : p.wtype == GHIP_TYPE_Q5_K ? "q5_K" : "q6_K";
+    const int64_t tiles = blk * ((p.M + 31) / 32);
+    const int kw = sub ? 4 : kq32_waves(tiles, p.nb);
+    return ctx->launch(std::string("ghip_gemm_kq32_") + tn + (sub ? "_sub" : kw == 8 ? "_k8" : "_k4"),
+                       dim3((unsigned)tiles), dim3(64 * kw), 0, s, g, (int64_t)p.w_row_bytes, (int)p.nb, act, act_rb,
+                       (int)p.M, sub);
+}
 
 bool use_gemm(const MulMatPlan &p) {
-    if (p.M > INT32_MAX) return false;
+    if (p.M > INT32_MAX || use_kq32(p)) return false;
     if (p.wtype == GHIP_TYPE_Q4_K) return p.M >= env_int("GHIP_GEMM_MIN_ROWS", 16);
     // Q5_K: the wide Q4_K tiles with a fifth-bit plane, from 16 rows
     if (p.wtype == GHIP_TYPE_Q5_K) return p.M >= env_int("GHIP_GEMM_Q5K_MIN_ROWS", 16);
@@ -1268,12 +1324,12 @@ ghip_status mul_mat_plane(ghip_context *ctx, const ghip_tensor *a, const ghip_te
     ctx->allow(sub, sub_bytes(p, p.M), "sub-sums");
     ctx->allow(act_out, (size_t)(p.M * p.act_row_bytes), "activation output");
     if (kq_type(p.wtype) && !act_out) {
-        // a kept copy of the records also pays at fewer rows (Q6_K keeps one
-        // rule: registered and not give the same bits).  Where the workspace
+        // a kept copy of the records also pays at fewer rows (Q6_K 37 x 14336 ->
+        // 4096: 28 us against 44 on the 32 x 32 tiles).  Where the workspace
         // cannot hold the layout (a caller's or a fixed one, or growth under
         // capture), first without the K split, else the decode kernels.
         p.kq_reg = kq_registered(ctx, p, a->data) != nullptr;
-        if (!p.kq_ns && p.kq_reg && p.wtype != GHIP_TYPE_Q6_K && p.M >= 9 && p.M <= INT32_MAX)
+        if (!p.kq_ns && p.kq_reg && p.M >= (p.wtype == GHIP_TYPE_Q6_K ? 17 : 9) && p.M <= INT32_MAX)
             p.kq_ns = kq_nsplit(p.M, p.N, p.nb);
         auto fits = [&] { return ctx->workspace_fits(mul_mat_ws_bytes(p, d != nullptr, false, nullptr, nullptr), s); };
         if (!kq_required(p)) {
@@ -1303,6 +1359,20 @@ ghip_status mul_mat_plane(ghip_context *ctx, const ghip_tensor *a, const ghip_te
     // (GHIP_DEBUG_LDD_SKEW=k, dry-run contexts only: a deliberately wrong
     // leading dimension, the kind of host bug the store check exists for)
     const int64_t ldd = (d ? (int64_t)d->nb[1] / 4 : p.N) + (ctx->dry_run ? env_int("GHIP_DEBUG_LDD_SKEW", 0) : 0);
+    if (use_kq32(p)) {
+        const uint8_t *a8 = (const uint8_t *)b->data;
+        if (!p.act_pre) {
+            st = quantize_act(ctx, p, b, act, s);
+            if (st != GHIP_STATUS_SUCCESS) return st;
+            a8 = (const uint8_t *)act;
+        }
+        Kq32Multi g{};
+        g.W[0] = (const uint8_t *)a->data;
+        g.dst[0] = dst;
+        g.ldd[0] = ldd;
+        g.rows[0] = (int)p.N;
+        return launch_kq32(ctx, p, g, 1, a8, p.act_row_bytes, sub, s);
+    }
     if (gemm_route(p, sub != nullptr))
         return run_gemm(ctx, p, a->data, (const uint8_t *)b->data, p.act_pre ? nullptr : b, dst, ldd, sub, lay, s);
     if (use_sq(p)) {
@@ -1868,7 +1938,7 @@ ghip_status mul_mat_multi_gemm(ghip_context *ctx, const ghip_node *nodes, int n,
     ghip_status st;
     for (int i = 0; i < n; i++) {
         if (!plan_mul_mat(ctx, nodes[i].src[0], nodes[i].src[1], nodes[i].dst, p[i], st)) return st;
-        if (p[i].M != p[0].M || p[i].wtype != GHIP_TYPE_Q4_K || !use_gemm(p[i]) || p[i].act_pre)
+        if (p[i].M != p[0].M || p[i].wtype != GHIP_TYPE_Q4_K || !(use_gemm(p[i]) || use_kq32(p[i])) || p[i].act_pre)
             return ctx->fail(GHIP_STATUS_BACKEND_ERROR, "graph_compute: internal: node not groupable");
     }
     if (!ctx->set_device()) return ctx->fail(GHIP_STATUS_BACKEND_ERROR, "hipSetDevice failed");
@@ -1879,6 +1949,29 @@ ghip_status mul_mat_multi_gemm(ghip_context *ctx, const ghip_node *nodes, int n,
     const MulMatPlan &p0 = p[0];
     const int64_t Mpad = (p0.M + 127) / 128 * 128, K = p0.K, nbk = p0.K / 256;
     const size_t lay_bytes = (size_t)Mpad * K + (size_t)nbk * Mpad * 32 + (size_t)nbk * Mpad * 4;
+    int64_t n_all = 0;
+    bool alone = true;
+    for (int i = 0; i < n; i++) {
+        n_all += p[i].N;
+        alone = alone && use_kq32(p[i]);
+    }
+    // (members that each take these tiles alone, together too wide for them, do
+    // so where a workspace sized for them alone does not hold the GEMM's layout)
+    if (use_kq32(p0, n_all) || (alone && !ctx->workspace_fits(lay_bytes, s))) {
+        void *act = nullptr;
+        st = ctx->workspace(((size_t)(p0.M * p0.act_row_bytes) + 255) & ~(size_t)255, s, &act);
+        if (st != GHIP_STATUS_SUCCESS) return st;
+        st = quantize_act(ctx, p0, nodes[0].src[1], act, s);
+        if (st != GHIP_STATUS_SUCCESS) return st;
+        Kq32Multi g{};
+        for (int i = 0; i < n; i++) {
+            g.W[i] = (const uint8_t *)nodes[i].src[0]->data;
+            g.dst[i] = (float *)nodes[i].dst->data;
+            g.ldd[i] = (int64_t)nodes[i].dst->nb[1] / 4;
+            g.rows[i] = (int)p[i].N;
+        }
+        return launch_kq32(ctx, p0, g, n, (const uint8_t *)act, p0.act_row_bytes, nullptr, s);
+    }
     void *ws = nullptr;
     st = ctx->workspace(lay_bytes, s, &ws);
     if (st != GHIP_STATUS_SUCCESS) return st;

@@ -1065,6 +1065,54 @@ __device__ __forceinline__ void mmid_kq_impl(const uint8_t *__restrict__ as, int
         });
 }
 
+// The same tiles for MUL_MAT with a short batch (9-64 activation rows, already
+// Q8_K): up to four sibling matrices of one K and one input in a launch.  The
+// prefill GEMM's 64 x 128 tiles leave most CUs one workgroup or none there;
+// these are 32 x 32 with K shared by four wavefronts, and need no layout pass
+// or K split over workgroups.  (24 rows, 4096 -> 14336:
+// Q6_K 83 -> 28 us against the decode kernels; the other types and the line to
+// the GEMM beside use_kq32, the host mirror, in ghip.cpp.)
+struct Kq32Multi {
+    const uint8_t *W[4];
+    float *dst[4];
+    int64_t ldd[4];
+    int rows[4];
+    int blk0[5];  // first 32-row block of each matrix
+};
+template <int TYPE, int KW, bool SUBSUMS>
+__device__ __forceinline__ void gemm_kq32_impl(const Kq32Multi &g, int64_t w_row_bytes, int nb,
+                                               const uint8_t *__restrict__ act, int64_t act_rb, int M,
+                                               int32_t *__restrict__ sub) {
+    // the token tiles of one row block next to each other on one XCD (workgroup
+    // b runs on XCD b % 8)
+    const int total = (int)gridDim.x, b = (int)blockIdx.x, xcd = b % 8;
+    const int id = xcd * (total / 8) + min(xcd, total % 8) + b / 8;
+    const int tm = (M + 31) / 32, m0 = id % tm * 32, blk = id / tm;
+    int i = 0;
+    while (i < 3 && blk >= g.blk0[i + 1]) i++;
+    const int li = threadIdx.x & 31, row = (blk - g.blk0[i]) * 32 + li, rows = g.rows[i];
+    float *dst = g.dst[i];
+    const int64_t ldd = g.ldd[i];
+    const int count = min(32, M - m0);
+    kq32_tile<TYPE, KW, SUBSUMS>(
+        g.W[i] + (int64_t)min(row, rows - 1) * w_row_bytes, row, rows, act + (int64_t)(m0 + min(li, count - 1)) * act_rb,
+        count, nb, [&](int t) { return dst + (int64_t)(m0 + t) * ldd + row; },
+        [&](int t) { return sub + ((int64_t)(m0 + t) * rows + row) * nb * (TYPE == 14 ? 1 : 2); });
+}
+#define KQ32_ONE(NAME, TYPE, KW, SUB, WAVES)                                                                        \
+    extern "C" __global__ void __launch_bounds__(64 * KW, WAVES)                                                    \
+        NAME(Kq32Multi g, int64_t w_row_bytes, int nb, const uint8_t *__restrict__ act, int64_t act_rb, int M,       \
+             int32_t *__restrict__ sub) {                                                                           \
+        gemm_kq32_impl<TYPE, KW, SUB>(g, w_row_bytes, nb, act, act_rb, M, sub);                                     \
+    }
+#define KQ32(TN, TYPE)                                                                                              \
+    KQ32_ONE(ghip_gemm_kq32_##TN##_k4, TYPE, 4, false, 2)                                                           \
+    KQ32_ONE(ghip_gemm_kq32_##TN##_k8, TYPE, 8, false, 2)                                                           \
+    KQ32_ONE(ghip_gemm_kq32_##TN##_sub, TYPE, 4, true, 1)
+KQ32(q4_K, 12)
+KQ32(q5_K, 13)
+KQ32(q6_K, 14)
+
 #define MMID_KQ_ONE(NAME, TYPE, KW, SUB, WAVES)                                                                     \
     extern "C" __global__ void __launch_bounds__(64 * KW, WAVES)                                                    \
         NAME(const uint8_t *__restrict__ as, int64_t as_nb1, int64_t as_nb2, const uint8_t *__restrict__ act,        \

@@ -1,5 +1,6 @@
-"""The Q2_K / Q3_K / Q6_K prefill GEMM (ghip_kq.hip): integer super-block sums
-equal to the oracle's, f32 results against 64-bit sums of the same terms."""
+"""The Q2_K / Q3_K / Q6_K prefill GEMM (ghip_kq.hip) and the Q4_K / Q5_K / Q6_K
+short-batch tiles (ghip_moe.hip): integer super-block sums equal to the
+oracle's, f32 results against 64-bit sums of the same terms."""
 import numpy as np
 import pytest
 
@@ -9,7 +10,7 @@ torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
 
 # bytes of a block, offsets of d and dmin
-BLOCK = {O.Q2_K: (84, 80, 82), O.Q3_K: (110, 108, None), O.Q6_K: (210, 208, None), O.Q4_K: (144, 0, 2)}
+BLOCK = {O.Q2_K: (84, 80, 82), O.Q3_K: (110, 108, None), O.Q6_K: (210, 208, None), O.Q4_K: (144, 0, 2), O.Q5_K: (176, 0, 2)}
 
 
 @pytest.fixture(scope="module")
@@ -78,7 +79,50 @@ def test_gemm(be, ty, M, N, K):
     assert np.array_equal(again, got) and np.array_equal(pre, got)
 
 
-@pytest.mark.parametrize("ty,M", [(O.Q2_K, 20), (O.Q3_K, 20), (O.Q6_K, 70), (O.Q4_K, 150)])
+@pytest.mark.parametrize("ty", [O.Q4_K, O.Q5_K, O.Q6_K])
+@pytest.mark.parametrize("M,N,K", [
+    (9, 24, 256),     # fewer rows than a block, one super-block: three idle wavefronts
+    (32, 64, 1024),   # whole tiles, one super-block per wavefront
+    (33, 33, 1280),   # one token and one row past them
+    (63, 200, 768),
+])
+def test_short_batch(be, ty, M, N, K):
+    w = weights(ty, N, K, M * N)
+    x = np.random.default_rng(M).standard_normal((M, K + 4)).astype(np.float32)
+    wd, xd = torch.from_numpy(w).cuda(), torch.from_numpy(x).cuda()[:, :K]
+    print(f"kq32 type={ty} M={M} N={N} K={K}", flush=True)
+    act = be.mul_mat_act(wd, ty, K, xd).cpu().numpy()
+    want_sub = np.asarray(O.mul_mat(ty, w, K, N, np.ascontiguousarray(x[:, :K]), M, want_subsums=True)[2])
+    out = torch.full((M + 1, N + 4), 7.0, device="cuda")
+    got = be.mul_mat(wd, ty, K, xd, out=out[:M, :N]).cpu().numpy()
+    sub = be.mul_mat_subsums(wd, ty, K, xd).cpu().numpy()
+    assert np.array_equal(sub, want_sub.reshape(sub.shape))
+    want, mag = exact(ty, w, K, sub.astype(np.float64), act)
+    # three roundings a term, a wavefront's chain, two additions over the wavefronts
+    assert np.all(np.abs(got - want) <= (4 + K // 1024 + 3) * 2.0 ** -23 * mag)
+    assert bool((out[M] == 7.0).all()) and bool((out[:, N:] == 7.0).all())
+    pre = be.mul_mat(wd, ty, K, torch.from_numpy(act).cuda()).cpu().numpy()
+    assert np.array_equal(pre, got)
+
+
+def test_short_batch_group(be):
+    """Siblings too wide together for these tiles, in a workspace sized for each
+    alone: the bits of the single calls."""
+    import ghip
+    M, N, K = 40, 4096, 256
+    xd = torch.randn(M, K, device="cuda")
+    ws = [torch.from_numpy(weights(O.Q4_K, N, K, i)).cuda() for i in range(3)]
+    want = [be.mul_mat(w, O.Q4_K, K, xd) for w in ws]
+    outs = [torch.empty_like(o) for o in want]
+    nodes = [ghip.mul_mat_node(w, O.Q4_K, K, xd, o) for w, o in zip(ws, outs)]
+    be.set_workspace(torch.empty(max(be.workspace_size(nd) for nd in nodes), dtype=torch.uint8, device="cuda"))
+    be.graph_compute(nodes)
+    torch.cuda.synchronize()
+    be.set_workspace(None)
+    assert all(torch.equal(a, b) for a, b in zip(outs, want))
+
+
+@pytest.mark.parametrize("ty,M", [(O.Q2_K, 20), (O.Q3_K, 20), (O.Q6_K, 70), (O.Q4_K, 150), (O.Q4_K, 24), (O.Q5_K, 24), (O.Q6_K, 24)])
 def test_infinite_scale(be, ty, M):
     """A block scale of infinity gives infinities (NaN where its sum is 0 or two
     of them cancel), K split and not, and leaves the other rows alone."""
