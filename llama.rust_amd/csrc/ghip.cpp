@@ -317,6 +317,7 @@ struct MulMatPlan {
     bool act_pre;     // src1 already holds the vec_dot_type blocks
     int kq_ns = 0;        // K slices of the Q2_K / Q3_K / Q6_K prefill GEMM (ghip_kq.hip); 0: not on it
     bool kq_reg = false;  // ... over a registered weight's records
+    bool no_copy = false;  // Q4_0 / IQ4_XS: the weight is known not to be registered (see use_kq32)
 };
 
 // Q2_K / Q3_K / Q6_K prefill: the int8 GEMM of ghip_kq.hip
@@ -431,7 +432,8 @@ bool plan_mul_mat(ghip_context *ctx, const ghip_tensor *a, const ghip_tensor *b,
     return true;
 }
 
-ghip_status quantize_act(ghip_context *ctx, const MulMatPlan &p, const ghip_tensor *b, void *out, hipStream_t s) {
+ghip_status quantize_act(ghip_context *ctx, const MulMatPlan &p, const ghip_tensor *b, void *out, hipStream_t s,
+                         bool x8 = false) {
     const int64_t x_stride = (int64_t)b->nb[1] / 4;
     ctx->expect(out, (size_t)(p.M * p.act_row_bytes), "quantized activations");
     if (p.act_type == GHIP_TYPE_Q8_K) {
@@ -442,7 +444,7 @@ ghip_status quantize_act(ghip_context *ctx, const MulMatPlan &p, const ghip_tens
     }
     const int64_t blocks = p.M * (p.K / 32);
     const unsigned grid = (unsigned)((blocks * 8 + 255) / 256);
-    return ctx->launch(p.act_type == GHIP_TYPE_Q8_1 ? "ghip_quantize_q8_1" : "ghip_quantize_q8_0", dim3(grid),
+    return ctx->launch(p.act_type == GHIP_TYPE_Q8_1 ? "ghip_quantize_q8_1" : x8 ? "ghip_quantize_q8_0_x8" : "ghip_quantize_q8_0", dim3(grid),
                        dim3(256), 0, s, (const float *)b->data, x_stride, (int64_t)p.K, (int64_t)p.M, (uint8_t *)out,
                        (int64_t)p.act_row_bytes);
 }
@@ -1162,9 +1164,9 @@ ghip_status run_gemm(ghip_context *ctx, const MulMatPlan &p, const void *w, cons
                        (int)p.N, dst, (int64_t)ldd);
 }
 
-// Q4_K / Q5_K / Q6_K with a short batch: the 32 x 32 tiles of ghip_moe.hip
-// (ghip_gemm_kq32_*) on Q8_K rows.  Measured against what served the rows
-// before, us, 4096 -> 14336 / 4096 -> 4096 / 14336 -> 4096:
+// A short batch: the 32 x 32 tiles of ghip_moe.hip (ghip_gemm_kq32_*) on Q8_K or
+// Q8_0 rows.  Measured against what served the rows before, us, 4096 -> 14336 /
+// 4096 -> 4096 / 14336 -> 4096:
 //  * Q5_K (to 15 rows the 8-column decode kernels, then the prefill GEMM): 9 rows
 //    21 / 13 / 27 against 48 / 25 / 84, 37 rows 37 / 16 / 32 against 39 / 25 / 44;
 //  * Q6_K (8-column decode kernels to 63 rows; a registered weight's records
@@ -1175,10 +1177,24 @@ ghip_status run_gemm(ghip_context *ctx, const MulMatPlan &p, const void *w, cons
 //    21 / 14 / -, and siblings in one launch 2 % slower: it stays);
 //  * Q4_K at 16-64 rows, against the prefill GEMM, 24 rows 21 / 14 / 26 and 22 / 17 /
 //    24, 37 rows 31 / 14 / 28 and 23 / 17 / 25: one token tile or few weight rows
-//    (n: of the launch, all grouped matrices), short K.
+//    (n: of the launch, all grouped matrices), short K;
+//  * Q4_0 / Q8_0 / IQ4_XS to 31 rows, against the 8-column decode kernels, at 16
+//    26 / 23 / 37, 48 / 27 / 69, 25 / 17 / 33 and 54 / 52 / 93, 80 / 98 / 179, 57 / 28 / 58;
+//  * the same against the prefill GEMM, which repacks a weight that is not
+//    registered and goes through K in one chain, 64 rows 50 / 21 / 48, 91 / 34 / 76,
+//    43 / 17 / 35 and 82 / 60 / 180, 84 / 58 / 181, 90 / 60 / 190 (registered 38 /
+//    37 / 112, 38 / 37 / 111, 40 / 37 / 122), 128 rows 84 / 31 / 79, 155 / 51 / 139, 68 /
+//    26 / 62 and 86 / 60 / 180, 85 / 60 / 182, 91 / 61 / 190: few weight rows, and
+//    wide matrices of the 4-bit types without a kept copy.
 bool use_kq32(const MulMatPlan &p, int64_t n = 0) {
     if (!n) n = p.N;
-    if (p.M < 9 || p.M > 64 || p.kq_ns) return false;
+    if (p.M < 9 || p.M > 128) return false;
+    if (p.wtype == GHIP_TYPE_Q4_0 || p.wtype == GHIP_TYPE_Q8_0 || p.wtype == GHIP_TYPE_IQ4_XS) {
+        if (p.K % 256 || (p.act_pre && p.wtype != GHIP_TYPE_IQ4_XS)) return false;
+        if (p.M < 32) return true;
+        return p.N <= 8192 ? p.M <= (p.wtype == GHIP_TYPE_Q8_0 ? 64 : 128) : p.M <= 96 && p.no_copy;
+    }
+    if (p.M > 64 || p.kq_ns) return false;
     if (p.wtype == GHIP_TYPE_Q6_K) return p.M < 64;
     if (p.wtype == GHIP_TYPE_Q5_K) return true;
     if (p.wtype != GHIP_TYPE_Q4_K) return false;
@@ -1214,11 +1230,13 @@ ghip_status launch_kq32(ghip_context *ctx, const MulMatPlan &p, Kq32Multi &g, in
         }
     }
     if (sub) ctx->expect(sub, sub_bytes(p, p.M), "sub-sums");
-    const char *tn = p.wtype == GHIP_TYPE_Q4_K ? "q4_K" : p.wtype == GHIP_TYPE_Q5_K ? "q5_K" : "q6_K";
-    const int64_t tiles = blk * ((p.M + 31) / 32);
-    const int kw = sub ? 4 : kq32_waves(tiles, p.nb);
+    const char *tn = p.wtype == GHIP_TYPE_Q4_K ? "q4_K" : p.wtype == GHIP_TYPE_Q5_K ? "q5_K"
+                   : p.wtype == GHIP_TYPE_Q6_K ? "q6_K" : p.wtype == GHIP_TYPE_IQ4_XS ? "iq4_xs"
+                   : p.wtype == GHIP_TYPE_Q4_0 ? "q4_0" : "q8_0";
+    const int64_t tiles = blk * ((p.M + 31) / 32), nb = p.K / 256;
+    const int kw = sub ? 4 : kq32_waves(tiles, nb);
     return ctx->launch(std::string("ghip_gemm_kq32_") + tn + (sub ? "_sub" : kw == 8 ? "_k8" : "_k4"),
-                       dim3((unsigned)tiles), dim3(64 * kw), 0, s, g, (int64_t)p.w_row_bytes, (int)p.nb, act, act_rb,
+                       dim3((unsigned)tiles), dim3(64 * kw), 0, s, g, (int64_t)p.w_row_bytes, (int)nb, act, act_rb,
                        (int)p.M, sub);
 }
 
@@ -1337,6 +1355,7 @@ ghip_status mul_mat_plane(ghip_context *ctx, const ghip_tensor *a, const ghip_te
             if (p.kq_ns == 1 && !fits()) p.kq_ns = 0;
         }
     }
+    if (p.wtype == GHIP_TYPE_Q4_0 || p.wtype == GHIP_TYPE_IQ4_XS) p.no_copy = !kq_registered(ctx, p, a->data);
     size_t act_bytes, lay_bytes;
     const size_t need = mul_mat_ws_bytes(p, d != nullptr, act_out != nullptr, &act_bytes, &lay_bytes, sub != nullptr);
     void *ws = nullptr;
@@ -1362,7 +1381,7 @@ ghip_status mul_mat_plane(ghip_context *ctx, const ghip_tensor *a, const ghip_te
     if (use_kq32(p)) {
         const uint8_t *a8 = (const uint8_t *)b->data;
         if (!p.act_pre) {
-            st = quantize_act(ctx, p, b, act, s);
+            st = quantize_act(ctx, p, b, act, s, p.act_type == GHIP_TYPE_Q8_0);
             if (st != GHIP_STATUS_SUCCESS) return st;
             a8 = (const uint8_t *)act;
         }

@@ -33,26 +33,8 @@ namespace {
 constexpr int RB = 8;  // weight rows per decode workgroup
 constexpr int WT_IQ4_NL = 20, WT_IQ4_XS = 23, WT_NVFP4 = 40, WT_Q1_0 = 41, WT_Q2_0 = 42;
 
-// 16-entry int8 tables as four little-endian dwords (entries 4i .. 4i+3 in T[i])
-struct Lut {
-    uint32_t t0, t1, t2, t3;
-};
-// KVALUES_IQ4NL: -127 -104 -83 -65 | -49 -35 -22 -10 | 1 13 25 38 | 53 69 89 113
-constexpr Lut kIq4nl = {0xBFAD9881u, 0xF6EADDCFu, 0x26190D01u, 0x71594535u};
 // KVALUES_MXFP4: 0 1 2 3 | 4 6 8 12 | 0 -1 -2 -3 | -4 -6 -8 -12
 constexpr Lut kMxfp4 = {0x03020100u, 0x0C080604u, 0xFDFEFF00u, 0xF4F8FAFCu};
-
-// Table values of four nibbles, one in bits 0-3 of each byte of x (higher bits
-// of a byte are ignored): v_perm_b32 picks from entries 0-7 and 8-15 by the
-// low three bits, and a third v_perm_b32 picks, per byte, the half that bit 3
-// names.
-DEV uint32_t lut4(const Lut &L, uint32_t x) {
-    const uint32_t idx = x & 0x07070707u;
-    const uint32_t lo = __builtin_amdgcn_perm(L.t1, L.t0, idx);
-    const uint32_t hi = __builtin_amdgcn_perm(L.t3, L.t2, idx);
-    const uint32_t sel = 0x03020100u | ((x >> 1) & 0x04040404u);  // byte i: i, or 4 + i where bit 3 is set
-    return __builtin_amdgcn_perm(hi, lo, sel);
-}
 
 // ue4m3_to_fp32 (quants.rs:699-712): exp 0 -> man * 2^-10, 0x7F -> 0, else
 // (8 + man) * 2^(exp - 11) (the halving included); built from bits, exact

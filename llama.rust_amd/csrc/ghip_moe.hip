@@ -878,22 +878,55 @@ constexpr int MMID_BR = 32;  // rows per workgroup
 // activation row arow: token li's) and the 32 rows from row - li on (a lane's
 // own row, its weights wrow).  out(i, row) is token i's output for that row,
 // part_of(i) the sub-sums of (token i, row), nb super-blocks.
-template <int TYPE, int KW, bool SUBSUMS, class Out, class Sub>  // 12 Q4_K, 13 Q5_K, 14 Q6_K; KW wavefronts
+// TYPE: 12 Q4_K, 13 Q5_K, 14 Q6_K and 23 IQ4_XS on Q8_K rows; 2 Q4_0 and 8 Q8_0 on
+// Q8_0 rows, eight blocks in the place of a super-block.  KW wavefronts.
+constexpr int kq32_subs(int type) { return type < 12 ? 8 : type < 14 ? 2 : 1; }  // sub-sums per super-block
+template <int TYPE, int KW, bool SUBSUMS, class Out, class Sub>
 __device__ __forceinline__ void kq32_tile(const uint8_t *__restrict__ wrow, int row, int rows,
                                           const uint8_t *__restrict__ arow, int count, int nb, Out out, Sub part_of) {
-    constexpr bool Q5 = TYPE == 13, Q6 = TYPE == 14;
-    constexpr int NW = Q6 ? 6 : Q5 ? 5 : 4;  // 16-byte pieces of codes per lane and super-block
-    __shared__ __attribute__((aligned(16))) float d8s[KW][32];
+    constexpr bool Q5 = TYPE == 13, Q6 = TYPE == 14, XS = TYPE == 23, B32 = TYPE < 12;
+    // 16-byte pieces of codes per lane and super-block (Q4_0: all 144 bytes)
+    constexpr int NW = TYPE == 2 ? 9 : XS || B32 ? 8 : Q6 ? 6 : Q5 ? 5 : 4;
+    __shared__ __attribute__((aligned(16))) float d8s[KW][B32 ? 8 : 1][32];
     __shared__ float red[KW][16][64];
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int li = lane & 31, h = lane >> 5;
     struct Ops {  // one super-block
         uint4 a[8], bs, hd, w[NW];
         float d8, dw;
+        uint4 d8b;        // the blocks' own scales, activations
+        uint32_t dwb[8];  // and weights (Q4_0: among w)
+    };
+    constexpr int AB = B32 ? 8 * 34 : Q8K_BYTES;
+    constexpr int WB = TYPE == 8 ? 8 * 34 : XS ? 136 : Q6 ? Q6K_BYTES : Q5 ? 176 : Q4K_BYTES;
+    // Q4_0, Q8_0, IQ4_XS: the loads in parts, each part's next reloaded where it
+    // was used (two copies of all do not fit the registers)
+    auto load_head = [&](int b, Ops &o) {
+        if constexpr (XS) {
+            const uint2 t = ld8(wrow + (int64_t)b * WB);
+            o.hd.x = t.x;
+            o.hd.y = t.y;
+            o.d8 = __uint_as_float(ld4(arow + (int64_t)b * AB));
+        } else {
+            o.d8b = ld16(arow + (int64_t)b * AB);
+        }
+    };
+    auto load_part = [&](int b, int c, Ops &o) {  // block c's activations, and the weights it is the last to use
+        const uint8_t *blk = wrow + (int64_t)b * WB;
+        o.a[c] = ld16(arow + (int64_t)b * AB + (XS ? 4 : 16) + 32 * c + 16 * h);
+        if constexpr (TYPE == 2) {
+            o.w[c] = ld16(blk + 16 * c);
+            if (c == 7) o.w[8] = ld16(blk + 128);
+        } else if constexpr (TYPE == 8) {
+            o.w[c] = ld16(blk + 34 * c + 2 + 16 * h);
+            o.dwb[c] = ld2(blk + 34 * c);
+        } else {  // (both halves of the wavefront read a block's 16 bytes: its nibbles)
+            o.w[c] = ld16(blk + 8 + 16 * c);
+        }
     };
     auto load = [&](int b, Ops &o) {
-        const uint8_t *ab = arow + (int64_t)b * Q8K_BYTES;
-        const uint8_t *blk = wrow + (int64_t)b * (Q6 ? Q6K_BYTES : Q5 ? 176 : Q4K_BYTES);
+        const uint8_t *ab = arow + (int64_t)b * AB;
+        const uint8_t *blk = wrow + (int64_t)b * WB;
         if constexpr (Q6) {
 #pragma unroll
             for (int k = 0; k < 4; k++) o.w[k] = ld16(blk + 32 * k + 16 * h);
@@ -913,17 +946,97 @@ __device__ __forceinline__ void kq32_tile(const uint8_t *__restrict__ wrow, int 
         for (int c = 0; c < 8; c++) o.a[c] = ld16(ab + 4 + 32 * c + 16 * h);
     };
     auto dwords = [](uint4 v, uint32_t (&x)[4]) { x[0] = v.x; x[1] = v.y; x[2] = v.z; x[3] = v.w; };
-    // Q4_K / Q5_K: the sum's and the min product's roundings are carried along
+    // All but Q6_K: the sum's and the min product's roundings are carried along
     // (without, 1.03e-7 from the 64-bit value at K = 14336 where the prefill
     // GEMM's chain is 0.85e-7)
     float part[16], lost[16];
 #pragma unroll
     for (int v = 0; v < 16; v++) part[v] = lost[v] = 0.0f;
-    auto block = [&](int b, const Ops &o) {
+    auto block = [&](int b, Ops &o, int bn) {  // bn: the next
         v16i is;
         v16f im = {};
         float dw, dm = 0.0f;
-        if constexpr (Q6) {
+        if constexpr (B32) {
+            // a block's dot is exact, so is the product of two f16 scales: one
+            // rounding a block, eight blocks apart from the carried sum
+            uint32_t ad[4];
+            dwords(o.d8b, ad);
+            load_head(bn, o);
+#pragma unroll
+            for (int c = 0; c < 8; c++) d8s[w][c][li] = h2f(ad[c >> 1] >> (16 * (c & 1)));  // (this wavefront's own: no barrier)
+            float unit[16];
+#pragma unroll
+            for (int c = 0; c < 8; c++) {
+                v4i q;
+                float dwc;
+                if constexpr (TYPE == 8) {
+                    q = __builtin_bit_cast(v4i, o.w[c]);
+                    dwc = h2f(o.dwb[c]);
+                } else {  // block c starts at dword 9c / 2, odd ones at its upper half
+                    uint32_t x[36];
+#pragma unroll
+                    for (int k = 0; k < 9; k++) {
+                        x[4 * k] = o.w[k].x; x[4 * k + 1] = o.w[k].y; x[4 * k + 2] = o.w[k].z; x[4 * k + 3] = o.w[k].w;
+                    }
+                    dwc = h2f(x[9 * c / 2] >> (c & 1 ? 16 : 0));
+#pragma unroll
+                    for (int k = 0; k < 4; k++) {
+                        const uint32_t t = c & 1 ? x[9 * c / 2 + 1 + k]
+                                                 : __builtin_amdgcn_alignbyte(x[9 * c / 2 + 1 + k], x[9 * c / 2 + k], 2);
+                        // nibble - 8 in every byte
+                        q[k] = (int)(((((t >> (4 * h)) & 0x0f0f0f0fu) | 0x80808080u) - 0x08080808u) ^ 0x80808080u);
+                    }
+                }
+                const v16i d = __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(v4i, o.a[c]), q, v16i{}, 0, 0, 0);
+                load_part(bn, c, o);
+#pragma unroll
+                for (int g = 0; g < 4; g++) {
+                    const float4 d4 = *reinterpret_cast<const float4 *>(&d8s[w][c][8 * g + 4 * h]);
+                    const float dd[4] = {d4.x, d4.y, d4.z, d4.w};
+#pragma unroll
+                    for (int k = 0; k < 4; k++) {
+                        const int v = 4 * g + k;
+                        unit[v] = c == 0 ? dwc * dd[k] * (float)d[v] : fmaf(dwc * dd[k], (float)d[v], unit[v]);
+                        if constexpr (SUBSUMS) {
+                            const int pi = crowm(v, lane);
+                            if (pi < count && row < rows) part_of(pi)[8 * b + c] = d[v];
+                        }
+                    }
+                }
+                // the sums here and not at the end of the eight blocks (whose dots and
+                // scales together do not fit the registers)
+                if (c & 1) {
+#pragma unroll
+                    for (int v = 0; v < 16; v++) asm volatile("" : "+v"(unit[v]));
+                }
+            }
+#pragma unroll
+            for (int v = 0; v < 16; v++) {
+                const float y = unit[v] + lost[v], z = part[v] + y;
+                lost[v] = sum_lost(y - (z - part[v]));
+                part[v] = z;
+            }
+            return;
+        } else if constexpr (XS) {
+            dw = h2f(o.hd.x);
+            const uint32_t sh = o.hd.x >> 16, sl = o.hd.y;
+            d8s[w][0][li] = o.d8;
+            load_head(bn, o);
+            is = v16i{};
+#pragma unroll
+            for (int c = 0; c < 8; c++) {
+                uint32_t x[4];
+                dwords(o.w[c], x);
+                v4i q;
+#pragma unroll
+                for (int k = 0; k < 4; k++) q[k] = (int)lut4(kIq4nl, x[k] >> (4 * h));
+                const v16i d = __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(v4i, o.a[c]), q, v16i{}, 0, 0, 0);
+                load_part(bn, c, o);
+                const int ls = (int)(((sl >> (4 * c)) & 15u) | (((sh >> (2 * c)) & 3u) << 4)) - 32;
+#pragma unroll
+                for (int v = 0; v < 16; v++) is[v] += __mul24(ls, d[v]);
+            }
+        } else if constexpr (Q6) {
             dw = o.dw;
             uint32_t sc[4];
             dwords(o.hd, sc);
@@ -983,16 +1096,20 @@ __device__ __forceinline__ void kq32_tile(const uint8_t *__restrict__ wrow, int 
                 for (int v = 0; v < 16; v++) is[v] += __mul24(sc, d[v]);
             }
         }
-        d8s[w][li] = o.d8;  // (this wavefront's own row: no barrier)
+        if constexpr (!XS) d8s[w][0][li] = o.d8;  // (this wavefront's own row: no barrier)
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-            const float4 d4 = *reinterpret_cast<const float4 *>(&d8s[w][8 * q + 4 * h]);
+            const float4 d4 = *reinterpret_cast<const float4 *>(&d8s[w][0][8 * q + 4 * h]);
             const float dd[4] = {d4.x, d4.y, d4.z, d4.w};
 #pragma unroll
             for (int k = 0; k < 4; k++) {
                 const int v = 4 * q + k;
                 if constexpr (Q6) {
                     part[v] = fmaf(dw * (float)is[v], dd[k], part[v]);
+                } else if constexpr (XS) {
+                    const float y = fmaf(dw * (float)is[v], dd[k], lost[v]), z = part[v] + y;
+                    lost[v] = sum_lost(y - (z - part[v]));
+                    part[v] = z;
                 } else {
                     const float t = dm * im[v], e = sum_lost(fmaf(dm, im[v], -t));
                     const float y = fmaf(fmaf(dw, (float)is[v], -t) - e, dd[k], lost[v]), z = part[v] + y;
@@ -1002,9 +1119,9 @@ __device__ __forceinline__ void kq32_tile(const uint8_t *__restrict__ wrow, int 
                 if constexpr (SUBSUMS) {
                     const int pi = crowm(v, lane);
                     if (pi < count && row < rows) {
-                        int32_t *sp = part_of(pi) + b * (Q6 ? 1 : 2);
+                        int32_t *sp = part_of(pi) + b * kq32_subs(TYPE);
                         sp[0] = is[v];
-                        if constexpr (!Q6) sp[1] = (int)im[v];
+                        if constexpr (!Q6 && !XS) sp[1] = (int)im[v];
                     }
                 }
             }
@@ -1012,11 +1129,22 @@ __device__ __forceinline__ void kq32_tile(const uint8_t *__restrict__ wrow, int 
     };
     if (w < nb) {
         Ops cur, nxt;
-        load(w, cur);
+        if constexpr (B32 || XS) {
+            load_head(w, cur);
+#pragma unroll
+            for (int c = 0; c < 8; c++) load_part(w, c, cur);
+        } else {
+            load(w, cur);
+        }
         for (int b = w; b < nb; b += KW) {
-            load(b + KW < nb ? b + KW : b, nxt);  // (the last again, unused)
-            block(b, cur);
-            cur = nxt;
+            const int bn = b + KW < nb ? b + KW : b;  // (the last again, unused)
+            if constexpr (B32 || XS) {
+                block(b, cur, bn);
+            } else {
+                load(bn, nxt);
+                block(b, cur, bn);
+                cur = nxt;
+            }
         }
     }
 #pragma unroll
@@ -1026,8 +1154,13 @@ __device__ __forceinline__ void kq32_tile(const uint8_t *__restrict__ wrow, int 
 #pragma unroll
     for (int u = 0; u < 16 / KW; u++) {
         const int v = 16 / KW * w + u, pi = crowm(v, lane);
-        float y = (red[0][v][lane] + red[1][v][lane]) + (red[2][v][lane] + red[3][v][lane]);
-        if constexpr (KW == 8) y += (red[4][v][lane] + red[5][v][lane]) + (red[6][v][lane] + red[7][v][lane]);
+        float y = red[0][v][lane], l = 0.0f;
+#pragma unroll
+        for (int k = 1; k < KW; k++) {
+            const float t = red[k][v][lane] + l, z = y + t;
+            l = sum_lost(t - (z - y));
+            y = z;
+        }
         if (pi < count) *out(pi) = y;
     }
 }
@@ -1061,12 +1194,13 @@ __device__ __forceinline__ void mmid_kq_impl(const uint8_t *__restrict__ as, int
         },
         [&](int i) {
             int ti, si;
-            return sub + ((int64_t)pair(i, ti, si) * rows + row) * nb * (TYPE == 14 ? 1 : 2);
+            return sub + ((int64_t)pair(i, ti, si) * rows + row) * nb * kq32_subs(TYPE);
         });
 }
 
-// The same tiles for MUL_MAT with a short batch (9-64 activation rows, already
-// Q8_K): up to four sibling matrices of one K and one input in a launch.  The
+// The same tiles for MUL_MAT with a short batch (9-64 activation rows, to 128 for
+// Q4_0 and IQ4_XS, already quantized): up to four sibling matrices of one K and
+// one input in a launch.  The
 // prefill GEMM's 64 x 128 tiles leave most CUs one workgroup or none there;
 // these are 32 x 32 with K shared by four wavefronts, and need no layout pass
 // or K split over workgroups.  (24 rows, 4096 -> 14336:
@@ -1097,7 +1231,7 @@ __device__ __forceinline__ void gemm_kq32_impl(const Kq32Multi &g, int64_t w_row
     kq32_tile<TYPE, KW, SUBSUMS>(
         g.W[i] + (int64_t)min(row, rows - 1) * w_row_bytes, row, rows, act + (int64_t)(m0 + min(li, count - 1)) * act_rb,
         count, nb, [&](int t) { return dst + (int64_t)(m0 + t) * ldd + row; },
-        [&](int t) { return sub + ((int64_t)(m0 + t) * rows + row) * nb * (TYPE == 14 ? 1 : 2); });
+        [&](int t) { return sub + ((int64_t)(m0 + t) * rows + row) * nb * kq32_subs(TYPE); });
 }
 #define KQ32_ONE(NAME, TYPE, KW, SUB, WAVES)                                                                        \
     extern "C" __global__ void __launch_bounds__(64 * KW, WAVES)                                                    \
@@ -1112,6 +1246,9 @@ __device__ __forceinline__ void gemm_kq32_impl(const Kq32Multi &g, int64_t w_row
 KQ32(q4_K, 12)
 KQ32(q5_K, 13)
 KQ32(q6_K, 14)
+KQ32(iq4_xs, 23)
+KQ32(q4_0, 2)
+KQ32(q8_0, 8)
 
 #define MMID_KQ_ONE(NAME, TYPE, KW, SUB, WAVES)                                                                     \
     extern "C" __global__ void __launch_bounds__(64 * KW, WAVES)                                                    \

@@ -69,10 +69,11 @@ extern "C" __global__ void __launch_bounds__(256) ghip_quantize_q8_K_segs(Q8KSeg
 }
 
 // quantize_row_q8_0 (runtime AVX2 arithmetic, quants.rs:331-362): 8 lanes per
-// 32-element block, 8 blocks per wavefront.
-extern "C" __global__ void __launch_bounds__(256)
-ghip_quantize_q8_0(const float *__restrict__ x, int64_t x_stride, int64_t n, int64_t nrows,
-                   uint8_t *__restrict__ y, int64_t y_stride) {
+// 32-element block, 8 blocks per wavefront.  X8 (n % 256 == 0): eight blocks as
+// their eight scales and then their 256 codes, so that both are 16-byte aligned.
+template <bool X8>
+__device__ __forceinline__ void quantize_q8_0_impl(const float *__restrict__ x, int64_t x_stride, int64_t n,
+                                                   int64_t nrows, uint8_t *__restrict__ y, int64_t y_stride) {
     const int lane = threadIdx.x & 63;
     const int64_t nb = n / 32;
     const int64_t blk_id = ((int64_t)blockIdx.x * 256 + threadIdx.x) >> 3;
@@ -96,12 +97,22 @@ ghip_quantize_q8_0(const float *__restrict__ x, int64_t x_stride, int64_t n, int
         const int v = (r != r || fabsf(r) >= 2147483648.0f) ? -128 : (int)r;
         packed |= (uint32_t)(v & 0xff) << (8 * i);
     }
-    uint8_t *blk = y + row * y_stride + b * Q8_0_BYTES;
-    __builtin_memcpy(blk + 2 + sub * 4, &packed, 4);
+    uint8_t *blk = X8 ? y + row * y_stride + b / 8 * (8 * Q8_0_BYTES) + b % 8 * 2 : y + row * y_stride + b * Q8_0_BYTES;
+    __builtin_memcpy(blk + (X8 ? 16 + 30 * (b % 8) : 2) + sub * 4, &packed, 4);
     if (sub == 0) {
         const unsigned short dh = f2h_rn(d);
         __builtin_memcpy(blk, &dh, 2);
     }
+}
+extern "C" __global__ void __launch_bounds__(256)
+ghip_quantize_q8_0(const float *__restrict__ x, int64_t x_stride, int64_t n, int64_t nrows,
+                   uint8_t *__restrict__ y, int64_t y_stride) {
+    quantize_q8_0_impl<false>(x, x_stride, n, nrows, y, y_stride);
+}
+extern "C" __global__ void __launch_bounds__(256)
+ghip_quantize_q8_0_x8(const float *__restrict__ x, int64_t x_stride, int64_t n, int64_t nrows,
+                      uint8_t *__restrict__ y, int64_t y_stride) {
+    quantize_q8_0_impl<true>(x, x_stride, n, nrows, y, y_stride);
 }
 
 // f32 rows -> Q8_1 blocks (36 B: f16 d, f16 s, int8 qs[32]), quantize_row_q8_1

@@ -1,5 +1,5 @@
 """The Q2_K / Q3_K / Q6_K prefill GEMM (ghip_kq.hip) and the Q4_K / Q5_K / Q6_K
-short-batch tiles (ghip_moe.hip): integer super-block sums equal to the
+short-batch tiles (ghip_moe.hip; Q4_0, Q8_0 and IQ4_XS too): integer super-block sums equal to the
 oracle's, f32 results against 64-bit sums of the same terms."""
 import numpy as np
 import pytest
@@ -103,6 +103,51 @@ def test_short_batch(be, ty, M, N, K):
     assert bool((out[M] == 7.0).all()) and bool((out[:, N:] == 7.0).all())
     pre = be.mul_mat(wd, ty, K, torch.from_numpy(act).cuda()).cpu().numpy()
     assert np.array_equal(pre, got)
+
+
+@pytest.mark.parametrize("ty", [O.Q4_0, O.Q8_0, O.IQ4_XS])
+@pytest.mark.parametrize("M,N,K,skew", [
+    (9, 24, 256, 0),      # fewer rows than a block, one wavefront with work
+    (32, 64, 2048, 0),    # whole tiles, a super-block for each of eight wavefronts
+    (33, 33, 1280, 2),    # one token and one row past them; weights 2-byte aligned
+    (64, 200, 2304, 0),
+    (40, 8224, 256, 0),   # too wide for Q8_0, the 4-bit types unless registered
+])
+def test_short_batch_q8(be, ty, M, N, K, skew):
+    qk, size = O.BLOCK[ty]
+    rng = np.random.default_rng(M * N)
+    w = rng.integers(0, 256, (N, K // qk, size), dtype=np.uint8)
+    w[:, :, :2] = (rng.random((N, K // qk)) * 0.01).astype(np.float16).view(np.uint8).reshape(N, -1, 2)
+    w = w.reshape(N, -1)
+    x = rng.standard_normal((M, K + 4)).astype(np.float32)
+    x[:, 32:64] = 0.0  # a zero block
+    wd = torch.empty(w.size + 16, dtype=torch.uint8, device="cuda")[skew:skew + w.size].view(N, -1)
+    wd.copy_(torch.from_numpy(w))
+    xd = torch.from_numpy(x).cuda()[:, :K]
+    print(f"kq32 type={ty} M={M} N={N} K={K}", flush=True)
+    act = be.mul_mat_act(wd, ty, K, xd).cpu().numpy()
+    w8 = np.concatenate([w, np.zeros((-N % 8, w.shape[1]), np.uint8)])  # (the oracle's Q4_0 rows go by eight)
+    want_sub = np.asarray(O.mul_mat(ty, w8, K, len(w8), np.ascontiguousarray(x[:, :K]), M, want_subsums=True)[2])[:, :N]
+    out = torch.full((M + 1, N + 4), 7.0, device="cuda")
+    got = be.mul_mat(wd, ty, K, xd, out=out[:M, :N]).cpu().numpy()
+    sub = be.mul_mat_subsums(wd, ty, K, xd).cpu().numpy()
+    assert np.array_equal(sub, want_sub.reshape(sub.shape))
+    d = w.reshape(N, -1, size)[:, :, :2].copy().view(np.float16)[..., 0].astype(np.float64)
+    if ty == O.IQ4_XS:
+        d8 = act.reshape(M, -1, 292)[:, :, :4].copy().view(np.float32)[..., 0].astype(np.float64)
+    else:
+        d8 = act.reshape(M, -1, 34)[:, :, :2].copy().view(np.float16)[..., 0].astype(np.float64)
+    t = d * sub.reshape(M, N, -1) * d8[:, None, :]
+    # three roundings a term (Q4_0 / Q8_0: one, in sums of eight), a carried chain,
+    # carried additions over the wavefronts; the prefill GEMM: a chain over K / 32
+    n = 16 if N <= 8192 else 4 + K // 32
+    assert np.all(np.abs(got - t.sum(-1)) <= n * 2.0 ** -24 * np.abs(t).sum(-1))
+    assert bool((out[M] == 7.0).all()) and bool((out[:, N:] == 7.0).all())
+    if skew == 0:  # registered: this or the prefill GEMM
+        be.register_weight(wd, ty, K)
+        again = be.mul_mat(wd, ty, K, xd).cpu().numpy()
+        be.unregister_weight(wd, ty, K)
+        assert np.all(np.abs(again - t.sum(-1)) <= (4 + K // 32) * 2.0 ** -24 * np.abs(t).sum(-1))
 
 
 def test_short_batch_group(be):
