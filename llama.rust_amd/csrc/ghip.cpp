@@ -1170,7 +1170,7 @@ ghip_status run_gemm(ghip_context *ctx, const MulMatPlan &p, const void *w, cons
 //  * Q5_K (to 15 rows the 8-column decode kernels, then the prefill GEMM): 9 rows
 //    21 / 13 / 27 against 48 / 25 / 84, 37 rows 37 / 16 / 32 against 39 / 25 / 44;
 //  * Q6_K (8-column decode kernels to 63 rows; a registered weight's records
-//    serve it better from 17 rows, see mul_mat_plane): 24 rows 28 / 18 / 42
+//    serve it better from 17 rows, see mul_mat_plane): 24 rows 26 / 15 / 38
 //    against 83 / 42 / 88;
 //  * Q4_K at 9-15 rows where the LDS image of the matrix-core decode kernel does
 //    not fit: - / - / 23 against 74-123 (with it, 17-20 / 13-15 / - against

@@ -899,13 +899,20 @@ __device__ __forceinline__ void kq32_tile(const uint8_t *__restrict__ wrow, int 
     };
     constexpr int AB = B32 ? 8 * 34 : Q8K_BYTES;
     constexpr int WB = TYPE == 8 ? 8 * 34 : XS ? 136 : Q6 ? Q6K_BYTES : Q5 ? 176 : Q4K_BYTES;
-    // Q4_0, Q8_0, IQ4_XS: the loads in parts, each part's next reloaded where it
-    // was used (two copies of all do not fit the registers)
+    // Q6_K, Q4_0, Q8_0, IQ4_XS: the loads in parts, each part's next reloaded where it
+    // was used (two copies of all leave two wavefronts a SIMD or do not fit the
+    // registers; Q6_K experts, 64 tokens, top-8 of 64, 2048 -> 1536: 71 us so, 61 here;
+    // Q4_K / Q5_K are slower so, 24 x 4096 -> 14336 Q4_K 18.7 -> 22.9 us)
+    constexpr bool PARTS = Q6 || XS || B32;
     auto load_head = [&](int b, Ops &o) {
         if constexpr (XS) {
             const uint2 t = ld8(wrow + (int64_t)b * WB);
             o.hd.x = t.x;
             o.hd.y = t.y;
+            o.d8 = __uint_as_float(ld4(arow + (int64_t)b * AB));
+        } else if constexpr (Q6) {
+            o.hd = ld16(wrow + (int64_t)b * WB + 192);
+            o.dw = h2f(ld2(wrow + (int64_t)b * WB + 208));
             o.d8 = __uint_as_float(ld4(arow + (int64_t)b * AB));
         } else {
             o.d8b = ld16(arow + (int64_t)b * AB);
@@ -913,34 +920,29 @@ __device__ __forceinline__ void kq32_tile(const uint8_t *__restrict__ wrow, int 
     };
     auto load_part = [&](int b, int c, Ops &o) {  // block c's activations, and the weights it is the last to use
         const uint8_t *blk = wrow + (int64_t)b * WB;
-        o.a[c] = ld16(arow + (int64_t)b * AB + (XS ? 4 : 16) + 32 * c + 16 * h);
+        o.a[c] = ld16(arow + (int64_t)b * AB + (B32 ? 16 : 4) + 32 * c + 16 * h);
         if constexpr (TYPE == 2) {
             o.w[c] = ld16(blk + 16 * c);
             if (c == 7) o.w[8] = ld16(blk + 128);
         } else if constexpr (TYPE == 8) {
             o.w[c] = ld16(blk + 34 * c + 2 + 16 * h);
             o.dwb[c] = ld2(blk + 34 * c);
+        } else if constexpr (Q6) {
+            const int n = c >> 2, j = c & 3;
+            if (j >= 2) o.w[2 * n + j - 2] = ld16(blk + 64 * n + 32 * (j - 2) + 16 * h);
+            if (j == 3) o.w[4 + n] = ld16(blk + 128 + 32 * n + 16 * h);
         } else {  // (both halves of the wavefront read a block's 16 bytes: its nibbles)
             o.w[c] = ld16(blk + 8 + 16 * c);
         }
     };
-    auto load = [&](int b, Ops &o) {
+    auto load = [&](int b, Ops &o) {  // Q4_K, Q5_K
         const uint8_t *ab = arow + (int64_t)b * AB;
         const uint8_t *blk = wrow + (int64_t)b * WB;
-        if constexpr (Q6) {
+        o.hd = ld16(blk);
+        if constexpr (Q5) o.w[4] = ld16(blk + 16 + 16 * h);
 #pragma unroll
-            for (int k = 0; k < 4; k++) o.w[k] = ld16(blk + 32 * k + 16 * h);
-#pragma unroll
-            for (int n = 0; n < 2; n++) o.w[4 + n] = ld16(blk + 128 + 32 * n + 16 * h);
-            o.hd = ld16(blk + 192);
-            o.dw = h2f(ld2(blk + 208));
-        } else {
-            o.hd = ld16(blk);
-            if constexpr (Q5) o.w[4] = ld16(blk + 16 + 16 * h);
-#pragma unroll
-            for (int k = 0; k < 4; k++) o.w[k] = ld16(blk + (Q5 ? 48 : 16) + 32 * k + 16 * h);
-            o.bs = ld16(ab + 260 + 16 * h);
-        }
+        for (int k = 0; k < 4; k++) o.w[k] = ld16(blk + (Q5 ? 48 : 16) + 32 * k + 16 * h);
+        o.bs = ld16(ab + 260 + 16 * h);
         o.d8 = __uint_as_float(ld4(ab));
 #pragma unroll
         for (int c = 0; c < 8; c++) o.a[c] = ld16(ab + 4 + 32 * c + 16 * h);
@@ -1040,6 +1042,8 @@ __device__ __forceinline__ void kq32_tile(const uint8_t *__restrict__ wrow, int 
             dw = o.dw;
             uint32_t sc[4];
             dwords(o.hd, sc);
+            d8s[w][0][li] = o.d8;
+            load_head(bn, o);
             v16i lo, hi;
 #pragma unroll
             for (int c = 0; c < 8; c++) {
@@ -1056,6 +1060,7 @@ __device__ __forceinline__ void kq32_tile(const uint8_t *__restrict__ wrow, int 
                 const v4i a = __builtin_bit_cast(v4i, o.a[c]);
                 lo = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, pl, c == 0 ? v16i{} : lo, 0, 0, 0);
                 hi = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, ph, c == 0 ? v16i{} : hi, 0, 0, 0);
+                load_part(bn, c, o);
             }
             is = hi * 128 + lo;
         } else {
@@ -1096,7 +1101,7 @@ __device__ __forceinline__ void kq32_tile(const uint8_t *__restrict__ wrow, int 
                 for (int v = 0; v < 16; v++) is[v] += __mul24(sc, d[v]);
             }
         }
-        if constexpr (!XS) d8s[w][0][li] = o.d8;  // (this wavefront's own row: no barrier)
+        if constexpr (!PARTS) d8s[w][0][li] = o.d8;  // (this wavefront's own row: no barrier)
 #pragma unroll
         for (int q = 0; q < 4; q++) {
             const float4 d4 = *reinterpret_cast<const float4 *>(&d8s[w][0][8 * q + 4 * h]);
@@ -1129,7 +1134,7 @@ __device__ __forceinline__ void kq32_tile(const uint8_t *__restrict__ wrow, int 
     };
     if (w < nb) {
         Ops cur, nxt;
-        if constexpr (B32 || XS) {
+        if constexpr (PARTS) {
             load_head(w, cur);
 #pragma unroll
             for (int c = 0; c < 8; c++) load_part(w, c, cur);
@@ -1138,7 +1143,7 @@ __device__ __forceinline__ void kq32_tile(const uint8_t *__restrict__ wrow, int 
         }
         for (int b = w; b < nb; b += KW) {
             const int bn = b + KW < nb ? b + KW : b;  // (the last again, unused)
-            if constexpr (B32 || XS) {
+            if constexpr (PARTS) {
                 block(b, cur, bn);
             } else {
                 load(bn, nxt);
@@ -1204,7 +1209,7 @@ __device__ __forceinline__ void mmid_kq_impl(const uint8_t *__restrict__ as, int
 // prefill GEMM's 64 x 128 tiles leave most CUs one workgroup or none there;
 // these are 32 x 32 with K shared by four wavefronts, and need no layout pass
 // or K split over workgroups.  (24 rows, 4096 -> 14336:
-// Q6_K 83 -> 28 us against the decode kernels; the other types and the line to
+// Q6_K 83 -> 26 us against the decode kernels; the other types and the line to
 // the GEMM beside use_kq32, the host mirror, in ghip.cpp.)
 struct Kq32Multi {
     const uint8_t *W[4];
