@@ -2302,12 +2302,16 @@ static ghip_status fa_sequence(ghip_context *ctx, const ghip_tensor *q, const gh
     // both run on the MFMA kernel below.  Fewer rows take the one-chunk walk
     // with its f16 accumulator, reproduced by the row-sequential kernel.
     if (!(T == 1 && S >= 512) && T < 64 && !env_int("GHIP_FA_FORCE_MFMA", 0)) {
-        // 8 walked rows per workgroup where that still gives nearly two
-        // workgroups per CU (63 rows of 64 / 8 heads over 2111 keys: 91 us
-        // against 110 with 4), else 4 (37 rows over 1061 keys: 45 against 50)
-        const int rows = G * T, nc = (int64_t)H_kv * ((rows + 7) / 8) >= 448 ? 8 : 4;
+        // 8 walked rows per workgroup (K and V staged half as often) where the
+        // busiest of the 256 CUs then walks no more rows than with 4.  us with 4 / 8:
+        // 63 rows of 64 / 8 heads over 2111 keys 168 / 151, 37 of 32 / 8 (D = 128) over
+        // 1061 78 / 60; 37 of 64 / 8 over 1061 (12 and 16 rows) 60 / 82, 2 of 32 / 8
+        // over 4096 (4 and 8) 135 / 198
+        const int rows = G * T;
+        auto busiest = [&](int64_t n) { return n * ((H_kv * ((rows + n - 1) / n) + 255) / 256); };
+        const int nc = busiest(8) <= busiest(4) ? 8 : 4;
         const std::string rs = std::string("ghip_fa_rows") + (nc == 8 ? "8" : "4") + (D == 128 ? "_d128" : "_d64");
-        return ctx->launch(rs, dim3((unsigned)(H_kv * ((rows + nc - 1) / nc))), dim3(64 * (nc + 4)), 0, s, p);
+        return ctx->launch(rs, dim3((unsigned)(H_kv * ((rows + nc - 1) / nc))), dim3(64 * (nc + 5)), 0, s, p);
     }
     if (T == 1) {
         // single-query split-KV route: the bandwidth-bound vector kernel

@@ -27,7 +27,6 @@ typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef _Float16 v4h __attribute__((ext_vector_type(4)));
 typedef __fp16 v4fp16 __attribute__((__vector_size__(8)));  // the transposing LDS read's type
 typedef float v16f __attribute__((ext_vector_type(16)));
-typedef float v4f __attribute__((ext_vector_type(4)));
 
 constexpr int FA_BQ = 32;   // query positions per workgroup
 constexpr int FA_BK = 64;   // keys per tile
@@ -831,35 +830,34 @@ ghip_fa_merge(const float *__restrict__ part, const float *__restrict__ sinks, f
 // a few 1e-3 at S ~ 1000), so the accumulator takes the reference's steps in
 // the reference's order -- skip masked (-inf) keys, new max => rescale by
 // exp(Mold - M) and round, then acc = f16(fma(v, vs, acc)) -- while all that
-// does not depend on it is done for many keys at once.
+// does not depend on it is done for many keys at once.  The scores and the row
+// sum take the walk's steps too (one fma chain over the head's dims per score,
+// one over the keys per sum): a score or sum rounded otherwise turns some of the
+// accumulator's f16 roundings (outputs 1.7e-4 apart, matrix-core scores).
 //
 // A workgroup owns NC of the G * T rows that read one KV head: NC wavefronts
-// walk a row each, four more prepare their tiles of 64 keys, in three steps
-// that run side by side on three successive tiles (one barrier per tile):
-//  * scores of tile i + 2: preparing wavefront w multiplies keys 16w .. 16w+15
-//    with all the rows on v_mfma_f32_16x16x32_f16 (K fragments straight from
-//    memory, one tile ahead) and leaves scaled, masked scores in LDS (masked
-//    keys as FR_DEAD);
-//  * softmax of tile i + 1, a row at a time: lane j holds key j's score.
-//    Without a new max among them one exp per lane gives the keys' vs; with
-//    one, a prefix max over the lanes gives the running max before and after
-//    every key, and with it the key's vs and, where the max moves, its ms.
-//    V of the tile goes through registers into LDS;
+// walk a row each, four more prepare their tiles of 64 keys and one adds up the
+// rows' sums, in steps that run side by side on successive tiles (one barrier per tile):
+//  * K of tile i + 2 and V of tile i + 1 go through registers into LDS (K's
+//    16-byte pieces swizzled by the key, so that lanes read a key each);
+//  * scores and softmax of tile i + 1, a row at a time: lane j scores key j.
+//    Without a new max among the scores one exp per lane gives the keys' vs;
+//    with one, a prefix max over the lanes gives the running max before and
+//    after every key, and with it the key's vs and, where the max moves, its
+//    ms (masked keys: 0 and 1);
 //  * the walk over tile i: lane l owns dims PL*l .., per key one readlane and
-//    PL fused multiply-adds with f16 rounding (v_fma_mix).  Sixteen keys
+//    PL fused multiply-adds rounded to f16.  Sixteen keys
 //    with a new max among them rescale at every key (by 1 where the max
-//    stays); a tile with masked keys tests every key.
+//    stays); a tile with masked keys tests every key;
+//  * the row sums over tile i, a lane each.
 //
-// Bound by the walk, a serial chain of 4 + 8 PL clocks per key (v_fma_mix
-// issues in 8) on one wavefront per row, and by the preparation's share of the
-// same SIMDs.  Measured: 37 rows of 64 / 8 heads, D = 64, 1061 keys, sinks:
-// 188 us with one wavefront per row that scored a key per lane and took one
-// exp per key, 66 us with matrix-core scores and an exp per lane in the
-// walking wavefront itself, 59 us with wavefronts of their own for that,
-// 42 us with a tile's loads issued before its arithmetic, no branches for the
-// tiles whose max moves and the walk at a raised priority.
-constexpr uint32_t FR_DEAD = 0xFFFFFFFFu;  // no score has this NaN's payload
-
+// Bound by the walk, a serial chain of 4 + 12 PL clocks per key (v_fma_mix issues
+// in 8, the rounding in 4) on one wavefront per row, and by the scores' chain of 8 D
+// clocks per row and tile on the same SIMDs.  Measured: 37 rows of 64 / 8 heads,
+// D = 64, 1061 keys, sinks: 206 us with one wavefront per row that scored a key per
+// lane and took one exp per key, 60 us here with the same bits (45 us with
+// matrix-core scores, lane-wise row sums and f16 sums rounded once); the row
+// sums on a preparing wavefront: 74 us.
 // running max over the lanes up to and including each lane
 DEV float wave_cummax(float v) {
     const int ninf = __float_as_int(-__builtin_inff());
@@ -878,11 +876,12 @@ DEV float readlane_f(float v, int l) { return __int_as_float(__builtin_amdgcn_re
 
 template <int D, int NC>
 __device__ __forceinline__ void fa_rows_impl(const FaParams &p) {
-    constexpr int PL = D / 64, KS = D / 32, RP = NC / 4;  // rows per preparing wavefront
-    constexpr int VP = FA_BK * D * 2 / 16 / 256;           // 16-byte V pieces per preparing thread and tile
-    __shared__ __attribute__((aligned(16))) uint32_t sc[2][NC][FA_BK + 4];
+    constexpr int PL = D / 64, NP = D / 8, RP = NC / 4;  // 16-byte pieces of a head; rows per preparing wavefront
+    constexpr int VP = FA_BK * NP / 256;                 // K (and V) pieces per preparing thread and tile
+    __shared__ __attribute__((aligned(16))) uint4 kt[2][FA_BK][NP];
     __shared__ __attribute__((aligned(16))) uint16_t vt[2][FA_BK][D];
-    __shared__ float vsb[2][NC][FA_BK], msb[2][NC][FA_BK];
+    __shared__ __attribute__((aligned(16))) uint16_t qs[NC][D];
+    __shared__ __attribute__((aligned(16))) float vsb[2][NC][FA_BK + 4], msb[2][NC][FA_BK + 4];
     __shared__ uint64_t liveb[2][NC], evb[2][NC];
     __shared__ float Mb[NC], Sb[NC];
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -890,111 +889,129 @@ __device__ __forceinline__ void fa_rows_impl(const FaParams &p) {
     const int hk = (int)blockIdx.x % p.H_kv, r0 = (int)blockIdx.x / p.H_kv * NC;
     const int ntile = (p.S + FA_BK - 1) / FA_BK;
 
+    if (w == NC + 4) {  // the row sums: row r in lane r
+        const int r = min(lane, NC - 1);
+        float S = 0.0f;
+        for (int it = -2; it < ntile; it++) {
+            if (it >= 0) {
+                const int q = it & 1;
+                const bool ev = evb[q][r] != 0;
+                if (__ballot(ev) == 0) {
+#pragma unroll 8
+                    for (int j = 0; j < FA_BK; j += 4) {
+                        const float4 v = *reinterpret_cast<const float4 *>(&vsb[q][r][j]);
+                        S = (((S + v.x) + v.y) + v.z) + v.w;
+                    }
+                } else {
+#pragma unroll 4
+                    for (int j = 0; j < FA_BK; j += 4) {
+                        const float4 v = *reinterpret_cast<const float4 *>(&vsb[q][r][j]);
+                        float4 m = make_float4(1.0f, 1.0f, 1.0f, 1.0f);
+                        if (ev) m = *reinterpret_cast<const float4 *>(&msb[q][r][j]);
+                        S = fmaf(fmaf(fmaf(fmaf(S, m.x, v.x), m.y, v.y), m.z, v.z), m.w, v.w);
+                    }
+                }
+                if (lane < NC) Sb[lane] = S;
+            }
+            __syncthreads();
+        }
+        return;
+    }
     if (w >= NC) {  // prepare
         const int pw = w - NC, tid = threadIdx.x - 64 * NC;
-        const int c = lane & 15, g4 = lane >> 4;
-        // this lane's score column: row r0 + c (rows past the end repeat the last)
-        const int ci = min(r0 + c, nrow - 1), ct = ci / G, ch = hk * G + (ci - ct * G);
-        const float slope = head_slope(p, ch);
-        const uint16_t *mrow = p.mask ? p.mask + (int64_t)(ch % p.mask_ne2) * p.mask_nb2 + (int64_t)ct * p.mask_nb1 : nullptr;
-        const int mk = 16 * pw + 4 * g4;  // the lane's four keys of a tile
-        const uint8_t *kb = (const uint8_t *)(p.k + (int64_t)hk * p.k_nb2) + 16 * g4;
-        const uint8_t *vb = (const uint8_t *)(p.v + (int64_t)hk * p.v_nb2) + 16 * (tid % (D / 8));
-        const int vkey = tid / (D / 8), kkey = 16 * pw + c;
-        constexpr int VKS = 256 / (D / 8);  // keys between a thread's V pieces
-        v8h qf[KS];
-        {
-            const float *qr = p.q + (int64_t)ch * p.q_nb2 + (int64_t)ct * p.q_nb1 + 8 * g4;
-#pragma unroll
-            for (int ks = 0; ks < KS; ks++)
-#pragma unroll
-                for (int e = 0; e < 8; e++) qf[ks][e] = (_Float16)qr[32 * ks + e];
-        }
-        uint4 kr[KS], vr[VP];
-        uint32_t mr[2] = {0, 0};  // the four mask values, as loaded
-        const uint8_t *kp = kb + (int64_t)kkey * p.k_nb1 * 2, *vp = vb + (int64_t)vkey * p.v_nb1 * 2;
-        auto load_k = [&](int tile) {  // K and mask; keys past the end repeat the last
-            const int k0 = tile * FA_BK;
-            const bool full = k0 + FA_BK <= p.S;
-            const uint8_t *r = full ? kp + (int64_t)k0 * p.k_nb1 * 2 : kb + (int64_t)min(k0 + kkey, p.S - 1) * p.k_nb1 * 2;
-#pragma unroll
-            for (int ks = 0; ks < KS; ks++) kr[ks] = ld16(r + 64 * ks);
-            if (mrow && full) __builtin_memcpy(mr, mrow + k0 + mk, 8);
-            if (mrow && !full) {
-#pragma unroll
-                for (int i = 0; i < 2; i++)
-                    mr[i] = mrow[min(k0 + mk + 2 * i, p.S - 1)] | ((uint32_t)mrow[min(k0 + mk + 2 * i + 1, p.S - 1)] << 16);
-            }
-        };
-        auto load_v = [&](int tile) {
-            const int k0 = tile * FA_BK;
-            const uint8_t *r[VP];
-            if (k0 + FA_BK <= p.S) {
-#pragma unroll
-                for (int i = 0; i < VP; i++) r[i] = vp + (int64_t)(k0 + i * VKS) * p.v_nb1 * 2;
-            } else {
-#pragma unroll
-                for (int i = 0; i < VP; i++) r[i] = vb + (int64_t)min(k0 + vkey + i * VKS, p.S - 1) * p.v_nb1 * 2;
-            }
-#pragma unroll
-            for (int i = 0; i < VP; i++) vr[i] = ld16(r[i]);
-        };
-        float M[RP], S[RP];  // S: this lane's keys' share
+        // this wavefront's rows r0 + RP * pw .. (rows past the end repeat the last)
+        float slope[RP];
+        const uint16_t *mrow[RP];
 #pragma unroll
         for (int r = 0; r < RP; r++) {
-            M[r] = -__builtin_inff();
-            S[r] = 0.0f;
+            const int ri = min(r0 + pw * RP + r, nrow - 1), rt = ri / G, rh = hk * G + (ri - rt * G);
+            slope[r] = head_slope(p, rh);
+            mrow[r] = p.mask ? p.mask + (int64_t)(rh % p.mask_ne2) * p.mask_nb2 + (int64_t)rt * p.mask_nb1 : nullptr;
+            const float *qr = p.q + (int64_t)rh * p.q_nb2 + (int64_t)rt * p.q_nb1;
+            // (read by this wavefront alone)
+            for (int d = lane; d < D; d += 64) qs[pw * RP + r][d] = __builtin_bit_cast(uint16_t, (_Float16)qr[d]);
         }
+        const int pc = tid % NP, pkey = tid / NP;  // the thread's pieces: piece pc of keys pkey, pkey + KS, ..
+        constexpr int KS = 256 / NP;
+        const uint8_t *kb = (const uint8_t *)(p.k + (int64_t)hk * p.k_nb2) + 16 * pc;
+        const uint8_t *vb = (const uint8_t *)(p.v + (int64_t)hk * p.v_nb2) + 16 * pc;
+        uint4 kr[VP], vr[VP];
+        uint32_t mr[RP] = {};
+        auto load = [&](const uint8_t *base, int64_t nb1, int tile, uint4 (&x)[VP]) {  // keys past the end repeat the last
+            const int k0 = tile * FA_BK + pkey;
+            const uint8_t *r[VP];
+            if ((tile + 1) * FA_BK <= p.S) {
+#pragma unroll
+                for (int i = 0; i < VP; i++) r[i] = base + (int64_t)(k0 + i * KS) * nb1 * 2;
+            } else {
+#pragma unroll
+                for (int i = 0; i < VP; i++) r[i] = base + (int64_t)min(k0 + i * KS, p.S - 1) * nb1 * 2;
+            }
+#pragma unroll
+            for (int i = 0; i < VP; i++) x[i] = ld16(r[i]);
+        };
+        auto load_m = [&](int tile) {
+            if (p.mask) {
+#pragma unroll
+                for (int r = 0; r < RP; r++) mr[r] = mrow[r][min(tile * FA_BK + lane, p.S - 1)];
+            }
+        };
+        float M[RP];
+#pragma unroll
+        for (int r = 0; r < RP; r++) M[r] = -__builtin_inff();
         if (ntile > 0) {
-            load_k(0);
-            load_v(0);
+            load(kb, p.k_nb1, 0, kr);
+            load(vb, p.v_nb1, 0, vr);
+            load_m(0);
         }
         for (int it = -2; it < ntile; it++) {
             const int ta = it + 2, tb = it + 1;
+            const bool onb = tb >= 0 && tb < ntile;
             // what the last step loaded is used up and the next loads issued
             // before the rest, so that they have a whole step to arrive
-            v4f d = {0.0f, 0.0f, 0.0f, 0.0f};
-            const uint32_t mc[2] = {mr[0], mr[1]};
             if (ta < ntile) {
 #pragma unroll
-                for (int ks = 0; ks < KS; ks++)
-                    d = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, kr[ks]), qf[ks], d, 0, 0, 0);
+                for (int i = 0; i < VP; i++) kt[ta & 1][pkey + i * KS][pc ^ ((pkey + i * KS) & 7)] = kr[i];
             }
-            if (tb >= 0 && tb < ntile) {
+            if (onb) {
 #pragma unroll
                 for (int i = 0; i < VP; i++) reinterpret_cast<uint4 *>(&vt[tb & 1][0][0])[i * 256 + tid] = vr[i];
             }
-            if (ta + 1 < ntile) load_k(ta + 1);
-            if (tb >= 0 && tb + 1 < ntile) load_v(tb + 1);
-            if (ta < ntile) {
-                uint32_t sb[4];
-                d *= p.scale;
-                if (p.softcap != 0.0f) {
+            uint32_t mc[RP];
 #pragma unroll
-                    for (int i = 0; i < 4; i++) d[i] = p.softcap * tanhf(d[i]);
-                }
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const float mv = mrow ? slope * h2f(mc[i >> 1] >> (16 * (i & 1))) : 0.0f;
-                    const float s = d[i] + mv;
-                    const bool live = ta * FA_BK + mk + i < p.S && mv != -__builtin_inff();
-                    sb[i] = live ? __float_as_uint(s) : FR_DEAD;
-                }
-                if (c < NC) *reinterpret_cast<uint4 *>(&sc[ta & 1][c][mk]) = make_uint4(sb[0], sb[1], sb[2], sb[3]);
+            for (int r = 0; r < RP; r++) mc[r] = mr[r];
+            if (ta + 1 < ntile) load(kb, p.k_nb1, ta + 1, kr);
+            if (onb && tb + 1 < ntile) {
+                load(vb, p.v_nb1, tb + 1, vr);
+                load_m(tb + 1);
             }
-            if (tb >= 0 && tb < ntile) {
+            if (onb) {
                 const int q = tb & 1;
+                float dot[RP];
+#pragma unroll
+                for (int r = 0; r < RP; r++) dot[r] = 0.0f;
+#pragma unroll 4
+                for (int c = 0; c < NP; c++) {
+                    const v8h k8 = __builtin_bit_cast(v8h, kt[q][lane][c ^ (lane & 7)]);
+#pragma unroll
+                    for (int r = 0; r < RP; r++) {
+                        const v8h q8 = *reinterpret_cast<const v8h *>(&qs[pw * RP + r][8 * c]);
+#pragma unroll
+                        for (int e = 0; e < 8; e++) dot[r] = fmaf((float)k8[e], (float)q8[e], dot[r]);
+                    }
+                }
 #pragma unroll
                 for (int r = 0; r < RP; r++) {
                     const int row = pw * RP + r;
-                    const uint32_t b = sc[q][row][lane];
-                    const bool lv = b != FR_DEAD;
-                    const float s = lv ? __uint_as_float(b) : -__builtin_inff();
+                    float s = dot[r] * p.scale;
+                    if (p.softcap != 0.0f) s = p.softcap * tanhf(s);
+                    const float mv = p.mask ? slope[r] * h2f(mc[r]) : 0.0f;
+                    const bool lv = tb * FA_BK + lane < p.S && mv != -__builtin_inff();
+                    s = lv ? s + mv : -__builtin_inff();
                     uint64_t ev = 0;
-                    float vs, ms = 1.0f;
+                    float vs;
                     if (__ballot(s > M[r]) == 0) {
                         vs = expf(s - M[r]);
-                        S[r] += lv ? vs : 0.0f;
                     } else {
                         const float cum = wave_cummax(s);
                         const float run = fmaxf(M[r], cum);  // the max after key `lane`
@@ -1003,30 +1020,16 @@ __device__ __forceinline__ void fa_rows_impl(const FaParams &p) {
                         const bool up = lv && s > prev;
                         const float e = expf(up ? prev - s : s - prev);
                         vs = up ? 1.0f : e;
-                        ms = up ? e : 1.0f;
                         ev = __ballot(up);
-                        // S after the tile, scaled to its last max
-                        const float Mn = readlane_f(run, 63);
-                        const float wt = !lv ? 0.0f : run == Mn ? vs : vs * expf(run - Mn);
-                        S[r] = (M[r] == Mn ? S[r] : S[r] * expf(M[r] - Mn)) + wt;
-                        M[r] = Mn;
-                        msb[q][row][lane] = ms;
+                        M[r] = readlane_f(run, 63);
+                        msb[q][row][lane] = up ? e : 1.0f;
                     }
-                    vsb[q][row][lane] = vs;
+                    vsb[q][row][lane] = lv ? vs : 0.0f;
                     const uint64_t live = __ballot(lv);
                     if (lane == 0) {
                         liveb[q][row] = live;
                         evb[q][row] = ev;
-                    }
-                }
-            }
-            if (it == ntile - 1) {
-#pragma unroll
-                for (int r = 0; r < RP; r++) {
-                    const float st = wave_sum_dpp(S[r]);
-                    if (lane == 0) {
-                        Mb[pw * RP + r] = M[r];
-                        Sb[pw * RP + r] = st;
+                        Mb[row] = M[r];
                     }
                 }
             }
@@ -1040,13 +1043,14 @@ __device__ __forceinline__ void fa_rows_impl(const FaParams &p) {
     _Float16 acc[PL];
 #pragma unroll
     for (int i = 0; i < PL; i++) acc[i] = (_Float16)0.0f;
+    // (rounded to f32, then to f16, as the reference: v_fma_mixlo rounds once)
     auto add = [&](const _Float16 (&v)[PL], float vj) {
 #pragma unroll
-        for (int i = 0; i < PL; i++) acc[i] = (_Float16)fmaf((float)v[i], vj, (float)acc[i]);
+        for (int i = 0; i < PL; i++) acc[i] = (_Float16)opaque(fmaf((float)v[i], vj, (float)acc[i]));
     };
     auto rescale = [&](float mj) {
 #pragma unroll
-        for (int i = 0; i < PL; i++) acc[i] = (_Float16)((float)acc[i] * mj);
+        for (int i = 0; i < PL; i++) acc[i] = (_Float16)opaque((float)acc[i] * mj);
     };
     for (int it = -2; it < ntile; it++) {
         if (it >= 0) {
@@ -1235,9 +1239,9 @@ extern "C" __global__ void __launch_bounds__(512) ghip_fa_fwd_d128(FaParams p) {
 extern "C" __global__ void __launch_bounds__(512) ghip_fa_fwd_d64(FaParams p) { fa_fwd_impl<64, false>(p); }
 extern "C" __global__ void __launch_bounds__(512) ghip_fa_fwd_sc_d128(FaParams p) { fa_fwd_impl<128, true>(p); }
 extern "C" __global__ void __launch_bounds__(512) ghip_fa_fwd_sc_d64(FaParams p) { fa_fwd_impl<64, true>(p); }
-extern "C" __global__ void __launch_bounds__(512) ghip_fa_rows4_d128(FaParams p) { fa_rows_impl<128, 4>(p); }
-extern "C" __global__ void __launch_bounds__(768) ghip_fa_rows8_d128(FaParams p) { fa_rows_impl<128, 8>(p); }
-extern "C" __global__ void __launch_bounds__(512) ghip_fa_rows4_d64(FaParams p) { fa_rows_impl<64, 4>(p); }
-extern "C" __global__ void __launch_bounds__(768) ghip_fa_rows8_d64(FaParams p) { fa_rows_impl<64, 8>(p); }
+extern "C" __global__ void __launch_bounds__(576) ghip_fa_rows4_d128(FaParams p) { fa_rows_impl<128, 4>(p); }
+extern "C" __global__ void __launch_bounds__(832) ghip_fa_rows8_d128(FaParams p) { fa_rows_impl<128, 8>(p); }
+extern "C" __global__ void __launch_bounds__(576) ghip_fa_rows4_d64(FaParams p) { fa_rows_impl<64, 4>(p); }
+extern "C" __global__ void __launch_bounds__(832) ghip_fa_rows8_d64(FaParams p) { fa_rows_impl<64, 8>(p); }
 extern "C" __global__ void __launch_bounds__(256) ghip_fa_decode_d128(FaParams p) { fa_decode_impl<128>(p); }
 extern "C" __global__ void __launch_bounds__(256) ghip_fa_decode_d64(FaParams p) { fa_decode_impl<64>(p); }

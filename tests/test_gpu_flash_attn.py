@@ -313,3 +313,63 @@ def test_few_rows(be, H, Hkv, D, T, S, holes, sinks, softcap):
     got = be.flash_attn_ext(t(q), t(k).permute(1, 0, 2), t(v).permute(1, 0, 2), t(m), t(sk), 1.0 / np.sqrt(D), 0.0,
                             softcap).cpu().numpy()
     assert np.max(np.abs(got - want)) <= TOL
+
+
+def walk(q, k, v, m, sk, scale):
+    """The few-row route key by key in torch: f32 fma chains (taken in float64,
+    where a product of a half and a float is exact, and rounded), f16 accumulator."""
+    H, T, D = q.shape
+    S, G = k.shape[1], H // k.shape[0]
+    kr, vr = k.repeat_interleave(G, 0), v.repeat_interleave(G, 0)
+    q16, k64 = q.half().double(), kr.double()
+    dot = torch.zeros(H, T, S, device=q.device)
+    for d in range(D):
+        dot = (q16[:, :, d, None] * k64[:, None, :, d] + dot.double()).float()
+    s = dot * scale + m.float()
+    acc = torch.zeros(H, T, D, device=q.device, dtype=torch.float16)
+    M = torch.full((H, T), -np.inf, device=q.device)
+    tot = torch.zeros(H, T, device=q.device)
+    one = torch.ones_like(M)
+    for j in range(S):
+        sj, live = s[:, :, j], m[None, :, j].float() > -np.inf
+        up = sj > M
+        e = torch.exp(torch.where(up, M - sj, sj - M))
+        ms, vs = torch.where(up, e, one), torch.where(up, one, e)
+        a = torch.where(up[..., None], (acc.float() * ms[..., None]).half(), acc)
+        a = (vr[:, j].double()[:, None, :] * vs.double()[..., None] + a.double()).float().half()
+        acc = torch.where(live[..., None], a, acc)
+        tot = torch.where(live, (tot.double() * ms.double() + vs.double()).float(), tot)
+        M = torch.where(live & up, sj, M)
+    a, h = acc.float(), torch.arange(H, device=q.device)[:, None]
+    if sk is not None:
+        b = sk[:, None].expand(H, T)
+        up = b > M
+        e = torch.exp(torch.where(up, M - b, b - M))
+        a = torch.where(up[..., None], a * e[..., None], a)
+        tot = torch.where(up, tot * e + 1.0, tot + e)
+    return (a * (1.0 / tot)[..., None]).permute(1, 0, 2)
+
+
+@pytest.mark.parametrize("H,Hkv,D,T,S,holes,sinks", [
+    (8, 2, 64, 5, 300, False, True),
+    (8, 2, 128, 3, 257, True, False),
+    (64, 8, 64, 56, 200, False, False),   # 8 rows a workgroup
+    (64, 8, 128, 56, 130, True, True),
+])
+def test_few_rows_rounding(be, H, Hkv, D, T, S, holes, sinks):
+    """Every rounding of the walk, the scores', the row sum's and both of the
+    accumulator's (f32, then f16): the outputs have its bits.  (A tie that
+    float64 rounds twice moves an output one f16 step: 1 in 2^29 operations,
+    S D of them behind an output.)"""
+    g = torch.Generator(device="cuda").manual_seed(H + D + T + S)
+    q = torch.randn(H, T, D, generator=g, device="cuda")
+    k, v = (torch.randn(Hkv, S, D, generator=g, device="cuda").half() for _ in range(2))
+    m = torch.from_numpy(causal_mask(T, S)).cuda()
+    if holes:
+        m[:, :S - T][:, torch.rand(S - T, generator=g, device="cuda") < 0.3] = -np.inf
+    sk = torch.randn(H, generator=g, device="cuda") if sinks else None
+    scale = float(np.float32(1.0 / np.sqrt(D)))
+    print(f"fa walk H={H} Hkv={Hkv} D={D} T={T} S={S}", flush=True)
+    got = be.flash_attn_ext(q, k, v, m, sk, scale)
+    differ = float((got != walk(q, k, v, m, sk, scale)).float().mean())
+    assert differ <= 1e-3, differ
