@@ -1916,8 +1916,9 @@ bool multi_candidate(const ghip_node &n) {
 // node j joins the group nodes[i, j)
 bool joins_group(const ghip_node *nodes, int i, int j) {
     const ghip_node &c = nodes[j], &h = nodes[i];
+    // (the grouped kernels take one K and one weight row stride)
     if (!multi_candidate(c) || c.src[0]->type != h.src[0]->type || c.src[0]->ne[0] != h.src[0]->ne[0] ||
-        !same_view(c.src[1], h.src[1]))
+        c.src[0]->nb[1] != h.src[0]->nb[1] || !same_view(c.src[1], h.src[1]))
         return false;
     // Q4_K activations take the 4x8 values for the leading rows only when
     // N % 8 == 0 (compute.rs:5350-5398): one quantization per group

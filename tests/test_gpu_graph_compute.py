@@ -266,3 +266,19 @@ def test_prequantized_inputs_past_eight(be, monkeypatch):
         single = be.mul_mat(ws[i], ty, k, xs[i])
         torch.cuda.synchronize()
         assert torch.equal(got[i], single), i
+
+
+@pytest.mark.parametrize("ty,m", [(12, 2), (12, 6), (12, 24), (12, 100), (14, 1), (2, 2)])
+def test_siblings_with_other_row_strides(be, ty, m):
+    """A strided view of a weight beside a packed one, either first: the
+    outputs of the single calls."""
+    import ghip
+    k = 1024
+    wide = weights(be, ty, 512, 2 * k, 1)  # rows of 2 k: its left half is a view with the wide rows' stride
+    view, packed = wide[:, :wide.shape[1] // 2], weights(be, ty, 384, k, 2)
+    x = torch.randn((m, k), device="cuda", generator=torch.Generator(device="cuda").manual_seed(3))
+    for ws in ((view, packed), (packed, view)):
+        outs = [torch.full((m, w.shape[0]), float("nan"), device="cuda") for w in ws]
+        be.graph_compute([ghip.mul_mat_node(w, ty, k, x, o) for w, o in zip(ws, outs)])
+        for w, o in zip(ws, outs):
+            assert torch.equal(o, be.mul_mat(w.contiguous(), ty, k, x))

@@ -124,3 +124,46 @@ def test_mul_mat_id_stores_inside_dst():
                 assert st == 0, (ty, n_tokens, L.ghip_last_error(ctx).decode())
             finally:
                 L.ghip_free(ctx)
+
+
+def _grouped(ty, m, pad):
+    """Two sibling MUL_MATs, the first one's weight rows `pad` blocks further
+    apart: does a graph run them as one launch?  (A dry run under
+    GHIP_DEBUG_LDD_SKEW: the skew reaches single launches only.)"""
+    ghip, L = _lib()
+    ctx = C.c_void_p()
+    assert L.ghip_init_dry_run(C.byref(ctx)) == 0
+    try:
+        blck, bs = ghip.BLOCK[ty]
+        k, n = 1024, 512
+        ws = [_tensor(ghip, ty, [k, n, 1, 1], bs, blck, W_BASE + (i << 32)) for i in range(2)]
+        for d, rows in ((1, 1), (2, n), (3, n)):
+            ws[0].nb[d] += pad * bs * rows
+        x = _tensor(ghip, ghip.F32, [k, m, 1, 1], 4, 1, X_BASE)
+        ds = [_tensor(ghip, ghip.F32, [n, m, 1, 1], 4, 1, D_BASE + (i << 32)) for i in range(2)]
+        arr = (ghip.GNode * 2)()
+        for i in range(2):
+            arr[i].op = ghip.OP_MUL_MAT
+            arr[i].src[0], arr[i].src[1] = C.pointer(ws[i]), C.pointer(x)
+            arr[i].dst = C.pointer(ds[i])
+        st = L.ghip_graph_compute(ctx, arr, 2, None)
+        assert st == 0 or "store check" in L.ghip_last_error(ctx).decode()
+        return st == 0
+    finally:
+        L.ghip_free(ctx)
+
+
+def test_groups_share_the_weight_row_stride():
+    """A grouped launch has one row stride for its members: siblings that
+    differ in it (a padded or strided view beside a packed matrix) run alone."""
+    code = (
+        "import sys; sys.path.insert(0, %r); sys.path.insert(0, %r)\n"
+        "import test_store_check as T, ghip\n"
+        "for ty, m in [(ghip.Q4_K, 2), (ghip.Q4_K, 6), (ghip.Q4_K, 24), (ghip.Q4_K, 100), (ghip.Q5_K, 2), (ghip.Q4_0, 2),"
+        " (ghip.Q8_0, 4)]:\n"
+        "    assert T._grouped(ty, m, 0), (ty, m)\n"
+        "    assert not T._grouped(ty, m, 1), (ty, m)\n"
+    ) % (os.path.join(ROOT, "tests"), os.path.join(ROOT, "llama.rust_amd"))
+    env = dict(os.environ, GHIP_DEBUG_LDD_SKEW="1")
+    r = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout + r.stderr
