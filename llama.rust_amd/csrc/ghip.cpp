@@ -1276,18 +1276,51 @@ size_t mul_mat_ws_bytes(const MulMatPlan &p, bool has_dst, bool act_out, size_t 
     return (act_out ? 0 : act_bytes) + lay_bytes + (has_dst || act_out ? 0 : (size_t)(p.M * p.N * 4));
 }
 
-// Tile edge of the dense prefill GEMM (ghip_dense.hip): the largest whose grid
-// still fills the 256 CUs.  Measured, F16, us with 32 / 64 / 128: 64 x 4096 ->
-// 4096 (256 / 64 / 32 tiles) 19 / 25 / 53, 200 x 4096 -> 4096 (896 / 256 / 64)
+// Tile edge of the dense prefill GEMM (ghip_dense.hip): 128 from 384 tiles (1.5 a
+// CU), 64 from 192 (3/4 of the CUs), else 32.  Measured, F16, us with 32 / 64 /
+// 128: 64 x 4096 -> 4096 (256 / 64 / 32 tiles) 19 / 25 / 53, 200 x 4096 -> 4096 (896 / 256 / 64)
 // 49 / 30 / 60, 300 x 2048 -> 12000 (3750 / 940 / 282) 89 / 57 / 61, 512 x 1024 ->
 // 16384 (8192 / 2048 / 512) 106 / 64 / 39.
 int dense_gemm_tile(int64_t M, int64_t N) {
     auto tiles = [&](int64_t t) { return ((M + t - 1) / t) * ((N + t - 1) / t); };
     return tiles(128) >= 384 ? 128 : tiles(64) >= 192 ? 64 : 32;
 }
+// F16 / BF16 with few rows, where the decode kernel (8 rows a launch) is the faster
+// one: the GEMM takes K in one chain, 3.3 ns an element (BF16 6.1, for the
+// activations' rounding), however few the tiles.  vec: 16-byte aligned rows.
+bool dense_decode_pays(const MulMatPlan &p, bool vec) {
+    const bool bf = p.wtype == GHIP_TYPE_BF16;
+    const int64_t M = p.M, K = p.K, N = p.N;
+    if (K % 8) {
+        // The element-by-element GEMM against the decode kernel's element loads, both
+        // sides as measured (us of the GEMM and of 8 rows of decode; estimate / measured,
+        // F16: 24 x 4095 -> 64 100 / 100 and 12 / 12, 24 x 4095 -> 14336 187 / 190 and 45 / 45,
+        // 24 x 1001 -> 4096 31 / 28 and 11 / 10).  24 x 4095 -> 4096: 121 us and 51;
+        // 64 x 1001 -> 4096: 28 and 82.
+        const double k = (double)K, n = (double)N, t = (double)((M + 31) / 32 * ((N + 31) / 32));
+        const double rounds = t <= 256 ? 1 + std::min(t, 128.0) / 750 : 0.94 * std::ceil(t / 256);
+        const double groups = (double)(M / 8) + (M % 8 ? 0.3 + (double)(M % 8) / 11 : 0.0);
+        const double gemm = (3 + (bf ? 0.0262 : 0.0236) * k) * rounds;
+        const double group = (bf ? 9.5 + 0.00175 * k : 6.5 + 0.00135 * k) + 2e-7 * k * n + (bf ? 0.0023 : 0.0019) * std::max(0.0, n - 3000);
+        return groups * group < gemm;
+    }
+    if (!vec) return false;
+    // us, GEMM and decode.  F16: 9 x 14336 -> 512 50 and 30, -> 2048 51 and 49, 9 x 4096 -> 1024
+    // 17 and 15, 12 x 14336 -> 512 50 and 44; but 9 x 4096 -> 2048 17 and 21, 12 x 14336 ->
+    // 1024 50 and 58, 16 x 14336 -> 512 50 and 50.  BF16: 9 x 4096 -> 4096 29 and 25, 12 x 14336 ->
+    // 4096 92 and 78, 16 x 8192 -> 2048 54 and 53, 17 x 14336 -> 512 90 and 76; 24 x 14336
+    // -> 512 90 and 96, 9 x 4096 -> 14336 39 and 69.
+    if (!bf) {
+        if (M == 9) return K >= 4096 && N <= std::min<int64_t>(K / 4, 2048);
+        return M <= (K > 16384 ? 16 : 12) && K >= 8192 && N <= 512 && N * K <= 512 * 16384;
+    }
+    if (M <= 12) return K >= 2048 && N <= 4096;
+    if (M <= 16) return K >= 4096 && N <= std::min<int64_t>(K / 4, 4096);
+    return M <= 20 && K >= 8192 && N <= 512;
+}
 // F32 / F16 / BF16 weights (compute.rs:1680-1745): F16 / BF16 from 9 activation
-// rows on the matrix cores, the rest on the dense decode kernel over groups
-// of at most 8 rows
+// rows on the matrix cores where that pays, the rest on the dense decode kernel
+// over groups of at most 8 rows
 ghip_status run_dense(ghip_context *ctx, const MulMatPlan &p, const ghip_tensor *a, const ghip_tensor *b, float *dst,
                       int64_t ldd, hipStream_t s) {
     const char *tn = p.wtype == GHIP_TYPE_F32 ? "f32" : p.wtype == GHIP_TYPE_F16 ? "f16" : "bf16";
@@ -1295,7 +1328,7 @@ ghip_status run_dense(ghip_context *ctx, const MulMatPlan &p, const ghip_tensor 
     const int vec = p.K % 8 == 0 && (uintptr_t)a->data % 16 == 0 && p.w_row_bytes % 16 == 0 ? 1 : 0;
     const int64_t x_stride = (int64_t)b->nb[1] / 4;
     // (9 x 4096 -> 4096 F16: 18 us against 28 in two launches of the decode kernel)
-    if (p.wtype != GHIP_TYPE_F32 && p.M >= 9 && p.M <= INT32_MAX) {
+    if (p.wtype != GHIP_TYPE_F32 && p.M >= 9 && p.M <= INT32_MAX && !dense_decode_pays(p, vec)) {
         const bool odd = p.K % 8 != 0;  // rows that end inside a 16-byte piece
         const int64_t t = odd ? 32 : dense_gemm_tile(p.M, p.N), tiles = ((p.M + t - 1) / t) * ((p.N + t - 1) / t);
         if (tiles <= INT32_MAX) {

@@ -1,5 +1,6 @@
 // ghip_dense.hip -- MUL_MAT with F32, F16 and BF16 weights: the decode kernel
-// (up to 8 activation rows a launch) and, for F16 / BF16 from 9 rows, the
+// (up to 8 activation rows a launch) and, for F16 / BF16 from 9 rows (a few rows
+// of a long K aside: dense_decode_pays in ghip.cpp), the
 // prefill GEMM on the matrix cores.
 //
 // Reference (compute.rs:1680-1745; vec_dot.rs:1700-1727): F16 / BF16 weights

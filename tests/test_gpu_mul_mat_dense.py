@@ -121,3 +121,29 @@ def test_prefill_gemm(be, ty, M, N, K):
     err = (got.cpu().double() - want).abs()
     assert bool((err <= (64 + 8 + K // 512 + 1 + 3) * 2.0 ** -24 * mag).all()), float((err / mag.clamp_min(1e-30)).max())
     assert bool((out[M] == 7.0).all()) and bool((out[:, N:] == 7.0).all())
+
+
+@pytest.mark.parametrize("ty,M,N,K,decode", [
+    ("f16", 9, 512, 14336, True),
+    ("f16", 12, 64, 8192, True),
+    ("f16", 24, 1000, 4095, True),    # K not a multiple of 8
+    ("bf16", 16, 1024, 8192, True),
+    ("bf16", 10, 100, 2047, True),
+    ("f16", 16, 512, 14336, False),
+    ("bf16", 24, 512, 4096, False),
+    ("f16", 64, 512, 1001, False),
+])
+def test_few_rows_long_k(be, ty, M, N, K, decode):
+    """9 rows and more of a long K: the faster of the decode kernel (its bits:
+    those of its groups of 8 rows) and the GEMM, whose K is one chain."""
+    import ghip
+    td = torch.float16 if ty == "f16" else torch.bfloat16
+    g = torch.Generator().manual_seed(M + N + K)
+    w, x = (torch.randn((N, K), generator=g) * 0.02).to(td), torch.randn((M, K), generator=g)
+    t = ghip.F16 if ty == "f16" else ghip.BF16
+    got = be.mul_mat(w.cuda(), t, K, x.cuda())
+    first = be.mul_mat(w.cuda(), t, K, x[:8].cuda())
+    assert torch.equal(got[:8], first) == decode
+    xr, wr = x.to(td).double(), w.double()
+    err = (got.cpu().double() - xr @ wr.t()).abs()
+    assert bool((err <= (64 + 8 + K // 512 + 1 + 3) * 2.0 ** -24 * (xr.abs() @ wr.abs().t())).all())
