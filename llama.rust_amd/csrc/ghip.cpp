@@ -1170,7 +1170,7 @@ ghip_status run_gemm(ghip_context *ctx, const MulMatPlan &p, const void *w, cons
 //  * Q5_K (to 15 rows the 8-column decode kernels, then the prefill GEMM): 9 rows
 //    21 / 13 / 27 against 48 / 25 / 84, 37 rows 37 / 16 / 32 against 39 / 25 / 44;
 //  * Q6_K (8-column decode kernels to 63 rows; a registered weight's records
-//    serve it better from 17 rows, see mul_mat_plane): 24 rows 26 / 15 / 38
+//    serve it better from 17 rows, see mul_mat_plane): 24 rows 27 / 15 / 39
 //    against 83 / 42 / 88;
 //  * Q4_K at 9-15 rows where the LDS image of the matrix-core decode kernel does
 //    not fit: - / - / 23 against 74-123 (with it, 17-20 / 13-15 / - against
@@ -1376,7 +1376,7 @@ ghip_status mul_mat_plane(ghip_context *ctx, const ghip_tensor *a, const ghip_te
     ctx->allow(act_out, (size_t)(p.M * p.act_row_bytes), "activation output");
     if (kq_type(p.wtype) && !act_out) {
         // a kept copy of the records also pays at fewer rows (Q6_K 37 x 14336 ->
-        // 4096: 28 us against 44 on the 32 x 32 tiles).  Where the workspace
+        // 4096: 28 us against 41 on the 32 x 32 tiles).  Where the workspace
         // cannot hold the layout (a caller's or a fixed one, or growth under
         // capture), first without the K split, else the decode kernels.
         p.kq_reg = kq_registered(ctx, p, a->data) != nullptr;

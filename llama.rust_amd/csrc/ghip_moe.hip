@@ -948,9 +948,9 @@ __device__ __forceinline__ void kq32_tile(const uint8_t *__restrict__ wrow, int 
         for (int c = 0; c < 8; c++) o.a[c] = ld16(ab + 4 + 32 * c + 16 * h);
     };
     auto dwords = [](uint4 v, uint32_t (&x)[4]) { x[0] = v.x; x[1] = v.y; x[2] = v.z; x[3] = v.w; };
-    // All but Q6_K: the sum's and the min product's roundings are carried along
-    // (without, 1.03e-7 from the 64-bit value at K = 14336 where the prefill
-    // GEMM's chain is 0.85e-7)
+    // The sum's and the min product's roundings are carried along (without, Q4_K is
+    // 1.03e-7 from the 64-bit value at K = 14336 where the prefill GEMM's chain is
+    // 0.85e-7)
     float part[16], lost[16];
 #pragma unroll
     for (int v = 0; v < 16; v++) part[v] = lost[v] = 0.0f;
@@ -1109,9 +1109,7 @@ __device__ __forceinline__ void kq32_tile(const uint8_t *__restrict__ wrow, int 
 #pragma unroll
             for (int k = 0; k < 4; k++) {
                 const int v = 4 * q + k;
-                if constexpr (Q6) {
-                    part[v] = fmaf(dw * (float)is[v], dd[k], part[v]);
-                } else if constexpr (XS) {
+                if constexpr (Q6 || XS) {
                     const float y = fmaf(dw * (float)is[v], dd[k], lost[v]), z = part[v] + y;
                     lost[v] = sum_lost(y - (z - part[v]));
                     part[v] = z;
@@ -1209,7 +1207,7 @@ __device__ __forceinline__ void mmid_kq_impl(const uint8_t *__restrict__ as, int
 // prefill GEMM's 64 x 128 tiles leave most CUs one workgroup or none there;
 // these are 32 x 32 with K shared by four wavefronts, and need no layout pass
 // or K split over workgroups.  (24 rows, 4096 -> 14336:
-// Q6_K 83 -> 26 us against the decode kernels; the other types and the line to
+// Q6_K 84 -> 27 us against the decode kernels; the other types and the line to
 // the GEMM beside use_kq32, the host mirror, in ghip.cpp.)
 struct Kq32Multi {
     const uint8_t *W[4];

@@ -150,6 +150,25 @@ def test_short_batch_q8(be, ty, M, N, K, skew):
         assert np.all(np.abs(again - t.sum(-1)) <= (4 + K // 32) * 2.0 ** -24 * np.abs(t).sum(-1))
 
 
+def test_short_batch_carries_its_sum(be):
+    """Q6_K, four wavefronts a tile, long K: the first super-block of every
+    wavefront's share is large, each of the others 0.9 * 2^-25 of it, below half
+    an ulp of the sum, so that a plain chain loses them all (5.8 * 2^-24 of the
+    result).  Every term is exact; what is left are the result's own rounding
+    and those of three additions, carried."""
+    M, N, K = 40, 4128, 14336
+    blk = np.zeros((K // 256, 210), np.uint8)
+    blk[:, :128], blk[:, 128:192], blk[:, 192:208] = 0x11, 0xAA, 1  # every code 33 (value 1), scales 1
+    d = np.full(K // 256, 0.9 * 2.0 ** -15, np.float16)
+    d[:4] = 1024.0
+    blk[:, 208:210] = d.view(np.uint8).reshape(-1, 2)
+    wd = torch.from_numpy(blk.reshape(1, -1)).cuda().expand(N, -1).contiguous()
+    x = torch.full((M, K), 127.0, device="cuda")
+    got = be.mul_mat(wd, O.Q6_K, K, x).cpu().numpy().astype(np.float64)
+    want = float(d.astype(np.float64).sum()) * 256 * 127
+    assert np.all(np.abs(np.abs(got) - want) <= 2 * 2.0 ** -24 * want), (got[0, 0], want)
+
+
 def test_short_batch_group(be):
     """Siblings too wide together for these tiles, in a workspace sized for each
     alone: the bits of the single calls."""
