@@ -317,7 +317,7 @@ struct MulMatPlan {
     bool act_pre;     // src1 already holds the vec_dot_type blocks
     int kq_ns = 0;        // K slices of the Q2_K / Q3_K / Q6_K prefill GEMM (ghip_kq.hip); 0: not on it
     bool kq_reg = false;  // ... over a registered weight's records
-    bool no_copy = false;  // Q4_0 / IQ4_XS: the weight is known not to be registered (see use_kq32)
+    bool no_copy = false;  // Q4_0 / IQ4_XS: no registered copy that this call can use (see use_kq32)
 };
 
 // Q2_K / Q3_K / Q6_K prefill: the int8 GEMM of ghip_kq.hip
@@ -1388,7 +1388,13 @@ ghip_status mul_mat_plane(ghip_context *ctx, const ghip_tensor *a, const ghip_te
             if (p.kq_ns == 1 && !fits()) p.kq_ns = 0;
         }
     }
-    if (p.wtype == GHIP_TYPE_Q4_0 || p.wtype == GHIP_TYPE_IQ4_XS) p.no_copy = !kq_registered(ctx, p, a->data);
+    if (p.wtype == GHIP_TYPE_Q4_0 || p.wtype == GHIP_TYPE_IQ4_XS) {
+        // (a registered weight's tiles serve it too where the workspace cannot hold
+        // the prefill GEMM's layout)
+        p.no_copy = !kq_registered(ctx, p, a->data);
+        if (!p.no_copy && !act_out)
+            p.no_copy = !ctx->workspace_fits(mul_mat_ws_bytes(p, d != nullptr, false, nullptr, nullptr), s);
+    }
     size_t act_bytes, lay_bytes;
     const size_t need = mul_mat_ws_bytes(p, d != nullptr, act_out != nullptr, &act_bytes, &lay_bytes, sub != nullptr);
     void *ws = nullptr;

@@ -150,6 +150,40 @@ def test_short_batch_q8(be, ty, M, N, K, skew):
         assert np.all(np.abs(again - t.sum(-1)) <= (4 + K // 32) * 2.0 ** -24 * np.abs(t).sum(-1))
 
 
+@pytest.mark.parametrize("ty", [O.Q4_0, O.IQ4_XS])
+def test_registering_keeps_a_call_served(ty):
+    """A wide weight that is registered after the call's first run: its capture
+    may not grow the workspace, and a caller's need not hold the GEMM's layout."""
+    import ghip
+    M, N, K = 40, 8224, 256
+    be = ghip.Backend(0)
+    qk, size = O.BLOCK[ty]
+    rng = np.random.default_rng(1)
+    w = rng.integers(0, 256, (N, K // qk, size), dtype=np.uint8)
+    w[:, :, :2] = (rng.random((N, K // qk)) * 0.01).astype(np.float16).view(np.uint8).reshape(N, -1, 2)
+    wd = torch.from_numpy(w.reshape(N, -1)).cuda()
+    x = torch.from_numpy(rng.standard_normal((M, K)).astype(np.float32)).cuda()
+    out = torch.empty((M, N), device="cuda")
+    want = be.mul_mat(wd, ty, K, x, out=out).clone()
+    be.register_weight(wd, ty, K)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        be.mul_mat(wd, ty, K, x, out=out)
+    for _ in range(3):
+        out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+    del g
+    be.set_workspace(torch.empty(16384, dtype=torch.uint8, device="cuda"))
+    assert torch.equal(be.mul_mat(wd, ty, K, x), want)
+    be.set_workspace(None)
+    tol = 40 * 2.0 ** -24 * float(want.abs().max())
+    assert float((be.mul_mat(wd, ty, K, x) - want).abs().max()) <= tol  # the GEMM over the copy
+    be.unregister_weight(wd, ty, K)
+    be.close()
+
+
 def test_short_batch_carries_its_sum(be):
     """Q6_K, four wavefronts a tile, long K: the first super-block of every
     wavefront's share is large, each of the others 0.9 * 2^-25 of it, below half
