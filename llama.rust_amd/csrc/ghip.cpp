@@ -320,6 +320,21 @@ struct MulMatPlan {
     bool no_copy = false;  // Q4_0 / IQ4_XS: no registered copy that this call can use (see use_kq32)
 };
 
+// The type's prefill GEMM row switch is set: it alone then parts the GEMM from the
+// decode kernels
+bool gemm_rows_set(int wtype) {
+    const char *v = nullptr;
+    switch (wtype) {
+    case GHIP_TYPE_Q4_K: v = getenv("GHIP_GEMM_MIN_ROWS"); break;
+    case GHIP_TYPE_Q5_K: v = getenv("GHIP_GEMM_Q5K_MIN_ROWS"); break;
+    case GHIP_TYPE_Q6_K: v = getenv("GHIP_GEMM_Q6K_MIN_ROWS"); break;
+    case GHIP_TYPE_Q4_0:
+    case GHIP_TYPE_Q8_0:
+    case GHIP_TYPE_IQ4_XS: v = getenv("GHIP_GEMM_Q8_MIN_ROWS"); break;
+    }
+    return v && *v;
+}
+
 // Q2_K / Q3_K / Q6_K prefill: the int8 GEMM of ghip_kq.hip
 bool kq_type(int t) { return t == GHIP_TYPE_Q2_K || t == GHIP_TYPE_Q3_K || t == GHIP_TYPE_Q6_K; }
 // Activation rows from which it beats the decode kernels (groups of 4 or 8
@@ -1188,7 +1203,7 @@ ghip_status run_gemm(ghip_context *ctx, const MulMatPlan &p, const void *w, cons
 //    wide matrices of the 4-bit types without a kept copy.
 bool use_kq32(const MulMatPlan &p, int64_t n = 0) {
     if (!n) n = p.N;
-    if (p.M < 9 || p.M > 128) return false;
+    if (p.M < 9 || p.M > 128 || gemm_rows_set(p.wtype)) return false;
     if (p.wtype == GHIP_TYPE_Q4_0 || p.wtype == GHIP_TYPE_Q8_0 || p.wtype == GHIP_TYPE_IQ4_XS) {
         if (p.K % 256 || (p.act_pre && p.wtype != GHIP_TYPE_IQ4_XS)) return false;
         if (p.M < 32) return true;
@@ -1380,7 +1395,8 @@ ghip_status mul_mat_plane(ghip_context *ctx, const ghip_tensor *a, const ghip_te
         // cannot hold the layout (a caller's or a fixed one, or growth under
         // capture), first without the K split, else the decode kernels.
         p.kq_reg = kq_registered(ctx, p, a->data) != nullptr;
-        if (!p.kq_ns && p.kq_reg && p.M >= (p.wtype == GHIP_TYPE_Q6_K ? 17 : 9) && p.M <= INT32_MAX)
+        if (!p.kq_ns && p.kq_reg && p.M >= (p.wtype == GHIP_TYPE_Q6_K ? 17 : 9) && p.M <= INT32_MAX &&
+            !gemm_rows_set(p.wtype))
             p.kq_ns = kq_nsplit(p.M, p.N, p.nb);
         auto fits = [&] { return ctx->workspace_fits(mul_mat_ws_bytes(p, d != nullptr, false, nullptr, nullptr), s); };
         if (!kq_required(p)) {

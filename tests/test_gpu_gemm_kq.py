@@ -184,6 +184,24 @@ def test_registering_keeps_a_call_served(ty):
     be.close()
 
 
+def test_row_switch_holds_for_a_registered_weight(be, monkeypatch):
+    """Q6_K with GHIP_GEMM_Q6K_MIN_ROWS raised: registered or not, the decode
+    kernels in the workspace that ghip_workspace_size names."""
+    import ghip
+    M, N, K = 64, 128, 1024
+    wd = torch.from_numpy(weights(O.Q6_K, N, K, 2)).cuda()
+    x = torch.from_numpy(np.random.default_rng(3).standard_normal((M, K)).astype(np.float32)).cuda()
+    monkeypatch.setenv("GHIP_GEMM_Q6K_MIN_ROWS", "1000")
+    out = torch.empty((M, N), device="cuda")
+    want = be.mul_mat(wd, O.Q6_K, K, x)
+    be.register_weight(wd, O.Q6_K, K)
+    be.set_workspace(torch.empty(be.workspace_size(ghip.mul_mat_node(wd, O.Q6_K, K, x, out)), dtype=torch.uint8, device="cuda"))
+    got = be.mul_mat(wd, O.Q6_K, K, x, out=out)
+    be.set_workspace(None)
+    be.unregister_weight(wd, O.Q6_K, K)
+    assert torch.equal(got, want)
+
+
 def test_short_batch_carries_its_sum(be):
     """Q6_K, four wavefronts a tile, long K: the first super-block of every
     wavefront's share is large, each of the others 0.9 * 2^-25 of it, below half

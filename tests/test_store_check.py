@@ -167,3 +167,37 @@ def test_groups_share_the_weight_row_stride():
     env = dict(os.environ, GHIP_DEBUG_LDD_SKEW="1")
     r = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
+
+
+def _route(ty, k, n, m):
+    """the kernel that stores a MUL_MAT's dst (under GHIP_DEBUG_LDD_SKEW the store
+    check refuses it by name)"""
+    st, msg = _run(ty, k, n, m)
+    assert st != 0 and "store check" in msg, msg
+    return msg.split(" of ", 1)[1].split(" ", 1)[0]
+
+
+def _switches():
+    import ghip
+    for ty, var in [(ghip.Q4_K, "GHIP_GEMM_MIN_ROWS"), (ghip.Q5_K, "GHIP_GEMM_Q5K_MIN_ROWS"),
+                    (ghip.Q6_K, "GHIP_GEMM_Q6K_MIN_ROWS"), (ghip.Q4_0, "GHIP_GEMM_Q8_MIN_ROWS"),
+                    (ghip.Q8_0, "GHIP_GEMM_Q8_MIN_ROWS"), (ghip.IQ4_XS, "GHIP_GEMM_Q8_MIN_ROWS")]:
+        for m in (20, 40):
+            assert "_kq32_" in _route(ty, 4096, 4096, m), (ty, m)
+            os.environ[var] = str(m)
+            at = _route(ty, 4096, 4096, m)
+            os.environ[var] = str(m + 1)
+            below = _route(ty, 4096, 4096, m)
+            del os.environ[var]
+            assert "gemm" in at and "_kq32_" not in at, (ty, m, at)
+            assert "gemm" not in below, (ty, m, below)
+
+
+def test_row_switches_part_gemm_and_decode():
+    """GHIP_GEMM_*_MIN_ROWS, where set: the prefill GEMM from that many rows, the
+    decode kernels below."""
+    code = ("import sys; sys.path.insert(0, %r); sys.path.insert(0, %r)\n"
+            "import test_store_check as T\nT._switches()\n") % (os.path.join(ROOT, "tests"), os.path.join(ROOT, "llama.rust_amd"))
+    env = dict(os.environ, GHIP_DEBUG_LDD_SKEW="1")
+    r = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout + r.stderr
