@@ -313,9 +313,10 @@ ghip_status ghip_workspace_size(int op, const ghip_tensor *dst, const ghip_tenso
  * once on `stream` now instead of on every call -- the reference's repack
  * cache (repack_*_cached, crates/ggml/src/repack.rs:4250-4480, and the
  * CPU_REPACK buffer it stands for).  Today those are the Q2_K / Q3_K / Q6_K
- * prefill GEMM's records (about 1.1 bytes a weight), the Q4_0 / Q5_0 / Q8_0 prefill GEMM's
- * int8 code plane with its f32 block scales, and (3-D MXFP4 expert weights)
- * the MUL_MAT_ID kernel's 80-byte windows; other types are read in their
+ * prefill GEMM's records (1.16 / 1.02 / 1.08 bytes a weight: 3.5 / 2.4 / 1.3 times
+ * the GGUF blocks), the int8 code plane with its f32 block scales of the
+ * Q4_0 / Q5_0 / Q8_0 / IQ4_NL / IQ4_XS / Q1_0 / Q2_0 prefill GEMM, and (3-D MXFP4 expert
+ * weights) the MUL_MAT_ID kernel's 80-byte windows; other types are read in their
  * GGUF layout and register as a no-op.  Later MUL_MAT calls whose src0 has the same data
  * pointer, type, ne[0], ne[1] and nb[1] use the copy.  The same switches as
  * the reference: LLAMA_RUST_REPACK=0 turns it off, LLAMA_RUST_REPACK_MAX_MB
@@ -330,8 +331,9 @@ ghip_status ghip_weight_register(ghip_context *ctx, const ghip_tensor *w, void *
  * that reads them completes).  Unknown weights are a no-op. */
 ghip_status ghip_weight_unregister(ghip_context *ctx, const ghip_tensor *w);
 
-/* Copies kept, their bytes, and how many were built so far (hits do not
- * count) -- repack_stats (repack.rs:4329-4334).  Any pointer may be NULL. */
+/* Copies kept, the bytes they count against the limit (their own; Q6_K 336
+ * per row and super-block, of which a copy takes 276), and how many were
+ * built so far (hits do not count) -- repack_stats (repack.rs:4329-4334).  Any pointer may be NULL. */
 ghip_status ghip_weight_cache_stats(ghip_context *ctx, size_t *n_weights, size_t *bytes, size_t *built);
 
 /* ---- GGUF files (crates/ggml/src/gguf.rs:388-655, a port of

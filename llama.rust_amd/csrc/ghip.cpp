@@ -140,7 +140,7 @@ struct ghip_context {
     // once the copy engine has drained it (its event)
     void *stage[2] = {nullptr, nullptr};
     hipEvent_t stage_ev[2] = {nullptr, nullptr};
-    size_t wcache_bytes = 0;   // bytes held by wcache
+    size_t wcache_bytes = 0;   // bytes counted against the cache limit
     size_t wcache_built = 0;   // copies materialized so far (hits do not count)
 
     // Store check (GHIP_CHECK_STORES=1, and every dry-run context): before a
@@ -937,9 +937,9 @@ size_t kq_weight_bytes(int wtype, int64_t N, int64_t nb) {
     const size_t rec = wtype == GHIP_TYPE_Q6_K ? 8832 : wtype == GHIP_TYPE_Q3_K ? 8320 : 9472;
     return (size_t)((N + 31) / 32) * (size_t)nb * rec;
 }
-// a registered weight's copy (Q6_K: 336 bytes per row and super-block at
-// least, the size its budget has always counted)
-size_t kq_copy_bytes(int wtype, int64_t N, int64_t nb) {
+// what a registered weight's copy counts against the cache limit: its records, for
+// Q6_K at least the 336 bytes per row and super-block that the limit is stated in
+size_t kq_charge_bytes(int wtype, int64_t N, int64_t nb) {
     const size_t n = kq_weight_bytes(wtype, N, nb);
     return wtype == GHIP_TYPE_Q6_K ? std::max(n, (size_t)N * (size_t)nb * 336) : n;
 }
@@ -2538,7 +2538,7 @@ ghip_status ghip_weight_register(ghip_context *ctx, const ghip_tensor *w, void *
                          "weight_register: Q6_K / Q4_0 / Q5_0 / Q8_0 / IQ4_NL / IQ4_XS / Q1_0 / Q2_0 weights are 2-D");
     // every other type is read in its GGUF layout: nothing to build
     if (!(q6k || mx || q8 || k23) || !repack_enabled()) return GHIP_STATUS_SUCCESS;
-    size_t bytes;
+    size_t bytes, held = 0;  // counted; allocated, where that is less
     int64_t nbk = 0, nrb = 0, ngp = 0;
     Q8Layout QL{};
     if (q8) {
@@ -2550,14 +2550,16 @@ ghip_status ghip_weight_register(ghip_context *ctx, const ghip_tensor *w, void *
         bytes = QL.w_b + QL.dw_b + q8_extra_b(w->type, QL);
     } else if (k23) {
         nbk = w->ne[0] / 256;
-        bytes = kq_copy_bytes(w->type, w->ne[1], nbk);
+        bytes = kq_charge_bytes(w->type, w->ne[1], nbk);
+        held = kq_weight_bytes(w->type, w->ne[1], nbk);
     } else if (q6k) {
         if (w->ne[0] % 256 || w->nb[0] != 210 || w->nb[1] < (uint64_t)(w->ne[0] / 256 * 210))
             return ctx->fail(GHIP_STATUS_BACKEND_ERROR, "weight_register: bad Q6_K geometry");
         if (w->ne[1] > INT32_MAX || w->ne[0] / 256 > INT32_MAX)
             return ctx->fail(GHIP_STATUS_BACKEND_ERROR, "weight_register: dimension too large");
         nbk = w->ne[0] / 256;
-        bytes = kq_copy_bytes(w->type, w->ne[1], nbk);
+        bytes = kq_charge_bytes(w->type, w->ne[1], nbk);
+        held = kq_weight_bytes(w->type, w->ne[1], nbk);
     } else {
         if (w->ne[0] % 32 || w->nb[0] != 17 || w->nb[1] < (uint64_t)(w->ne[0] / 32 * 17) ||
             (w->ne[2] > 1 && w->nb[2] < w->nb[1] * (uint64_t)w->ne[1]))
@@ -2578,16 +2580,17 @@ ghip_status ghip_weight_register(ghip_context *ctx, const ghip_tensor *w, void *
     ghip_status st = ctx->begin(s);
     if (st != GHIP_STATUS_SUCCESS) return st;
     void *rep = nullptr;
-    if (hipMalloc(&rep, bytes) != hipSuccess) {
+    if (!held) held = bytes;
+    if (hipMalloc(&rep, held) != hipSuccess) {
         (void)hipGetLastError();
         if (k23) return GHIP_STATUS_SUCCESS;  // not kept
-        return ctx->fail(GHIP_STATUS_OUT_OF_MEMORY, "weight_register: hipMalloc(%zu) failed", bytes);
+        return ctx->fail(GHIP_STATUS_OUT_OF_MEMORY, "weight_register: hipMalloc(%zu) failed", held);
     }
     if (q8) {
         st = q8w_repack(ctx, w->type, w->data, (int64_t)w->nb[1], w->ne[1], w->ne[0] / type_info(w->type).blck, QL, (int8_t *)rep,
                         (float *)((uint8_t *)rep + QL.w_b), s);
     } else if (q6k || k23) {
-        ctx->allow(rep, bytes, "weight records");
+        ctx->allow(rep, held, "weight records");
         st = kq_repack(ctx, w->type, w->data, (int64_t)w->nb[1], w->ne[1], nbk, (uint8_t *)rep, s);
     } else {
         const int64_t chunks = (int64_t)(bytes / 16);

@@ -173,3 +173,17 @@ def test_register_mxfp4_experts_bit_identical(be, monkeypatch, n, rows, n_as, n_
     assert torch.equal(sub1, sub0)
     be.unregister_weight(w, ghip.MXFP4, n)
     assert be.weight_cache_stats()[:2] == (n0, b0)
+
+
+def test_q6k_copy_takes_its_records(be):
+    """A kept Q6_K weight takes the device memory of its records (276 bytes a row
+    and super-block; 2 MiB pages), not the 336 that it counts."""
+    rows, n = 4096, 14336
+    w = torch.zeros((rows, n // 256 * 210), dtype=torch.uint8, device="cuda")
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    be.register_weight(w, O.Q6_K, n)
+    torch.cuda.synchronize()
+    took = free - torch.cuda.mem_get_info()[0]
+    be.unregister_weight(w, O.Q6_K, n)
+    assert rows * (n // 256) * 276 <= took <= rows * (n // 256) * 276 + (4 << 20), took
