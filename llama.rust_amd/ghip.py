@@ -92,7 +92,7 @@ def describe(t, ty, ne0=None):
     """ggml view of a torch tensor.  For quantized types `t` is uint8 with the
     packed rows in its last dim and ne0 gives the logical row length.
     (Three of these are most of the host time of a small call: 3.5 us each by
-    element assignments, 1.4 us packed in one go.)"""
+    element assignments, 1.2 us packed in one go.)"""
     if t is None:
         return None
     shape, stride = t.shape, t.stride()
@@ -107,6 +107,7 @@ def describe(t, ty, ne0=None):
         ne, nb = list(shape[::-1]), [s * e for s in stride[::-1]]
     else:
         assert t.dtype == torch.uint8
+        ne0 = int(ne0)
         if len(shape) == 2:
             n1, nb1 = shape[0], stride[0]
             nb2 = nb1 * n1

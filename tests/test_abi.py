@@ -121,3 +121,13 @@ def test_workspace_size_query_without_gpu():
 
     assert need(512) >= 512 * 4096 + 16 * 512 * (32 + 4)
     assert need(1) >= 0
+
+
+def test_describe_takes_any_whole_number():
+    """A row length that Python arithmetic left a float (2 * 2048.0) describes the
+    same tensor as the int."""
+    import torch
+    import ghip
+    for shape in ((8, 2304), (2, 8, 2304)):
+        w = torch.zeros(shape, dtype=torch.uint8)
+        assert bytes(ghip.describe(w, ghip.Q4_K, 4096.0)) == bytes(ghip.describe(w, ghip.Q4_K, 4096))
