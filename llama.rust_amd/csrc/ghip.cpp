@@ -1812,6 +1812,23 @@ ghip_status mul_mat_id_generic(ghip_context *ctx, const MoePlan &p, const ghip_t
 
 // Q8_0 activations, routing, then the tiled MFMA kernel; pairs with an
 // invalid expert id get NaN rows (the reference asserts on them).
+// K-quant experts with few pairs each take the row kernel (ghip_moe.hip
+// mmid_row_impl).  Measured with its quantize and routing launches, us, row kernel / 32 x
+// 32 tiles, Q4_K: one token, top-8 of 64, 4096 -> 2304 21 / 27, 2048 -> 768 13 / 21, 1024
+// -> 2304 17 / 15; 16 tokens, top-1 and top-2 of 64, 4096 -> 2304 31 / 36 and 52 / 54; 64
+// tokens, top-1 73 / 59; 3 tokens, top-1 of 8, 2048 -> 2304 15 / 12.  Q6_K, whose row takes
+// twice the instructions: one token, top-8 of 64, 4096 -> 768 19 / 34, 4096 -> 2304 32 / 35,
+// 2048 -> 768 17 / 22, 2048 -> 2304 27 / 21; 3 tokens, top-2 of 64, 4096 -> 2304 23 / 34; 16
+// tokens, top-2 80 / 77.
+bool mmid_row(const MoePlan &p) {
+    const int64_t n_pairs = p.n_ids * p.n_tokens;
+    if (p.nb < 8) return false;
+    if (p.n_tokens == 1) return p.wtype != GHIP_TYPE_Q6_K || p.nb >= 16 || n_pairs * p.rows <= 6144;
+    if (p.n_as < 16) return false;  // tokens meet in an expert
+    if (p.wtype == GHIP_TYPE_Q6_K) return p.nb >= 16 && 8 * n_pairs <= 3 * p.n_as;
+    return 4 * n_pairs <= (p.nb >= 16 ? 3 : 2) * p.n_as;
+}
+
 ghip_status mul_mat_id_impl(ghip_context *ctx, const ghip_tensor *as, const ghip_tensor *b, const ghip_tensor *ids,
                             const ghip_tensor *d, int32_t *sub, void *stream) {
     if (!ctx) return GHIP_STATUS_BACKEND_ERROR;
@@ -1863,6 +1880,11 @@ ghip_status mul_mat_id_impl(ghip_context *ctx, const ghip_tensor *as, const ghip
     if (st != GHIP_STATUS_SUCCESS) return st;
     if (kq) {
         const char *tn = p.wtype == GHIP_TYPE_Q4_K ? "q4_K" : p.wtype == GHIP_TYPE_Q5_K ? "q5_K" : "q6_K";
+        if (!sub && mmid_row(p))
+            return ctx->launch(std::string("ghip_mmid_") + tn + "_row", dim3((unsigned)max_tiles, (unsigned)((p.rows + 15) / 16)),
+                               dim3(256), 0, s, (const uint8_t *)as->data, (int64_t)as->nb[1], (int64_t)as->nb[2],
+                               (const uint8_t *)act, p.act_row_bytes, (int)p.ne11, (const int32_t *)route, (int)n_pairs,
+                               (int)p.n_ids, dst, dst_nb1, dst_nb2, (int)p.rows, (int)p.nb);
         // (about as many tiles as the experts that can be met)
         const int64_t blocks = (p.rows + 31) / 32, tiles = std::min(p.n_as, n_pairs) + n_pairs / 32;
         const int kw = sub ? 4 : kq32_waves(tiles * blocks, p.nb);

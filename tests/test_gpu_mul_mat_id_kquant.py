@@ -159,3 +159,15 @@ def test_invalid_id_gives_nan(be):
 def test_expert_tiles(be, tid, n, rows, n_as, n_tokens, n_ids):
     """The 32-pair x 32-row tiles at their edges, sub-sums bit-exact."""
     test_random_experts(be, tid, n, rows, n_as, n_tokens, 1, n_ids)
+
+
+@pytest.mark.parametrize("tid,n,rows,n_as,n_tokens,ne11,n_ids", [
+    (O.Q4_K, 2048, 37, 16, 1, 1, 5),    # one token; a wavefront short of its 4 rows
+    (O.Q5_K, 4352, 16, 4, 1, 2, 2),     # 17 super-blocks: a second pass
+    (O.Q6_K, 4096, 33, 16, 3, 1, 2),    # 6 pairs of 16 experts
+    (O.Q4_K, 4096, 50, 16, 3, 4, 4),    # 12 pairs: experts with more than one
+    (O.Q6_K, 2048, 64, 16, 1, 1, 8),
+])
+def test_few_pairs(be, tid, n, rows, n_as, n_tokens, ne11, n_ids):
+    """The row kernel of experts with about one pair each."""
+    test_random_experts(be, tid, n, rows, n_as, n_tokens, ne11, n_ids)
