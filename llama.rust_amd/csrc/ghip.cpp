@@ -317,7 +317,7 @@ struct MulMatPlan {
     bool act_pre;     // src1 already holds the vec_dot_type blocks
     int kq_ns = 0;        // K slices of the Q2_K / Q3_K / Q6_K prefill GEMM (ghip_kq.hip); 0: not on it
     bool kq_reg = false;  // ... over a registered weight's records
-    bool no_copy = false;  // Q4_0 / IQ4_XS: no registered copy that this call can use (see use_kq32)
+    bool no_copy = false;  // Q4_0 / Q8_0 / IQ4_XS: no registered copy that this call can use (see use_kq32)
 };
 
 // The type's prefill GEMM row switch is set: it alone then parts the GEMM from the
@@ -1183,37 +1183,50 @@ ghip_status run_gemm(ghip_context *ctx, const MulMatPlan &p, const void *w, cons
 // Q8_0 rows.  Measured against what served the rows before, us, 4096 -> 14336 /
 // 4096 -> 4096 / 14336 -> 4096:
 //  * Q5_K (to 15 rows the 8-column decode kernels, then the prefill GEMM): 9 rows
-//    21 / 13 / 27 against 48 / 25 / 84, 37 rows 37 / 16 / 32 against 39 / 25 / 44;
+//    21 / 13 / 27 against 48 / 25 / 84, 37 rows 37 / 16 / 32 against 39 / 25 / 44; not 33 rows
+//    of a wide K = 8192 (-> 14336 73 and 63; K = 6144 44 and 63, K = 11008 78 and 96);
 //  * Q6_K (8-column decode kernels to 63 rows; a registered weight's records
 //    serve it better from 17 rows, see mul_mat_plane): 24 rows 27 / 15 / 39
-//    against 83 / 42 / 88;
+//    against 83 / 42 / 88; not 9-16 rows of a long K with few weight rows (14336 -> 1024,
+//    9 rows 34 and 25, 16 rows 36 and 32; 8192 -> 1024 23 and 20, 24 and 25);
 //  * Q4_K at 9-15 rows where the LDS image of the matrix-core decode kernel does
 //    not fit: - / - / 23 against 74-123 (with it, 17-20 / 13-15 / - against
 //    21 / 14 / -, and siblings in one launch 2 % slower: it stays);
-//  * Q4_K at 16-64 rows, against the prefill GEMM, 24 rows 21 / 14 / 26 and 22 / 17 /
-//    24, 37 rows 31 / 14 / 28 and 23 / 17 / 25: one token tile or few weight rows
-//    (n: of the launch, all grouped matrices), short K;
+//  * Q4_K at 16-64 rows, against the prefill GEMM (n: weight rows of the launch, all
+//    grouped matrices): 32 rows 4096 -> 14336 20 and 23, 7168 -> 8192 18 and 22, 8192 ->
+//    4096 23 and 19; 33 rows, two token tiles, 4096 -> 8192 19 and 21, 7168 -> 4096 16 and 20,
+//    7168 -> 6144 24 and 21, 8192 -> 6144 36 and 22;
 //  * Q4_0 / Q8_0 / IQ4_XS to 31 rows, against the 8-column decode kernels, at 16
-//    26 / 23 / 37, 48 / 27 / 69, 25 / 17 / 33 and 54 / 52 / 93, 80 / 98 / 179, 57 / 28 / 58;
+//    26 / 23 / 37, 48 / 27 / 69, 25 / 17 / 33 and 54 / 52 / 93, 80 / 98 / 179, 57 / 28 / 58; not
+//    IQ4_XS with 9-11 rows of a long K and few weight rows (14336 -> 1024 26 and 23);
 //  * the same against the prefill GEMM, which repacks a weight that is not
 //    registered and goes through K in one chain, 64 rows 50 / 21 / 48, 91 / 34 / 76,
-//    43 / 17 / 35 and 82 / 60 / 180, 84 / 58 / 181, 90 / 60 / 190 (registered 38 /
-//    37 / 112, 38 / 37 / 111, 40 / 37 / 122), 128 rows 84 / 31 / 79, 155 / 51 / 139, 68 /
-//    26 / 62 and 86 / 60 / 180, 85 / 60 / 182, 91 / 61 / 190: few weight rows, and
-//    wide matrices of the 4-bit types without a kept copy.
+//    43 / 17 / 35 and 82 / 60 / 180, 84 / 58 / 181, 90 / 60 / 190, 128 rows 84 / 31 / 79,
+//    155 / 51 / 139, 68 / 26 / 62 and 86 / 60 / 180, 85 / 60 / 182, 91 / 61 / 190: few weight
+//    rows, and wide matrices of the 4-bit types.  Registered (GEMM 38 / 37 / 112, 38 / 37 / 111,
+//    40 / 37 / 122) while the tiles are few: Q8_0 64 rows 4096 -> 4096 (256 tiles) 34, -> 6144
+//    47 and 37; Q4_0 96 rows 2048 -> 6144 (576) 25 and 23, 4096 -> 8192 (768) 37 and 38, 128
+//    rows -> 8192 (1024) 47 and 38.
 bool use_kq32(const MulMatPlan &p, int64_t n = 0) {
     if (!n) n = p.N;
     if (p.M < 9 || p.M > 128 || gemm_rows_set(p.wtype)) return false;
+    // (the decode kernels' 8-column launches where those serve such a K)
+    const bool narrow = p.N <= 2048 && p.nb <= 56;
     if (p.wtype == GHIP_TYPE_Q4_0 || p.wtype == GHIP_TYPE_Q8_0 || p.wtype == GHIP_TYPE_IQ4_XS) {
         if (p.K % 256 || (p.act_pre && p.wtype != GHIP_TYPE_IQ4_XS)) return false;
+        if (p.wtype == GHIP_TYPE_IQ4_XS && p.M <= 11 && narrow && p.nb >= 48) return false;
         if (p.M < 32) return true;
-        return p.N <= 8192 ? p.M <= (p.wtype == GHIP_TYPE_Q8_0 ? 64 : 128) : p.M <= 96 && p.no_copy;
+        if (p.wtype == GHIP_TYPE_Q8_0 && p.M > 64) return false;
+        if (p.N > 8192) return p.M <= 96 && p.no_copy && p.wtype != GHIP_TYPE_Q8_0;
+        const int64_t tiles = ((p.M + 31) / 32) * ((p.N + 31) / 32);
+        return p.no_copy || p.wtype == GHIP_TYPE_IQ4_XS || tiles <= (p.wtype == GHIP_TYPE_Q8_0 ? 256 : p.K >= 4096 ? 768 : 512);
     }
     if (p.M > 64 || p.kq_ns) return false;
-    if (p.wtype == GHIP_TYPE_Q6_K) return p.M < 64;
-    if (p.wtype == GHIP_TYPE_Q5_K) return true;
+    if (p.wtype == GHIP_TYPE_Q6_K) return p.M < 64 && !(narrow && p.nb >= 32 && p.M <= (p.nb >= 40 ? 16 : 12));
+    if (p.wtype == GHIP_TYPE_Q5_K) return p.M <= 32 || n <= 8192 || p.nb != 32;
     if (p.wtype != GHIP_TYPE_Q4_K) return false;
-    return p.M < 16 ? !use_skinny(p) : p.nb <= 32 && (p.M <= 32 || n <= 8192);
+    if (p.M < 16) return !use_skinny(p);
+    return p.M <= 32 ? p.nb < 32 || (p.nb == 32 && p.M == 16) : p.nb < 32 && n <= (p.nb <= 16 ? 8192 : 4096);
 }
 // wavefronts that share K in a 32 x 32 tile: 8 where the tiles are few (4096 ->
 // 4096, 24 rows, Q5_K, 128 tiles: 16.1 us with 4, 14.4 with 8; 4096 -> 14336, 448
@@ -1404,7 +1417,7 @@ ghip_status mul_mat_plane(ghip_context *ctx, const ghip_tensor *a, const ghip_te
             if (p.kq_ns == 1 && !fits()) p.kq_ns = 0;
         }
     }
-    if (p.wtype == GHIP_TYPE_Q4_0 || p.wtype == GHIP_TYPE_IQ4_XS) {
+    if (p.wtype == GHIP_TYPE_Q4_0 || p.wtype == GHIP_TYPE_Q8_0 || p.wtype == GHIP_TYPE_IQ4_XS) {
         // (a registered weight's tiles serve it too where the workspace cannot hold
         // the prefill GEMM's layout)
         p.no_copy = !kq_registered(ctx, p, a->data);

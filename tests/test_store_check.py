@@ -201,3 +201,25 @@ def test_row_switches_part_gemm_and_decode():
     env = dict(os.environ, GHIP_DEBUG_LDD_SKEW="1")
     r = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
+
+
+def _short_batches():
+    import ghip
+    for ty, k, n, m, tiles in [
+            (ghip.Q4_K, 4096, 8192, 40, True), (ghip.Q4_K, 8192, 8192, 40, False), (ghip.Q4_K, 7168, 6144, 40, False),
+            (ghip.Q4_K, 7168, 14336, 24, True), (ghip.Q4_K, 8192, 4096, 24, False), (ghip.Q5_K, 8192, 14336, 40, False),
+            (ghip.Q5_K, 8192, 14336, 32, True), (ghip.Q6_K, 14336, 1024, 16, False), (ghip.Q6_K, 14336, 4096, 9, True),
+            (ghip.Q6_K, 8192, 1024, 13, True), (ghip.Q6_K, 20480, 1024, 9, True), (ghip.IQ4_XS, 14336, 1024, 9, False),
+            (ghip.IQ4_XS, 14336, 1024, 12, True), (ghip.Q8_0, 4096, 8192, 40, True)]:
+        name = _route(ty, k, n, m)
+        assert ("_kq32_" in name) == tiles, (ty, k, n, m, name)
+
+
+def test_short_batch_routes():
+    """Which short batches take the 32 x 32 tiles: not a long K of few or many
+    weight rows that the GEMMs and decode kernels run faster."""
+    code = ("import sys; sys.path.insert(0, %r); sys.path.insert(0, %r)\n"
+            "import test_store_check as T\nT._short_batches()\n") % (os.path.join(ROOT, "tests"), os.path.join(ROOT, "llama.rust_amd"))
+    env = dict(os.environ, GHIP_DEBUG_LDD_SKEW="1")
+    r = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout + r.stderr
