@@ -1829,7 +1829,7 @@ ghip_status mul_mat_id_generic(ghip_context *ctx, const MoePlan &p, const ghip_t
 // mmid_row_impl).  Measured with its quantize and routing launches, us, row kernel / 32 x
 // 32 tiles, Q4_K: one token, top-8 of 64, 4096 -> 2304 21 / 27, 2048 -> 768 13 / 21, 1024
 // -> 2304 17 / 15; 16 tokens, top-1 and top-2 of 64, 4096 -> 2304 31 / 36 and 52 / 54; 64
-// tokens, top-1 73 / 59; 3 tokens, top-1 of 8, 2048 -> 2304 15 / 12.  Q6_K, whose row takes
+// tokens, top-1 73 / 59; 16 tokens, top-2 of 64, 2048 -> 2304 45 / 38.  Q6_K, whose row takes
 // twice the instructions: one token, top-8 of 64, 4096 -> 768 19 / 34, 4096 -> 2304 32 / 35,
 // 2048 -> 768 17 / 22, 2048 -> 2304 27 / 21; 3 tokens, top-2 of 64, 4096 -> 2304 23 / 34; 16
 // tokens, top-2 80 / 77.
@@ -1837,9 +1837,8 @@ bool mmid_row(const MoePlan &p) {
     const int64_t n_pairs = p.n_ids * p.n_tokens;
     if (p.nb < 8) return false;
     if (p.n_tokens == 1) return p.wtype != GHIP_TYPE_Q6_K || p.nb >= 16 || n_pairs * p.rows <= 6144;
-    if (p.n_as < 16) return false;  // tokens meet in an expert
-    if (p.wtype == GHIP_TYPE_Q6_K) return p.nb >= 16 && 8 * n_pairs <= 3 * p.n_as;
-    return 4 * n_pairs <= (p.nb >= 16 ? 3 : 2) * p.n_as;
+    // (few experts: tokens meet in one)
+    return p.nb >= 16 && p.n_as >= 16 && (p.wtype == GHIP_TYPE_Q6_K ? 8 : 4) * n_pairs <= 3 * p.n_as;
 }
 
 ghip_status mul_mat_id_impl(ghip_context *ctx, const ghip_tensor *as, const ghip_tensor *b, const ghip_tensor *ids,
