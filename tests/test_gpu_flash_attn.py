@@ -373,3 +373,23 @@ def test_few_rows_rounding(be, H, Hkv, D, T, S, holes, sinks):
     got = be.flash_attn_ext(q, k, v, m, sk, scale)
     differ = float((got != walk(q, k, v, m, sk, scale)).float().mean())
     assert differ <= 1e-3, differ
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_few_rows_specials(be, D):
+    """Infinities and NaN in live rows: a V element, a K element (scores of both
+    signs), a query that rounds to infinity, a score that overflows its f16
+    accumulator; each as the walk has it, the other rows untouched."""
+    H, Hkv, T, S = 8, 2, 5, 200
+    g = torch.Generator(device="cuda").manual_seed(D)
+    q = torch.randn(H, T, D, generator=g, device="cuda")
+    k, v = (torch.randn(Hkv, S, D, generator=g, device="cuda").half() for _ in range(2))
+    v[0, 10, 3], v[0, 70, 5], v[1, 100, 7] = float("inf"), float("nan"), 6e4
+    k[1, 150, 2] = float("inf")
+    q[1, 2, 4], q[6, 3, 9] = 1e5, float("nan")
+    m = torch.from_numpy(causal_mask(T, S)).cuda()
+    scale = float(np.float32(1.0 / np.sqrt(D)))
+    got, want = be.flash_attn_ext(q, k, v, m, None, scale), walk(q, k, v, m, None, scale)
+    assert bool(want.isnan().any()) and bool(want.isinf().any()) and bool(want.isfinite().any())
+    assert torch.equal(got.isnan(), want.isnan())
+    assert float((got != want)[~want.isnan()].float().mean()) <= 1e-3

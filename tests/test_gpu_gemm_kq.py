@@ -261,6 +261,49 @@ def test_infinite_scale(be, ty, M):
     assert np.isfinite(got[np.isfinite(want)]).all()
 
 
+def same_specials(got, want):
+    """NaN and infinities where the 64-bit value has them, finite elsewhere"""
+    assert np.isinf(want).any() and np.isnan(want).any() and np.isfinite(want).any()
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(np.where(np.isinf(want), got, 0), np.where(np.isinf(want), want, 0))
+    assert np.isfinite(got[np.isfinite(want)]).all()
+
+
+@pytest.mark.parametrize("ty,M", [(O.Q4_0, 24), (O.Q8_0, 24), (O.IQ4_XS, 24), (O.Q2_K, 20), (O.Q4_K, 24), (O.Q5_K, 24),
+                                  (O.Q4_K, 150)])
+def test_infinite_scale_or_min(be, ty, M):
+    """The short-batch tiles' Q8_0-row types with an infinite block scale, the
+    types with mins with an infinite dmin: infinities and NaN (zero sums, two
+    infinities that cancel) as in 64 bits."""
+    K, N = 2048, 136
+    qk, size = O.BLOCK[ty]
+    rng = np.random.default_rng(4)
+    at = BLOCK[ty][2] if ty in BLOCK else 0
+    if ty in BLOCK:
+        w = weights(ty, N, K, 3).reshape(N, -1, size)
+    else:
+        w = rng.integers(0, 256, (N, K // qk, size), dtype=np.uint8)
+        w[:, :, :2] = (rng.random((N, K // qk)) * 0.01).astype(np.float16).view(np.uint8).reshape(N, -1, 2)
+    for row, bs in ((3, (0,)), (40, (5,)), (135, (1, 3, 6))):
+        for i, b in enumerate(bs):
+            w[row, b, at:at + 2] = np.array([-np.inf if i == 1 else np.inf], np.float16).view(np.uint8)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    x[::3, :1024] = 0.0  # zero blocks: infinity times zero
+    wd, xd = torch.from_numpy(w.reshape(N, -1)).cuda(), torch.from_numpy(x).cuda()
+    got = be.mul_mat(wd, ty, K, xd).cpu().numpy()
+    sub = be.mul_mat_subsums(wd, ty, K, xd).cpu().numpy().astype(np.float64)
+    act = be.mul_mat_act(wd, ty, K, xd).cpu().numpy()
+    with np.errstate(invalid="ignore"):
+        if ty in BLOCK:
+            want, _ = exact(ty, w.reshape(N, -1), K, sub, act)
+        else:
+            d = w[:, :, :2].copy().view(np.float16)[..., 0].astype(np.float64)
+            d8 = (act.reshape(M, -1, 292)[:, :, :4].copy().view(np.float32) if ty == O.IQ4_XS
+                  else act.reshape(M, -1, 34)[:, :, :2].copy().view(np.float16))[..., 0].astype(np.float64)
+            want = (d * sub.reshape(M, N, -1) * d8[:, None, :]).sum(-1)
+    same_specials(got, want)
+
+
 @pytest.mark.parametrize("ty", [O.Q2_K, O.Q3_K])
 def test_small_workspace(be, ty):
     """A caller's workspace too small for the GEMM's layout still serves the

@@ -147,3 +147,23 @@ def test_few_rows_long_k(be, ty, M, N, K, decode):
     xr, wr = x.to(td).double(), w.double()
     err = (got.cpu().double() - xr @ wr.t()).abs()
     assert bool((err <= (64 + 8 + K // 512 + 1 + 3) * 2.0 ** -24 * (xr.abs() @ wr.abs().t())).all())
+
+
+@pytest.mark.parametrize("ty", ["f16", "bf16"])
+@pytest.mark.parametrize("M,N,K", [(40, 70, 264), (300, 4000, 256), (12, 33, 77)])
+def test_prefill_gemm_specials(be, ty, M, N, K):
+    """Infinities and NaN in activations and weights, and activations that round
+    to infinity, reach their own rows and columns only, as in 64 bits."""
+    import ghip
+    td = torch.float16 if ty == "f16" else torch.bfloat16
+    g = torch.Generator().manual_seed(K)
+    w, x = torch.randn((N, K), generator=g).to(td), torch.randn((M, K), generator=g)
+    x[1, 3], x[5, K - 1], x[8, 0] = float("inf"), float("nan"), 3.4e38 if ty == "bf16" else 7e4
+    x[9, 5] = 0.0
+    w[2, 3], w[7, K - 1], w[11, 5], w[30, 0] = float("-inf"), float("nan"), float("inf"), 0.0
+    got = be.mul_mat(w.cuda(), ghip.F16 if ty == "f16" else ghip.BF16, K, x.cuda()).cpu()
+    want = x.to(td).double() @ w.double().t()
+    assert bool(want.isnan().any()) and bool(want.isinf().any())
+    assert torch.equal(got.isnan(), want.isnan())
+    assert torch.equal(torch.where(want.isinf(), got, 0.0), torch.where(want.isinf(), want, 0.0).float())
+    assert bool(got[want.isfinite()].isfinite().all())

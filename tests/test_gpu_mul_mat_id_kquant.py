@@ -3,7 +3,8 @@
 The reference routes K-quant experts three ways (compute.rs:1917-2202): the
 Q4_K 8x8 repack gemv when an expert has rows % 8 == 0, the tiled kernel for
 experts with >= 8 routed pairs, the row vec_dot for the rest -- all on
-quantize_row_q8_K activations.  The GPU runs one kernel for all of them.
+quantize_row_q8_K activations.  The GPU runs 32 x 32 tiles, and with about one
+pair an expert a row kernel.
 Bar: the per-super-block int32 sums bit-exact against the oracle's (they do
 not depend on the route); fp32 outputs within 1e-5 relative of the oracle's
 routed result on quantized real-valued weights, and within the rounding bound
@@ -171,3 +172,38 @@ def test_expert_tiles(be, tid, n, rows, n_as, n_tokens, n_ids):
 def test_few_pairs(be, tid, n, rows, n_as, n_tokens, ne11, n_ids):
     """The row kernel of experts with about one pair each."""
     test_random_experts(be, tid, n, rows, n_as, n_tokens, ne11, n_ids)
+
+
+@pytest.mark.parametrize("tid", [O.Q4_K, O.Q5_K, O.Q6_K])
+@pytest.mark.parametrize("n_as,n_tokens,n_ids", [(2, 40, 2), (16, 1, 8)])  # the tiles; the row kernel
+def test_infinite_block_scale(be, tid, n_as, n_tokens, n_ids):
+    """A block scale (and a dmin) of infinity: infinities and NaN where the 64-bit
+    value of the integer sums has them, the other outputs finite."""
+    n, rows = 2048, 37  # (not a multiple of 8: mul_mat_act quantizes row by row, as the experts do)
+    rng = np.random.default_rng(tid)
+    size, at_d, at_m = {O.Q4_K: (144, 0, 2), O.Q5_K: (176, 0, 2), O.Q6_K: (210, 208, None)}[tid]
+    w = rng.integers(0, 256, (n_as, rows, n // 256, size), dtype=np.uint8)
+    for at in (at_d, at_m):
+        if at is not None:
+            w[..., at:at + 2] = (rng.random(w.shape[:3]) * 0.01).astype(np.float16)[..., None].view(np.uint8)
+    inf = np.array([np.inf], np.float16).view(np.uint8)
+    w[:, 3, 2, at_d:at_d + 2] = inf
+    w[:, 17, 5, (at_m or at_d):(at_m or at_d) + 2] = inf
+    y = rng.standard_normal((n_tokens, 1, n)).astype(np.float32)
+    y[::2, :, :768] = 0.0
+    ids = np.stack([rng.permutation(n_as)[:n_ids] for _ in range(n_tokens)]).astype(np.int32)
+    wd, yd, idd = torch.from_numpy(w.reshape(n_as, rows, -1)).cuda(), torch.from_numpy(y).cuda(), torch.from_numpy(ids).cuda()
+    got = be.mul_mat_id(wd, n, yd, idd, ty=tid).cpu().numpy()
+    sub = be.mul_mat_id_subsums(wd, n, yd, idd, ty=tid).cpu().numpy().astype(np.float64).reshape(n_tokens, n_ids, rows, n // 256, -1)
+    act = be.mul_mat_act(wd[0], tid, n, yd[:, 0]).cpu().numpy()
+    d8 = act.reshape(n_tokens, -1, 292)[:, :, :4].copy().view(np.float32)[..., 0].astype(np.float64)
+    f16 = lambda at: w[ids][..., at:at + 2].copy().view(np.float16)[..., 0].astype(np.float64)  # noqa: E731
+    with np.errstate(invalid="ignore"):
+        v = f16(at_d) * sub[..., 0]
+        if at_m is not None:
+            v = v - f16(at_m) * sub[..., 1]
+        want = (v * d8[:, None, None, :]).sum(-1)
+    assert np.isinf(want).any() and np.isnan(want).any()
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(np.where(np.isinf(want), got, 0), np.where(np.isinf(want), want, 0))
+    assert np.isfinite(got[np.isfinite(want)]).all()
