@@ -150,6 +150,55 @@ def test_short_batch_q8(be, ty, M, N, K, skew):
         assert np.all(np.abs(again - t.sum(-1)) <= (4 + K // 32) * 2.0 ** -24 * np.abs(t).sum(-1))
 
 
+@pytest.mark.parametrize("ty,M,N,K", [
+    (O.Q4_K, 24, 136, 8448),   # 33 super-blocks: split K, one partial token tile
+    (O.Q4_K, 33, 204, 8192),   # N % 8 != 0: row by row activations
+    (O.Q4_K, 40, 8224, 256),
+    (O.Q5_K, 100, 64, 1024),   # scales and mins 63, codes 31 and 0 (below)
+    (O.Q5_K, 70, 136, 2048),
+])
+def test_q4_q5_gemm(be, ty, M, N, K):
+    """The Q4_K GEMM where short batches reach it, and the Q5_K one, whose
+    fifth-bit plane 2 * sc * bit the extreme blocks take to its ends."""
+    w = weights(ty, N, K, M)
+    if ty == O.Q5_K:
+        blk = w.reshape(N, K // 256, 176)
+        blk[::2, :, 4:16] = 0xFF
+        blk[::4, :, 16:176] = 0xFF
+        blk[1::4, :, 16:176] = 0
+    x = np.random.default_rng(N).standard_normal((M, K)).astype(np.float32)
+    wd, xd = torch.from_numpy(w).cuda(), torch.from_numpy(x).cuda()
+    print(f"gemm type={ty} M={M} N={N} K={K}", flush=True)
+    sub = be.mul_mat_subsums(wd, ty, K, xd).cpu().numpy()
+    want_sub = np.asarray(O.mul_mat(ty, w, K, N, x, M, want_subsums=True)[2])
+    assert np.array_equal(sub, want_sub.reshape(sub.shape))
+    out = torch.full((M + 1, N + 4), 7.0, device="cuda")
+    got = be.mul_mat(wd, ty, K, xd, out=out[:M, :N]).cpu().numpy()
+    want, mag = exact(ty, w, K, sub.astype(np.float64), be.mul_mat_act(wd, ty, K, xd).cpu().numpy())
+    # three roundings a term, a chain over the super-blocks
+    assert np.all(np.abs(got - want) <= (4 + K // 256) * 2.0 ** -23 * mag)
+    assert bool((out[M] == 7.0).all()) and bool((out[:, N:] == 7.0).all())
+
+
+def test_wide_group(be):
+    """Gate and up of a 37-row batch, together too wide for the tiles: the GEMM on
+    the library's own workspace, against 64-bit sums."""
+    import ghip
+    M, N, K = 37, 5000, 512
+    x = np.random.default_rng(7).standard_normal((M, K)).astype(np.float32)
+    xd = torch.from_numpy(x).cuda()
+    ws = [weights(O.Q4_K, N, K, 20 + i) for i in range(2)]
+    wds = [torch.from_numpy(w).cuda() for w in ws]
+    outs = [torch.full((M + 1, N + 4), 7.0, device="cuda") for _ in ws]
+    be.graph_compute([ghip.mul_mat_node(wd, O.Q4_K, K, xd, o[:M, :N]) for wd, o in zip(wds, outs)])
+    for w, wd, o in zip(ws, wds, outs):
+        sub = be.mul_mat_subsums(wd, O.Q4_K, K, xd).cpu().numpy().astype(np.float64)
+        want, mag = exact(O.Q4_K, w, K, sub, be.mul_mat_act(wd, O.Q4_K, K, xd).cpu().numpy())
+        # three roundings a term, a chain over the super-blocks
+        assert np.all(np.abs(o[:M, :N].cpu().numpy() - want) <= (4 + K // 256) * 2.0 ** -23 * mag)
+        assert bool((o[M] == 7.0).all()) and bool((o[:, N:] == 7.0).all())
+
+
 @pytest.mark.parametrize("ty,N", [(O.Q4_0, 8224), (O.IQ4_XS, 8224), (O.Q8_0, 6144)])
 def test_registering_keeps_a_call_served(ty, N):
     """A wide weight that is registered after the call's first run: its capture

@@ -158,26 +158,29 @@ def test_unsupported_type_raises(be):
 
 # ---------------------------------------------------------------- prefill GEMM
 @pytest.mark.parametrize("n,rows,cols", [(256, 32, 16), (512, 136, 37), (1024, 128, 128),
-                                         (768, 200, 130), (4096, 256, 64)])
+                                         (768, 200, 130), (4096, 256, 64),
+                                         (256, 8224, 40)])
 def test_gemm_q4K_small(be, n, rows, cols):
-    """Q4_K with >= 16 activation rows takes the int8-MFMA GEMM; tile edges in
-    both M (tokens) and N (weight rows)."""
+    """Q4_K with >= 16 activation rows: the int8-MFMA GEMM from 65 rows, at 33-64
+    with many weight rows (and from a long K on: test_gpu_gemm_kq.py), the 32 x
+    32 tiles else; edges of both in M (tokens) and N (weight rows)."""
     run_case(be, O.Q4_K, n, rows, cols, seed=rows)
 
 
 @pytest.mark.parametrize("n,rows,cols", [(256, 32, 16), (512, 136, 37), (1024, 128, 128), (768, 200, 130),
-                                         (4096, 300, 64), (2048, 64, 16)])
+                                         (4096, 300, 64), (2048, 64, 16), (2048, 136, 70)])
 def test_gemm_q5K_small(be, n, rows, cols):
-    """Q5_K with >= 16 activation rows takes the wide int8-MFMA GEMM with the
-    fifth-bit plane (split K when the tiles are few); tile edges in tokens and
-    rows; Q8_K bytes and int32 {iacc, imin} sub-sums bit-exact."""
+    """Q5_K with > 64 activation rows takes the wide int8-MFMA GEMM with the
+    fifth-bit plane (split K when the tiles are few), fewer the 32 x 32 tiles;
+    tile edges in tokens and rows; Q8_K bytes and int32 {iacc, imin} sub-sums
+    bit-exact."""
     run_case(be, O.Q5_K, n, rows, cols, seed=rows + 7)
 
 
 def test_gemm_q5K_extreme_blocks(be):
     """Q5_K blocks at the ends of every field (6-bit scales and mins 63, all
-    codes 31 with qh all ones, or 0) against the oracle: the fifth-bit plane
-    2 * sc * bit stays within int8 and the sums exact."""
+    codes 31 with qh all ones, or 0) against the oracle, on the 32 x 32 tiles:
+    the sums exact (the GEMM's fifth-bit plane: test_gpu_gemm_kq.py)."""
     rng = np.random.default_rng(11)
     n, rows, cols = 1024, 64, 32
     w = rng.integers(0, 256, size=(rows, O.row_size(O.Q5_K, n)), dtype=np.uint8)
@@ -194,9 +197,9 @@ def test_gemm_q5K_extreme_blocks(be):
 @pytest.mark.parametrize("n,rows,cols", [(512, 136, 64), (1024, 200, 100), (768, 128, 130), (4096, 256, 64),
                                          (512, 8, 200)])
 def test_gemm_q6K_small(be, n, rows, cols):
-    """Q6_K with >= 64 activation rows takes the f16-MFMA GEMM (repacked
-    weights, exact split-scale planes); tile edges in tokens and rows; int32
-    sub-sums bit-exact."""
+    """Q6_K with >= 64 activation rows takes the int8-MFMA GEMM (repacked
+    weights, the scaled codes as two int8 planes); tile edges in tokens and
+    rows; int32 sub-sums bit-exact."""
     run_case(be, O.Q6_K, n, rows, cols, seed=rows + cols)
 
 
@@ -244,7 +247,7 @@ def test_gemm_q4K_prefill_shapes(be, tokens, n, rows):
 def test_gemm_q4K_rows_not_multiple_of_8(be, n, rows, cols):
     """Q4_K with N % 8 != 0 and >= 16 activation rows: the reference takes the
     tiled route (compute.rs:1596) with quantize_row_q8_K_ref activations for
-    every row (no 4x8 values); the GPU runs its GEMM on those bytes.  The
+    every row (no 4x8 values); the GPU runs its GEMM or tiles on those bytes.  The
     activation bytes are compared in full; at 4100 rows the oracle checks the
     last 516 rows (the ragged tile edge) and the sub-sums of the last 4."""
     w, x = make(O.Q4_K, n, rows, cols, seed=rows + cols)
@@ -269,18 +272,21 @@ def test_gemm_q4K_rows_not_multiple_of_8(be, n, rows, cols):
 
 
 @pytest.mark.parametrize("ty", [O.Q4_0, O.Q5_0, O.Q8_0])
-@pytest.mark.parametrize("n,rows,cols", [(256, 64, 32), (1024, 200, 100), (2880, 136, 130), (4096, 256, 64)])
+@pytest.mark.parametrize("n,rows,cols", [(256, 64, 32), (1024, 200, 100), (2880, 136, 130), (4096, 256, 64),
+                                         (256, 64, 129), (4096, 256, 136), (2880, 72, 33)])
 def test_gemm_q8_family(be, ty, n, rows, cols):
-    """Q4_0 / Q5_0 / Q8_0 with >= 32 f32 activation rows take the int8-MFMA
-    GEMM (one exact 32-block dot per MFMA); K not a multiple of 128 (2880)
-    pads with zeros; int32 block dots bit-exact."""
+    """Q4_0 / Q5_0 / Q8_0 with many f32 activation rows (Q5_0, and K that is no
+    multiple of 256, from 32; Q8_0 from 65, Q4_0 from 129; fewer: the 32 x 32
+    tiles) take the int8-MFMA GEMM (one exact 32-block dot per MFMA); K not a
+    multiple of 128 (2880) pads with zeros; int32 block dots bit-exact."""
     run_case(be, ty, n, rows, cols, seed=rows + cols + ty)
 
 
-def test_gemm_q8_family_registered(be):
+@pytest.mark.parametrize("cols", [96, 136])  # the 32 x 32 tiles, which read no copy; the GEMM
+def test_gemm_q8_family_registered(be, cols):
     """A registered Q4_0 weight (its int8 codes kept on the device) gives the
     same bits as the per-call repack."""
-    n, rows, cols = 4096, 512, 96
+    n, rows = 4096, 512
     w, x = make(O.Q4_0, n, rows, cols, seed=9)
     wd, xd = torch.from_numpy(w).cuda(), torch.from_numpy(x).cuda()
     print(f"gemm q8 registered n={n} rows={rows} cols={cols}", flush=True)
@@ -405,7 +411,8 @@ def test_gemv_persistent_grid(be, monkeypatch, rows, wgs):
     (O.Q4_K, 2, 1, 4, 2, 4, False),    # r2 = 2, r3 = 2
     (O.Q8_0, 2, 2, 2, 2, 3, True),     # one-to-one planes, src1 planes not contiguous
     (O.Q6_K, 1, 2, 2, 4, 1, True),
-    (O.Q4_0, 3, 1, 3, 1, 40, False),   # 40 rows: the prefill GEMM per plane
+    (O.Q4_0, 3, 1, 3, 1, 40, False),   # 40 rows: the 32 x 32 tiles per plane
+    (O.Q4_0, 3, 1, 3, 1, 130, False),  # the prefill GEMM per plane
 ])
 def test_batched_broadcast(be, ty, ne02, ne03, ne12, ne13, m, perm):
     """Batched MUL_MAT (forward_mul_mat, compute.rs:1440-1450): dst plane
@@ -455,7 +462,7 @@ def test_batched_shape_errors(be):
 def test_q4K_long_k_9_to_15_rows(be, cols):
     """Q4_K down projection (K = 14336) at 9-15 activation rows: the
     matrix-core decode kernel's 16-column LDS image does not fit there, so
-    the rows go to the whole-row kernels in groups of 8 columns.  The oracle
+    the rows go to the 32 x 32 tiles.  The oracle
     takes the reference's tiled route from 8 columns; the bar is 1e-5 or the
     gap between the reference's own two routes on these inputs (row vec_dot
     per column against the tiled kernel), whichever is larger."""

@@ -168,12 +168,13 @@ def test_reference_dot(be, ty):
     assert abs(float(got) - float(want)) <= TOL * max(1.0, abs(float(want))), (got, want)
 
 
+@pytest.mark.parametrize("cols", [48, 136])  # (IQ4_XS at 48: the 32 x 32 tiles, which read no copy)
 @pytest.mark.parametrize("ty", [O.IQ4_NL, O.IQ4_XS, O.Q1_0, O.Q2_0])
-def test_registered_weight_gemm(be, ty):
+def test_registered_weight_gemm(be, ty, cols):
     """A registered IQ4_NL / IQ4_XS / Q1_0 / Q2_0 weight keeps its int8-code copy; the GEMM on
     it gives the bits of the per-call repack."""
     import ghip
-    k, rows, cols = 1024, 192, 48
+    k, rows = 1024, 192
     w = random_blocks(ty, rows, k, seed=5)  # model scale
     x = np.random.default_rng(6).standard_normal((cols, k)).astype(np.float32)
     wd, xd = torch.from_numpy(w).cuda(), torch.from_numpy(x).cuda()

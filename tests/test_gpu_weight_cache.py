@@ -2,14 +2,15 @@
 cache, repack.rs:4250-4480) and the Q6_K prefill GEMM's exactness on
 extreme valid blocks.
 
-Bar: a registered weight gives bit-identical MUL_MAT results to the per-call
-repack, before and after unregistering, also inside a captured HIP graph;
-the cache counts what it built (repack_stats, repack.rs:4329) so a second
-registration or call is shown to reuse the copy.  The Q6_K GEMM keeps one
-fp32 accumulator per scale plane, whose sums are exact integers for any
-valid block: on blocks at the extremes (scales -128 / 127, q = 0 / 63,
-activations +-127) its super-block sums equal the oracle's int32 ones and
-its outputs stay within 1e-5.
+Bar: a GEMM over a registered weight gives the bits of the one that repacks
+per call, before and after unregistering, also inside a captured HIP graph
+(where a few activation rows take other kernels unless a copy is kept, the
+two agree to rounding); the cache counts what it built (repack_stats,
+repack.rs:4329) so a second registration or call is shown to reuse the copy,
+and the copy is shown to be what is read.  The Q6_K GEMM sums two int8 planes
+of scaled codes in int32: on blocks at the extremes (scales -128 / 127, q =
+0 / 63, activations +-127) its super-block sums equal the oracle's int32 ones
+and its outputs stay within 1e-5.
 """
 import numpy as np
 import pytest
@@ -49,7 +50,7 @@ def test_register_reuses_copy_bit_identical(be):
     be.register_weight(w, O.Q6_K, n)  # second registration: a hit
     n1, b1, built1 = be.weight_cache_stats()
     assert (n1, built1) == (n0 + 1, built0 + 1)
-    assert b1 - b0 == rows * (n // 256) * 336  # one 336-byte GEMM record per super-block
+    assert b1 - b0 == rows * (n // 256) * 336  # what a super-block counts (its record takes 276)
     first = be.mul_mat(w, O.Q6_K, n, x).clone()
     second = be.mul_mat(w, O.Q6_K, n, x).clone()
     assert be.weight_cache_stats()[2] == built1  # calls read the copy, build nothing
@@ -137,7 +138,7 @@ def test_q6K_gemm_extreme_blocks_exact(be):
     x[1] = -1.0
     print(f"q6_K GEMM extreme blocks rows={rows} n={n} tokens={tokens}", flush=True)
     want, _, want_sub = O.mul_mat(O.Q6_K, w, n, rows, x, tokens, want_subsums=True)
-    assert np.abs(want_sub).max() > 2 ** 24   # the case the per-plane accumulators exist for
+    assert np.abs(want_sub).max() > 2 ** 24   # more than f32 counts
     wd, xd = torch.from_numpy(w).cuda(), torch.from_numpy(x).cuda()
     got = be.mul_mat(wd, O.Q6_K, n, xd).cpu().numpy()
     assert rel_err(got, want) <= 1e-5, rel_err(got, want)
@@ -187,3 +188,25 @@ def test_q6k_copy_takes_its_records(be):
     took = free - torch.cuda.mem_get_info()[0]
     be.unregister_weight(w, O.Q6_K, n)
     assert rows * (n // 256) * 276 <= took <= rows * (n // 256) * 276 + (4 << 20), took
+
+
+@pytest.mark.parametrize("ty", [O.Q4_0, O.Q5_0, O.Q8_0, O.IQ4_NL, O.IQ4_XS, O.Q1_0, O.Q2_0, O.Q2_K, O.Q3_K, O.Q6_K])
+def test_the_copy_is_read(be, ty):
+    """The GEMM over a registered weight reads the copy: overwriting the GGUF
+    bytes (which a caller must not do) changes the result only after the
+    weight is unregistered."""
+    rows, n, tokens = 96, 1024, 136
+    qk, size = O.BLOCK[ty]
+    rng = np.random.default_rng(ty)
+    w = torch.from_numpy(rng.integers(0, 60, (rows, n // qk * size), dtype=np.uint8)).cuda()  # (finite scales)
+    x = torch.from_numpy(rng.standard_normal((tokens, n)).astype(np.float32)).cuda()
+    before = be.mul_mat(w, ty, n, x).clone()
+    assert bool(before.isfinite().all()) and float(before.abs().max()) > 0
+    be.register_weight(w, ty, n)
+    kept = w.clone()
+    w.zero_()
+    assert torch.equal(be.mul_mat(w, ty, n, x), before)
+    be.unregister_weight(w, ty, n)
+    assert float(be.mul_mat(w, ty, n, x).abs().max()) == 0
+    w.copy_(kept)
+    assert torch.equal(be.mul_mat(w, ty, n, x), before)
