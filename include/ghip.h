@@ -277,16 +277,17 @@ typedef struct ghip_node {
  * -> cpu_backend_graph_compute backend.rs:2169 -> compute::graph_compute
  * compute.rs:307).  Consecutive MUL_MAT nodes with 1-8 F32 activation rows
  * (Q6_K: one) that read the same src1 (same data and geometry) with the same
- * weight type (Q4_0, Q5_0, Q8_0, Q4_K, Q5_K, Q6_K) and the same K -- a
+ * weight type (Q4_0, Q5_0, Q8_0, Q4_K, Q5_K, Q6_K), K and row stride -- a
  * layer's q/k/v or gate/up at decode -- run as one launch of up to four
  * matrices (Q4_0 / Q5_0 / Q8_0 after one Q8_0 quantization), provided
  * no node of the group reads or overlaps another's dst (and, for Q4_K at 4+
  * rows, N % 8 == 0 holds for all or none: it selects the activation
  * quantizer); their results are bit-identical to the single-op calls.
- * Q4_K siblings with prefill batches (the GEMM's range, 16+ rows) likewise
- * run as one GEMM launch over all their tiles after one activation
+ * Q4_K siblings with 16+ rows likewise run as one launch, of the prefill GEMM
+ * or of the short-batch tiles, over all their tiles after one activation
  * quantization; results match the single-op calls within the MUL_MAT
- * tolerance (a small matrix alone sums split-K slices in order).  Returns the first failing node's status (the nodes before
+ * tolerance (a matrix alone may take the other kernel, or sum split-K slices
+ * in order).  Returns the first failing node's status (the nodes before
  * it have been enqueued); ghip_last_error names the failure.
  * GHIP_GRAPH_FUSE=0 in the environment turns the grouping off. */
 ghip_status ghip_graph_compute(ghip_context *ctx, const ghip_node *nodes, int32_t n_nodes, void *stream);
@@ -321,7 +322,7 @@ ghip_status ghip_workspace_size(int op, const ghip_tensor *dst, const ghip_tenso
  * pointer, type, ne[0], ne[1] and nb[1] use the copy.  The same switches as
  * the reference: LLAMA_RUST_REPACK=0 turns it off, LLAMA_RUST_REPACK_MAX_MB
  * caps the bytes kept (default 16384); a weight over the cap is not kept and
- * calls repack it per call as before (both return success).  Allocates
+ * calls repack it per call (both return success).  Allocates
  * (hipMalloc): fails with GHIP_STATUS_ALLOC_FAILED while `stream` is being
  * captured.  The weight's bytes must not change until
  * ghip_weight_unregister. */

@@ -889,7 +889,7 @@ ghip_status run_gemv(ghip_context *ctx, const MulMatPlan &p, const void *w, cons
 // out for the GEMM (codes | bsum16 | d, tokens padded to 128), then the int8
 // MFMA GEMM runs on 128 x 128 tiles.
 constexpr size_t kGemmSmem128 = 116224, kGemmSmem64 = 76544;  // sizeof(g3::Smem<BM>) in ghip_gemm.hip
-constexpr size_t kGemmSmemQ8 = 22528;                          // sizeof(g8::Smem) in ghip_gemm.hip                         // sizeof(g6::Smem) in ghip_gemm.hip
+constexpr size_t kGemmSmemQ8 = 22528;                          // sizeof(g8::Smem) in ghip_gemm.hip
 constexpr size_t kGemmSmemW8 = 148480;  // 2 * sizeof(g4::Stage<256>) in ghip_gemm.hip
 // GHIP_GEMM_BM=128 selects the 128 x 128 tiles of gemm_q4K_impl
 int gemm_bm() { return env_int("GHIP_GEMM_BM", 64) == 128 ? 128 : 64; }
@@ -1010,11 +1010,11 @@ ghip_status gemm_act(ghip_context *ctx, const MulMatPlan &p, const uint8_t *act,
               : ctx->launch("ghip_gemm_act_layout", dim3(lgrid), dim3(256), 0, s, act, (int64_t)p.act_row_bytes,
                             (int)p.M, (int)Mpad, (int)nbk, codes, bsT, dT);
 }
-// Q6_K from 64 rows has always needed its GEMM's workspace and is refused
-// without it; the others were served by the decode kernels' small one
+// Q6_K from 64 rows is refused without its GEMM's workspace; the others fall
+// back to kernels that need less
 bool kq_required(const MulMatPlan &p) { return p.wtype == GHIP_TYPE_Q6_K && p.M >= 64 && p.K >= 512; }
-// the K split, for those calls within the bytes they have always asked for
-// (f16 codes, scales, 336 bytes per row and super-block)
+// the K split; of those calls only as far as f16 codes, scales and 336 bytes per
+// row and super-block hold it, so that a caller's workspace of that size serves them
 int kq_plan_ns(MulMatPlan p) {
     p.kq_ns = kq_nsplit(p.M, p.N, p.nb);
     if (!kq_required(p)) return p.kq_ns;
@@ -1823,8 +1823,6 @@ ghip_status mul_mat_id_generic(ghip_context *ctx, const MoePlan &p, const ghip_t
                        kRows);
 }
 
-// Q8_0 activations, routing, then the tiled MFMA kernel; pairs with an
-// invalid expert id get NaN rows (the reference asserts on them).
 // K-quant experts with few pairs each take the row kernel (ghip_moe.hip
 // mmid_row_impl).  Measured with its quantize and routing launches, us, row kernel / 32 x
 // 32 tiles, Q4_K: one token, top-8 of 64, 4096 -> 2304 21 / 27, 2048 -> 768 13 / 21, 1024
@@ -1841,6 +1839,8 @@ bool mmid_row(const MoePlan &p) {
     return p.nb >= 16 && p.n_as >= 16 && (p.wtype == GHIP_TYPE_Q6_K ? 8 : 4) * n_pairs <= 3 * p.n_as;
 }
 
+// Quantized activations, routing, then the tiled MFMA or the row kernel; pairs with
+// an invalid expert id get NaN rows (the reference asserts on them).
 ghip_status mul_mat_id_impl(ghip_context *ctx, const ghip_tensor *as, const ghip_tensor *b, const ghip_tensor *ids,
                             const ghip_tensor *d, int32_t *sub, void *stream) {
     if (!ctx) return GHIP_STATUS_BACKEND_ERROR;

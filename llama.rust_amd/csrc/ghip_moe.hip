@@ -868,8 +868,8 @@ ghip_mxfp4_repack(const uint8_t *__restrict__ W, int64_t nb1, int64_t nb2, int r
 // Then one f32 scaling per super-block, as vec_dot_q4_K_q8_K and its kin
 // (vec_dot.rs:928-1040).
 //
-// Bound by the expert weights' way from memory; Q4_K, 64 experts of 2048 ->
-// 1536 rows, 64 tokens, top-8 (113 MB): 59 us (1.9 TB/s), 324 with a 64-lane dot per pair and
+// Bound by the scaling of the MFMAs' dots on the vector ALU (46 % busy, with 8 of a
+// tile's 32 tokens in use) and a tile's first loads; Q4_K, 64 experts of 2048 -> 1536 rows, 64 tokens, top-8 (113 MB): 59 us (1.9 TB/s), 324 with a 64-lane dot per pair and
 // row, which read the expert's rows once per 8 pairs.
 typedef int v16i __attribute__((ext_vector_type(16)));
 constexpr int MMID_BR = 32;  // rows per workgroup
