@@ -585,24 +585,15 @@ extern "C" __global__ void __launch_bounds__(512, 1)
 }
 
 
-// split-K partial sums [nsplit][M][N] -> dst, slices added in order; four
-// consecutive outputs per thread (N % 4 == 0).  Bound by the slices' latency, so
-// eight are in flight, whatever the carried sum waits for (128 x 14336 -> 1024 Q5_K,
-// the whole product: 42.0 us with a load a step, 31.7 here)
-extern "C" __global__ void __launch_bounds__(256)
-ghip_gemm_splitk_reduce(const float *__restrict__ part, int nsplit, int M, int N, float *__restrict__ dst,
-                        int64_t ldd) {
-    const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
-    if (i >= (int64_t)M * N) return;
-    const int m = (int)(i / N), n = (int)(i % N);
-    float acc[4], lost[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // lost: what the sum's roundings dropped, carried along
-    __builtin_memcpy(acc, part + i, 16);
-    constexpr int U = 8;
+// slices 1 .. nsplit - 1 of a split-K sum added in order, U of them in flight
+template <int U>
+DEV void splitk_add(const float *__restrict__ p, int64_t stride, int nsplit, float (&acc)[4]) {
+    float lost[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // what the sum's roundings dropped, carried along
     for (int z0 = 1; z0 < nsplit; z0 += U) {
         float v[U][4];
 #pragma unroll
         for (int u = 0; u < U; u++)  // (past the last: it again, not added)
-            __builtin_memcpy(v[u], part + (int64_t)min(z0 + u, nsplit - 1) * M * N + i, 16);
+            __builtin_memcpy(v[u], p + min(z0 + u, nsplit - 1) * stride, 16);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int u = 0; u < U; u++) {
@@ -615,6 +606,26 @@ ghip_gemm_splitk_reduce(const float *__restrict__ part, int nsplit, int M, int N
             }
         }
     }
+}
+// split-K partial sums [nsplit][M][N] -> dst, slices added in order; four
+// consecutive outputs per thread (N % 4 == 0).  Bound by the slices' latency, so
+// eight are in flight, whatever the carried sum waits for (128 x 14336 -> 1024 Q5_K,
+// the whole product: 42.0 us with a load a step, 31.7 here); two slices, bound by
+// their bytes, in one load (512 x 14336 -> 4096 Q6_K: 6.6 us with eight, 5.6 here)
+extern "C" __global__ void __launch_bounds__(256)
+ghip_gemm_splitk_reduce(const float *__restrict__ part, int nsplit, int M, int N, float *__restrict__ dst,
+                        int64_t ldd) {
+    const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+    if (i >= (int64_t)M * N) return;
+    const int m = (int)(i / N), n = (int)(i % N);
+    float acc[4];
+    __builtin_memcpy(acc, part + i, 16);
+    if (nsplit == 2)
+        splitk_add<1>(part + i, (int64_t)M * N, nsplit, acc);
+    else if (nsplit <= 4)
+        splitk_add<3>(part + i, (int64_t)M * N, nsplit, acc);
+    else
+        splitk_add<8>(part + i, (int64_t)M * N, nsplit, acc);
     float *d = dst + (int64_t)m * ldd + n;
 #pragma unroll
     for (int k = 0; k < 4; k++) d[k] = acc[k];

@@ -180,6 +180,12 @@ def test_q4_q5_gemm(be, ty, M, N, K):
     assert bool((out[M] == 7.0).all()) and bool((out[:, N:] == 7.0).all())
 
 
+@pytest.mark.parametrize("nb", [2, 3, 4, 5, 9, 10])
+def test_split_k_slices(be, nb):
+    """One super-block a slice: two, a few, and around eight slices after the first."""
+    test_q4_q5_gemm(be, O.Q4_K, 70, 136, 256 * nb)
+
+
 def test_wide_group(be):
     """Gate and up of a 37-row batch, together too wide for the tiles: the GEMM on
     the library's own workspace, against 64-bit sums."""
