@@ -1314,8 +1314,8 @@ int dense_gemm_tile(int64_t M, int64_t N) {
     return tiles(128) >= 384 ? 128 : tiles(64) >= 192 ? 64 : 32;
 }
 // F16 / BF16 with few rows, where the decode kernel (8 rows a launch) is the faster
-// one: the GEMM takes K in one chain, 3.3 ns an element (BF16 6.1, for the
-// activations' rounding), however few the tiles.  vec: 16-byte aligned rows.
+// one: the GEMM takes K in one chain, 3.3 ns an element (BF16 6.6, for the
+// activations' rounding and the carried sum), however few the tiles.  vec: 16-byte aligned rows.
 bool dense_decode_pays(const MulMatPlan &p, bool vec) {
     const bool bf = p.wtype == GHIP_TYPE_BF16;
     const int64_t M = p.M, K = p.K, N = p.N;
@@ -1337,7 +1337,7 @@ bool dense_decode_pays(const MulMatPlan &p, bool vec) {
     // 17 and 15, 12 x 14336 -> 512 50 and 44; but 9 x 4096 -> 2048 17 and 21, 12 x 14336 ->
     // 1024 50 and 58, 16 x 14336 -> 512 50 and 50.  BF16: 9 x 4096 -> 4096 29 and 25, 12 x 14336 ->
     // 4096 92 and 78, 16 x 8192 -> 2048 54 and 53, 17 x 14336 -> 512 90 and 76; 24 x 14336
-    // -> 512 90 and 96, 9 x 4096 -> 14336 39 and 69.
+    // -> 512 94 and 96, 9 x 4096 -> 14336 39 and 69.
     if (!bf) {
         if (M == 9) return K >= 4096 && N <= std::min<int64_t>(K / 4, 2048);
         return M <= (K > 16384 ? 16 : 12) && K >= 8192 && N <= 512 && N * K <= 512 * 16384;

@@ -140,7 +140,11 @@ __device__ __forceinline__ void gemv_dense_impl(const uint8_t *__restrict__ W, i
 // a second register set and those in a third.  With chains of 16 MFMAs and
 // one level the results were further from the 64-bit value (1.3e-7 at
 // K = 4096) than the decode kernel's 16-element chains and tree (1.0e-7);
-// these three levels are 0.94e-7 from it.
+// these three levels are 0.94e-7 from it.  BF16, whose decode kernel is 0.78e-7
+// from it (its products have fewer bits to lose) where the three levels are 0.85e-7,
+// adds the groups to one sum that carries its roundings along: 0.67e-7, for 1-4 % of
+// the time (200 x 4096 -> 4096 38.8 -> 40.2 us, 300 x 2048 -> 12000 80 -> 83; 512 x 1024
+// -> 16384 49 -> 55).
 //
 // Bound by a step's latency (LDS writes, barrier, LDS reads, MFMAs and the
 // next loads one after another) on one or two workgroups per CU, then by the
@@ -256,7 +260,8 @@ __device__ __forceinline__ void gemm_dense_impl(const uint8_t *__restrict__ W, i
             l[(BM + row) * P + (k8 ^ (row & 7))] = make_uint4(p.x & in, p.y & in, p.z & in, p.w & in);
         }
     };
-    v16f part[TM][TN] = {}, sum[TM][TN] = {};  // of a wavefront's last (up to) eight groups; of those before
+    // of a wavefront's last (up to) eight groups (BF16: what the sum's roundings dropped); of those before (all)
+    v16f part[TM][TN] = {}, sum[TM][TN] = {};
     const int nstep = (K + KB - 1) / KB;
     constexpr int FOLD = 8 / (KG * NS) > 1 ? 8 / (KG * NS) : 1;  // loop rounds per eight 64-element groups
     auto mult = [&](int st) {
@@ -290,10 +295,22 @@ __device__ __forceinline__ void gemm_dense_impl(const uint8_t *__restrict__ W, i
 #pragma unroll
             for (int i = 0; i < TM; i++)
 #pragma unroll
-                for (int j = 0; j < TN; j++) part[i][j] += acc[i][j];
+                for (int j = 0; j < TN; j++) {
+                    if constexpr (WT == WT_BF16) {
+#pragma unroll
+                        for (int v = 0; v < 16; v++) {
+                            const float y = acc[i][j][v] + part[i][j][v], t = sum[i][j][v] + y;
+                            part[i][j][v] = sum_lost(y - (t - sum[i][j][v]));
+                            sum[i][j][v] = t;
+                        }
+                    } else {
+                        part[i][j] += acc[i][j];
+                    }
+                }
         }
     };
     auto fold = [&]() {
+        if constexpr (WT == WT_BF16) return;
 #pragma unroll
         for (int i = 0; i < TM; i++)
 #pragma unroll

@@ -167,3 +167,18 @@ def test_prefill_gemm_specials(be, ty, M, N, K):
     assert torch.equal(got.isnan(), want.isnan())
     assert torch.equal(torch.where(want.isinf(), got, 0.0), torch.where(want.isinf(), want, 0.0).float())
     assert bool(got[want.isfinite()].isfinite().all())
+
+
+def test_bf16_gemm_carries_its_sum(be):
+    """BF16, one 32 x 32 tile, K shared by four wavefronts: the first 64-element group
+    of each is 64, every later one 0.85 of half an ulp of that.  Every product and
+    group is exact; what is left are half an ulp of the result, the roundings of
+    the three additions of the wavefronts' parts and what these drop at the end."""
+    import ghip
+    M, N, K = 24, 64, 16384
+    w = torch.full((N, K), 0.85 * 2.0 ** -24).to(torch.bfloat16)
+    w[:, :256] = 1.0
+    x = torch.ones((M, K))
+    want = float(w[0].double().sum())
+    got = be.mul_mat(w.cuda(), ghip.BF16, K, x.cuda()).cpu().double()
+    assert float((got - want).abs().max()) <= 2 * 2.0 ** -23 * want, (float(got[0, 0]), want)
