@@ -1333,18 +1333,17 @@ bool dense_decode_pays(const MulMatPlan &p, bool vec) {
         return groups * group < gemm;
     }
     if (!vec) return false;
-    // us, GEMM and decode.  F16: 9 x 14336 -> 512 50 and 30, -> 2048 51 and 49, 9 x 4096 -> 1024
-    // 17 and 15, 12 x 14336 -> 512 50 and 44; but 9 x 4096 -> 2048 17 and 21, 12 x 14336 ->
-    // 1024 50 and 58, 16 x 14336 -> 512 50 and 50.  BF16: 9 x 4096 -> 4096 29 and 25, 12 x 14336 ->
-    // 4096 92 and 78, 16 x 8192 -> 2048 54 and 53, 17 x 14336 -> 512 90 and 76; 24 x 14336
-    // -> 512 94 and 96, 9 x 4096 -> 14336 39 and 69.
-    if (!bf) {
-        if (M == 9) return K >= 4096 && N <= std::min<int64_t>(K / 4, 2048);
-        return M <= (K > 16384 ? 16 : 12) && K >= 8192 && N <= 512 && N * K <= 512 * 16384;
-    }
-    if (M <= 12) return K >= 2048 && N <= 4096;
-    if (M <= 16) return K >= 4096 && N <= std::min<int64_t>(K / 4, 4096);
-    return M <= 20 && K >= 8192 && N <= 512;
+    // us, GEMM and decode (launches of 8 rows and the rest).  F16: 9 x 14336 -> 512 50 and
+    // 43, -> 2048 51 and 48; but 9 x 4096 -> 1024 16 and 19, 12 x 8192 -> 512 30 and 35,
+    // 12 x 14336 -> 512 51 and 58.
+    if (!bf) return M == 9 && K >= 12288 && N <= 2048;
+    // BF16: 9 x 2048 -> 512 15 and 13, 9 x 4096 -> 4096 29 and 26, but 9 x 2048 -> 4096
+    // 16 and 17; 12 x 14336 -> 4096 102 and 96,
+    // but 12 x 2048 -> 4096 16 and 20; 16 x 14336 -> 512 94 and 81, 16 x 8192 -> 2048 54 and 53,
+    // but -> 3500 of 14336 101 and 113, 13 x 4096 -> 1024 29 and 31; 17 x 14336 -> 512 94 and 94.
+    if (M == 9) return K >= 2048 && N <= std::min<int64_t>(K, 4096);
+    if (M <= 12) return K >= 8192 && N <= 4096;
+    return M <= 16 && K >= 8192 && N * K <= 2048 * 8192;
 }
 // F32 / F16 / BF16 weights (compute.rs:1680-1745): F16 / BF16 from 9 activation
 // rows on the matrix cores where that pays, the rest on the dense decode kernel

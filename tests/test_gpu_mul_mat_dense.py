@@ -125,7 +125,9 @@ def test_prefill_gemm(be, ty, M, N, K):
 
 @pytest.mark.parametrize("ty,M,N,K,decode", [
     ("f16", 9, 512, 14336, True),
-    ("f16", 12, 64, 8192, True),
+    ("f16", 9, 64, 12288, True),
+    ("f16", 12, 64, 8192, False),
+    ("bf16", 17, 64, 8192, False),
     ("f16", 24, 1000, 4095, True),    # K not a multiple of 8
     ("bf16", 16, 1024, 8192, True),
     ("bf16", 10, 100, 2047, True),
