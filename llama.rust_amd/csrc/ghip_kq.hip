@@ -18,16 +18,16 @@
 //         a weight).
 // Every partial sum fits int32 (|is| <= 2^27), so is is exact for any block, and
 // the f32 work is one conversion, one product and one fma per output and
-// super-block.  Eight super-blocks add up apart from the total, whose own
+// super-block.  Eight super-blocks (Q3_K: four) add up apart from the total, whose own
 // roundings are carried along: a plain chain is further from the 64-bit value
 // than the decode kernels' trees (Q3_K, K = 14336: 8.6e-8 with groups of four and
-// a plain total, 7.7e-8 the trees, 7.1e-8
-// here).
+// a plain total, 7.7e-8 the trees, 7.1e-8 with eights; 300 x 4096 -> 14336: trees
+// 6.5e-8, eights 6.6e-8 in 54 us, fours 5.7e-8 in 55).
 //
 // Bound, at 64 tokens x 128 rows a workgroup, by the wavefronts' serial steps
 // (LDS reads, MFMAs, the f32 work) with two wavefronts a SIMD.  300 x 4096 ->
 // 14336 Q3_K, kept records: 940 us in 75 launches of the 4-column decode kernel,
-// 51 us here; 512 x 14336 -> 4096 Q6_K, kept records: 157 us on f16 planes from
+// 55 us here; 512 x 14336 -> 4096 Q6_K, kept records: 157 us on f16 planes from
 // 336-byte records with 152 KB of LDS a workgroup, 114 us.
 #include "ghip_common.h"
 #include "ghip_kplanes.h"
@@ -197,6 +197,7 @@ __device__ __forceinline__ void gemm_kq_impl(const uint8_t *__restrict__ R, int 
     };
     auto piece = [&](int b, int c) { return *reinterpret_cast<const uint4 *>(wr + (int64_t)b * REC + c * 1024 + 16 * lane); };
 
+    constexpr int GROUP = TYPE == 3 ? 4 : 8;  // super-blocks that add up apart from the total
     v16f part[2] = {}, sum[2] = {}, comp[2] = {};
     auto total_up = [&]() {  // sum += part, comp what the sum's rounding lost
 #pragma unroll
@@ -274,7 +275,7 @@ __device__ __forceinline__ void gemm_kq_impl(const uint8_t *__restrict__ R, int 
                     }
                 }
             }
-        if ((b - b0) % 8 == 7) total_up();
+        if ((b - b0) % GROUP == GROUP - 1) total_up();
         stage(p ^ 1);
         __syncthreads();
     }
