@@ -276,6 +276,23 @@ def test_short_batch_carries_its_sum(be):
     assert np.all(np.abs(np.abs(got) - want) <= 2 * 2.0 ** -24 * want), (got[0, 0], want)
 
 
+def test_q3_gemm_sums_in_fours(be):
+    """Q3_K, whole K in one workgroup: a large super-block and seven of 0.9 * 2^-25 of
+    it, below half an ulp.  Three of them meet it in its four and are lost (1.35 *
+    2^-24 of the result), the other four reach the total; all seven are 3.15."""
+    M, N, K = 300, 14336, 2048
+    w = np.zeros((K // 256, 110), np.uint8)
+    w[:, :32], w[:, 32:96], w[:, 96:104], w[:, 104:108] = 0xFF, 0x55, 0x11, 0xAA  # every code and scale 1
+    d = np.full(K // 256, 0.9 * 2.0 ** -15, np.float16)
+    d[0] = 1024.0
+    w[:, 108:110] = d.view(np.uint8).reshape(-1, 2)
+    wd = torch.from_numpy(w.reshape(1, -1)).cuda().expand(N, -1).contiguous()
+    got = be.mul_mat(wd, O.Q3_K, K, torch.full((M, K), 127.0, device="cuda")).double().abs()
+    want = float(d.astype(np.float64).sum()) * 256 * 127
+    err = float((got - want).abs().max())
+    assert err <= 2.4 * 2.0 ** -24 * want, (float(got[0, 0]), want)  # (and the result's own rounding, 1)
+
+
 def test_short_batch_group(be):
     """Siblings too wide together for these tiles, in a workspace sized for each
     alone: the bits of the single calls."""
